@@ -2,140 +2,241 @@
 // members of one mesh: per-member matrix values and right-hand sides), on gfx950.
 //
 // Layout: every vector is [row][member] and the values are [entry][member], so the M members of
-// one row are M consecutive words. A workgroup of 256 threads takes a tile of kBlkTile rows;
-// thread t works on member m = t % M for the rows tile*kBlkTile + s + S*j (s = t / M, S = 256 / M,
-// j = 0 .. kBlkTile/S - 1). With M = 64 a wave is one row of 64 members: the row pointers and
-// column indices are one uniform load for all members and the value and vector gathers are
-// 512-byte coalesced segments. Each member keeps the reference's recurrences (pcg_solver.py:
-// 172-276, 881-947, 1075-1124; pcg_loop.cpp:361-413) and its own stopping rule; a member that has
-// stopped keeps its solution and drops out of the loads.
+// one row are M consecutive words (M a power of two). A workgroup takes a tile of
+// kBlkTile = 512 rows and W = min(M, 8 or 16) of its members (blk_wide): its lanes are W members of
+// 64 / W consecutive rows, so a gather is 64- or 128-byte segments and the row pointers and columns
+// are read once for W members. Each member keeps the reference's recurrences (pcg_solver.py:172-276, 881-947,
+// 1075-1124; pcg_loop.cpp:361-413) and its own stopping rule; a member that has stopped keeps its
+// solution and drops out of the loads.
 //
-// Dot products (FP64) are summed in one fixed order, restated by the oracle (or_pcg_block):
-//   a thread adds its rows' terms to 0.0 in row order; the tile partial of member m adds the
-//   S threads' sums to 0.0 in slot order; the reduction kernel (1024 threads, RS = 1024 / M
-//   slots per member) has slot r add the tile partials r, r + RS, ... to 0.0 and then adds the
-//   RS slot sums to 0.0 in slot order.
+// Dot products (FP64) are summed in one fixed order, restated by the oracle (or_pcg_block): slot s
+// of 256 / M adds the products of the tile's rows s, s + S, s + 2 S, ... (S = 256 / M) to 0.0 in that
+// order; the tile partial of member m adds the S slot sums to 0.0 in slot order; the reduction
+// kernel (1024 threads, RS = 1024 / M slots per member) has slot r add the tile partials r, r + RS,
+// ... to 0.0 and then adds the RS slot sums to 0.0 in slot order. The order fixes which rows form
+// one chain of additions, not who multiplies: all 512 rows' products go to LDS with every load in
+// flight, and W S threads then add them from there.
+//
 // Each iteration is four launches: phase A (p update, SpMV, p.q partials), the p.q reduction
 // (alpha), phase B (x, r, z updates, r.r and r.z partials) and their reduction (stopping test,
-// beta). With 64 members a phase moves gigabytes, so the launch boundaries cost little.
+// beta). Splitting a tile over members and rows instead of giving each of 256 threads its slot's
+// whole chain of rows (J = 128 rows one after another at M = 64, on n / 512 workgroups) takes phase A
+// from 501 to 27 us and phase B from 85 to 17 us at 16,000 rows x 64 members, where the vectors and
+// values (115 MB) sit in the last-level cache; what bounds them now is that cache's rate.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
 
 #include "device.h"
 #include "reduce.h"
 
 namespace gsh {
 
-__device__ __forceinline__ void blk_slot(int M, int& s, int& m, int& S) {
-  m = (int)threadIdx.x % M;
-  s = (int)threadIdx.x / M;
-  S = kTpb / M;
+constexpr int kBlkRows = 4;  // rows of a thread in flight
+template <int W>
+constexpr int kBlkThreads = W == 16 ? 512 : 1024;
+
+// A thread's place: member m, tile, and the rows rl, rl + L, ... of the tile.
+struct BlkPlace {
+  int M, lm, lw, tile, w, m, rl, L;
+};
+template <int W>
+__device__ __forceinline__ BlkPlace blk_place(int M) {
+  BlkPlace q;
+  q.M = M;
+  q.lm = __builtin_ctz(M);
+  q.lw = min(q.lm, __builtin_ctz(W));
+  const int b = xcd_block(blockIdx.x, gridDim.x);  // a tile's parts and its neighbours on one XCD (shared L2)
+  q.tile = b >> (q.lm - q.lw);
+  q.w = (int)threadIdx.x & ((1 << q.lw) - 1);
+  q.m = ((b - (q.tile << (q.lm - q.lw))) << q.lw) + q.w;
+  q.rl = (int)threadIdx.x >> q.lw;
+  q.L = kBlkThreads<W> >> q.lw;
+  return q;
 }
 
-// tile partial of member m: the S slot sums in slot order (thread slot 0 of each member writes)
-__device__ __forceinline__ void blk_tile_partial(double acc, int M, int s, int m, int S, double* lds,
-                                                 double* __restrict__ out) {
-  lds[threadIdx.x] = acc;
+// The tile partial of each member of the workgroup from the rows' products in pr ([row][W]), which
+// every thread passes after its own are written. A row beyond n or of a stopped member has the
+// product +0.0, and a sum that started at 0.0 is never -0.0, so adding it changes no bit.
+__device__ __forceinline__ void blk_tile_sum(const BlkPlace& q, const double* pr, double* slot,
+                                             double* __restrict__ part) {
+  constexpr int B = 16;
+  const int SS = kTpb >> q.lm, J = kBlkTile / kTpb << q.lm;
   __syncthreads();
-  if (s == 0) {
-    double t = 0.0;
-    for (int q = 0; q < S; ++q) t += lds[q * M + m];
-    *out = t;
+  if (q.rl < SS) {
+    double x = 0.0;
+    const int jn = min(B, J);
+    for (int j0 = 0; j0 < J; j0 += B) {
+      double v[B];
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const double y = pr[((q.rl + SS * (j0 + (u & (jn - 1)))) << q.lw) + q.w];
+        v[u] = u < jn ? y : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < B; ++u) x += v[u];
+    }
+    slot[threadIdx.x] = x;
+  }
+  __syncthreads();
+  if (q.rl == 0) {
+    double x = 0.0;
+    for (int r0 = 0; r0 < SS; r0 += B) {
+      double v[B];
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const double y = slot[(min(r0 + u, SS - 1) << q.lw) + q.w];
+        v[u] = r0 + u < SS ? y : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < B; ++u) x += v[u];
+    }
+    part[(int64_t)q.tile * q.M + q.m] = x;
   }
 }
 
 // ---------------------------------------------------------------- init
 // cold start: x = 0, r = b, invD = 1 / diag, z = invD r, p_old = 0; partials of b.b and r.z
-template <class VT>
-__global__ void __launch_bounds__(256) k_blk_init(BlkSys<VT> S) {
-  __shared__ double lds[2][kTpb];
-  int s, m, SS;
-  blk_slot(S.M, s, m, SS);
-  const int M = S.M;
-  const int tile = xcd_block(blockIdx.x, gridDim.x);  // neighbouring tiles on one XCD (shared L2)
-  double bb = 0.0, rz = 0.0;
-  for (int j = 0; j < kBlkTile / SS; ++j) {
-    const int i = tile * kBlkTile + s + SS * j;
-    if (i >= S.n) break;
-    const int64_t e = (int64_t)i * M + m;
-    const VT inv = (VT)(1.0 / (double)S.val[(int64_t)S.diag[i] * M + m]);
-    const double bi = S.b[e];
-    const VT ri = (VT)bi;
-    const VT zi = inv * ri;
-    S.invd[e] = inv;
-    S.x[e] = (VT)0;
-    S.r[e] = ri;
-    S.z[e] = zi;
-    S.pb[e] = (VT)0;
-    bb += bi * bi;
-    rz += (double)ri * (double)zi;
+template <class VT, int W>
+__global__ void __launch_bounds__(kBlkThreads<W>) k_blk_init(BlkSys<VT> S) {
+  __shared__ double pr[2][kBlkTile * W], slot[2][kTpb];
+  const BlkPlace q = blk_place<W>(S.M);
+  for (int r = q.rl; r < kBlkTile; r += q.L) {
+    const int i = q.tile * kBlkTile + r;
+    double bb = 0.0, rz = 0.0;
+    if (i < S.n) {
+      const int64_t e = (int64_t)i * q.M + q.m;
+      const VT inv = (VT)(1.0 / (double)S.val[(int64_t)S.diag[i] * q.M + q.m]);
+      const double bi = S.b[e];
+      const VT ri = (VT)bi;
+      const VT zi = inv * ri;
+      S.invd[e] = inv;
+      S.x[e] = (VT)0;
+      S.r[e] = ri;
+      S.z[e] = zi;
+      S.pb[e] = (VT)0;
+      bb = bi * bi;
+      rz = (double)ri * (double)zi;
+    }
+    pr[0][(r << q.lw) + q.w] = bb;
+    pr[1][(r << q.lw) + q.w] = rz;
   }
-  blk_tile_partial(bb, M, s, m, SS, lds[0], S.part_a + (int64_t)tile * M + m);
-  blk_tile_partial(rz, M, s, m, SS, lds[1], S.part_b + (int64_t)tile * M + m);
+  blk_tile_sum(q, pr[0], slot[0], S.part_a);
+  blk_tile_sum(q, pr[1], slot[1], S.part_b);
 }
 
 // ---------------------------------------------------------------- phase A
-// beta (set by the previous reduction) -> p = z + beta p_old, q = A p, partials of p.q
+// Row sum of a_ij (z_j + beta p_j) in column order: the columns of 8 entries are loaded together,
+// then their values and gathers, so a row waits for two memory steps per 8 entries, not per entry.
 template <class VT>
-__global__ void __launch_bounds__(256) k_blk_a(BlkSys<VT> S, int it) {
-  __shared__ double lds[kTpb];
-  int s, m, SS;
-  blk_slot(S.M, s, m, SS);
-  const int M = S.M;
-  const int tile = xcd_block(blockIdx.x, gridDim.x);  // neighbouring tiles on one XCD (shared L2)
-  const BlkState st = S.st[m];
-  double acc = 0.0;
-  if (st.done < 0) {
-    const VT beta = (VT)st.beta;
-    const VT* __restrict__ po = (it & 1) ? S.pa : S.pb;
-    VT* __restrict__ pn = (it & 1) ? S.pb : S.pa;
-    for (int j = 0; j < kBlkTile / SS; ++j) {
-      const int i = tile * kBlkTile + s + SS * j;
-      if (i >= S.n) break;
-      const int a = S.rowptr[i], b = S.rowptr[i + 1];
-      VT qv = (VT)0;
-      for (int kk = a; kk < b; ++kk) {
-        const int64_t c = (int64_t)S.col[kk] * M + m;
-        qv += S.val[(int64_t)kk * M + m] * (S.z[c] + beta * po[c]);
+__device__ __forceinline__ VT blk_row(const BlkSys<VT>& S, const VT* __restrict__ po, VT beta, int a, int b, int m,
+                                      int M) {
+  constexpr int B = 8;
+  VT qv = (VT)0;
+  for (int k0 = a; k0 < b; k0 += B) {
+    int c[B];
+    VT v[B], z[B], p[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) c[u] = k0 + u < b ? S.col[k0 + u] : -1;
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (c[u] >= 0) {
+        const int64_t g = (int64_t)c[u] * M + m;
+        v[u] = S.val[(int64_t)(k0 + u) * M + m];
+        z[u] = S.z[g];
+        p[u] = po[g];
       }
-      const int64_t e = (int64_t)i * M + m;
-      const VT pi = S.z[e] + beta * po[e];
-      pn[e] = pi;
-      S.q[e] = qv;
-      acc += (double)pi * (double)qv;
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (c[u] >= 0) qv += v[u] * (z[u] + beta * p[u]);
+  }
+  return qv;
+}
+
+// beta (set by the previous reduction) -> p = z + beta p_old, q = A p, partials of p.q
+template <class VT, int W>
+__global__ void __launch_bounds__(kBlkThreads<W>) k_blk_a(BlkSys<VT> S, int it) {
+  __shared__ double pr[kBlkTile * W], slot[kTpb];
+  const BlkPlace q = blk_place<W>(S.M);
+  const BlkState st = S.st[q.m];
+  const VT beta = (VT)st.beta;
+  const VT* __restrict__ po = (it & 1) ? S.pa : S.pb;
+  VT* __restrict__ pn = (it & 1) ? S.pb : S.pa;
+  for (int r0 = q.rl; r0 < kBlkTile; r0 += kBlkRows * q.L) {
+    // every row pointer first: they depend on nothing
+    int a[kBlkRows], b[kBlkRows];
+#pragma unroll
+    for (int u = 0; u < kBlkRows; ++u) {
+      const int r = r0 + u * q.L, i = q.tile * kBlkTile + r;
+      const bool in = st.done < 0 && r < kBlkTile && i < S.n;
+      a[u] = in ? S.rowptr[i] : 0;
+      b[u] = in ? S.rowptr[i + 1] : 0;
+    }
+#pragma unroll
+    for (int u = 0; u < kBlkRows; ++u) {
+      const int r = r0 + u * q.L, i = q.tile * kBlkTile + r;
+      if (r >= kBlkTile) break;
+      double pq = 0.0;
+      if (st.done < 0 && i < S.n) {
+        const int64_t e = (int64_t)i * q.M + q.m;
+        const VT pi = S.z[e] + beta * po[e];
+        const VT qv = blk_row(S, po, beta, a[u], b[u], q.m, q.M);
+        pn[e] = pi;
+        S.q[e] = qv;
+        pq = (double)pi * (double)qv;
+      }
+      pr[(r << q.lw) + q.w] = pq;
     }
   }
-  blk_tile_partial(acc, M, s, m, SS, lds, S.part_a + (int64_t)tile * M + m);
+  blk_tile_sum(q, pr, slot, S.part_a);
 }
 
 // ---------------------------------------------------------------- phase B
 // x += alpha p, r -= alpha q, z = invD r; partials of r.r and r.z
-template <class VT>
-__global__ void __launch_bounds__(256) k_blk_b(BlkSys<VT> S, int it) {
-  __shared__ double lds[2][kTpb];
-  int s, m, SS;
-  blk_slot(S.M, s, m, SS);
-  const int M = S.M;
-  const int tile = xcd_block(blockIdx.x, gridDim.x);  // neighbouring tiles on one XCD (shared L2)
-  const BlkState st = S.st[m];
-  double rr = 0.0, rz = 0.0;
-  if (st.done < 0) {
-    const VT alpha = (VT)st.alpha;
-    const VT* __restrict__ p = (it & 1) ? S.pb : S.pa;
-    for (int j = 0; j < kBlkTile / SS; ++j) {
-      const int i = tile * kBlkTile + s + SS * j;
-      if (i >= S.n) break;
-      const int64_t e = (int64_t)i * M + m;
-      S.x[e] = S.x[e] + alpha * p[e];
-      const VT ri = S.r[e] - alpha * S.q[e];
-      const VT zi = S.invd[e] * ri;
-      S.r[e] = ri;
-      S.z[e] = zi;
-      rr += (double)ri * (double)ri;
-      rz += (double)ri * (double)zi;
+template <class VT, int W>
+__global__ void __launch_bounds__(kBlkThreads<W>) k_blk_b(BlkSys<VT> S, int it) {
+  __shared__ double pr[2][kBlkTile * W], slot[2][kTpb];
+  const BlkPlace q = blk_place<W>(S.M);
+  const BlkState st = S.st[q.m];
+  const VT alpha = (VT)st.alpha;
+  const VT* __restrict__ p = (it & 1) ? S.pb : S.pa;
+  for (int r0 = q.rl; r0 < kBlkTile; r0 += kBlkRows * q.L) {
+    // the rows' loads first: a store between them would order the next row's loads after it
+    VT xv[kBlkRows], pv[kBlkRows], rv[kBlkRows], qv[kBlkRows], dv[kBlkRows];
+#pragma unroll
+    for (int u = 0; u < kBlkRows; ++u) {
+      const int r = r0 + u * q.L, i = q.tile * kBlkTile + r;
+      if (st.done < 0 && r < kBlkTile && i < S.n) {
+        const int64_t e = (int64_t)i * q.M + q.m;
+        xv[u] = S.x[e];
+        pv[u] = p[e];
+        rv[u] = S.r[e];
+        qv[u] = S.q[e];
+        dv[u] = S.invd[e];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kBlkRows; ++u) {
+      const int r = r0 + u * q.L, i = q.tile * kBlkTile + r;
+      if (r >= kBlkTile) break;
+      double rr = 0.0, rz = 0.0;
+      if (st.done < 0 && i < S.n) {
+        const int64_t e = (int64_t)i * q.M + q.m;
+        S.x[e] = xv[u] + alpha * pv[u];
+        const VT ri = rv[u] - alpha * qv[u];
+        const VT zi = dv[u] * ri;
+        S.r[e] = ri;
+        S.z[e] = zi;
+        rr = (double)ri * (double)ri;
+        rz = (double)ri * (double)zi;
+      }
+      pr[0][(r << q.lw) + q.w] = rr;
+      pr[1][(r << q.lw) + q.w] = rz;
     }
   }
-  blk_tile_partial(rr, M, s, m, SS, lds[0], S.part_a + (int64_t)tile * M + m);
-  blk_tile_partial(rz, M, s, m, SS, lds[1], S.part_b + (int64_t)tile * M + m);
+  blk_tile_sum(q, pr[0], slot[0], S.part_a);
+  blk_tile_sum(q, pr[1], slot[1], S.part_b);
 }
 
 // ---------------------------------------------------------------- reductions
@@ -153,9 +254,19 @@ __device__ __forceinline__ double blk_total(const double* __restrict__ P, int nt
   }
   lds[threadIdx.x] = u;
   __syncthreads();
+  // slots beyond the tiles hold +0.0, which changes no sum; the others are read 16 ahead of their
+  // additions (1,024 slots one at a time took most of an iteration of a one-member block)
   double t = 0.0;
-  if (r == 0)
-    for (int q = 0; q < RS; ++q) t += lds[q * M + m];
+  if (r == 0) {
+    const int nr = min(RS, ntiles);
+    for (int q0 = 0; q0 < nr; q0 += 16) {
+      double v[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) v[q] = q0 + q < nr ? lds[(q0 + q) * M + m] : 0.0;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) t += v[q];
+    }
+  }
   __syncthreads();
   return t;
 }
@@ -217,18 +328,37 @@ __global__ void k_blk_get(double* __restrict__ x, const VT* __restrict__ xblk, i
 }
 
 // ---------------------------------------------------------------- launchers
+// Members of a workgroup: 16 where that still gives two workgroups per CU, else 8. With 16 a gather
+// is a whole 128-byte line and the columns are read once for twice the members (305,500 rows x 64
+// members: 830 us per iteration against 980; 30,000 x 256: 420 against 490); with 8 a small block
+// fills twice the CUs (16,000 x 64: 54 us against 75). 512 threads measured best with 16 members,
+// 1024 with 8.
+template <class VT, class F>
+static void blk_wide(const BlkSys<VT>& S, F&& launch) {
+  constexpr int kFill = 512;  // workgroups
+  if (S.M >= 16 && S.ntiles * (S.M / 16) >= kFill)
+    launch(std::integral_constant<int, 16>(), dim3(S.ntiles * (S.M / 16)));
+  else
+    launch(std::integral_constant<int, 8>(), dim3(S.ntiles * (S.M / std::min(S.M, 8))));
+}
 template <class VT>
 void launch_blk_init(const BlkSys<VT>& S, hipStream_t st) {
-  hipLaunchKernelGGL(k_blk_init<VT>, dim3(S.ntiles), dim3(kTpb), 0, st, S);
+  blk_wide(S, [&](auto w, dim3 grid) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL((k_blk_init<VT, W>), grid, dim3(kBlkThreads<W>), 0, st, S);
+  });
 }
 template <class VT>
 void launch_blk_iter(const BlkSys<VT>& S, int it, double rtol, int maxiter, int check_every, hipStream_t st) {
-  hipLaunchKernelGGL(k_blk_a<VT>, dim3(S.ntiles), dim3(kTpb), 0, st, S, it);
-  hipLaunchKernelGGL(k_blk_reduce, dim3(1), dim3(1024), 0, st, S.st, S.part_a, S.part_b, S.ntiles, S.M, 1, it, rtol,
-                     maxiter, check_every);
-  hipLaunchKernelGGL(k_blk_b<VT>, dim3(S.ntiles), dim3(kTpb), 0, st, S, it);
-  hipLaunchKernelGGL(k_blk_reduce, dim3(1), dim3(1024), 0, st, S.st, S.part_a, S.part_b, S.ntiles, S.M, 2, it, rtol,
-                     maxiter, check_every);
+  blk_wide(S, [&](auto w, dim3 grid) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL((k_blk_a<VT, W>), grid, dim3(kBlkThreads<W>), 0, st, S, it);
+    hipLaunchKernelGGL(k_blk_reduce, dim3(1), dim3(1024), 0, st, S.st, S.part_a, S.part_b, S.ntiles, S.M, 1, it, rtol,
+                       maxiter, check_every);
+    hipLaunchKernelGGL((k_blk_b<VT, W>), grid, dim3(kBlkThreads<W>), 0, st, S, it);
+    hipLaunchKernelGGL(k_blk_reduce, dim3(1), dim3(1024), 0, st, S.st, S.part_a, S.part_b, S.ntiles, S.M, 2, it, rtol,
+                       maxiter, check_every);
+  });
 }
 template <class VT>
 void launch_blk_reduce_init(const BlkSys<VT>& S, double rtol, hipStream_t st) {

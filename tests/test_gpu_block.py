@@ -82,3 +82,19 @@ def test_block_set_member_zero_rhs_and_maxiter(ctx):
     assert ei.value.code == L.GSH_E_ARG
     blk.close()
     solo.close()
+
+
+@pytest.mark.parametrize("members,nx,ny", [(1, 31, 19), (3, 40, 27), (100, 48, 23), (256, 164, 100)])
+def test_block_member_and_row_splits(ctx, members, nx, ny):
+    """One to 256 members: 8 or fewer and 16 members per workgroup (the last size), chains of 2 to
+    512 rows per slot, last tiles of a few rows; 25 iterations, bit for bit."""
+    mesh, p, blk, solo, vals, bs = _ensemble(ctx, members, nx, ny)
+    ip, ix = mesh.topology(L.T_CSR_INDPTR), mesh.topology(L.T_CSR_INDICES)
+    print(f"[gpu] block of {members} members, n={mesh.n}", flush=True)
+    it, st = blk.solve(rtol=1e-14, maxiter=25, check_every=10)
+    xo, ito, _ = O.pcg_block(ip, ix, vals, bs, rtol=1e-14, maxiter=25, nthreads=8)
+    assert np.array_equal(it, ito)
+    for m in {0, members // 2, members - 1}:
+        assert_bitwise(blk.solution(m), xo[m], f"block member {m}")
+    blk.close()
+    solo.close()
