@@ -551,6 +551,7 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
   if (check_every < 1) check_every = 1;
   if (timeout_s <= 0.0) timeout_s = 60.0;
   PcgState* slots = ctx->pinned_slots(nsys);
+  const TileRef* ptiles = nsys == 1 ? nullptr : dtiles;  // one system's phases need no table
   launch_pcg_reset<VT>(dsys, nsys, rtol, maxiter, check_every, st, rtols_dev);
   if (dinit_tiles)
     launch_pcg_init<VT>(dsys, dinit_tiles, ninit_tiles, rpt, st);
@@ -582,8 +583,8 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
       std::vector<hipEvent_t> evs(4 * w);
       for (auto& e : evs) HIPCHK(hipEventCreate(&e));
       for (int i = 0; i < w; ++i) {
-        launch_pcg_phase<VT>(0, dsys, dtiles, ntiles, rpt, st, evs[4 * i], evs[4 * i + 1]);
-        launch_pcg_phase<VT>(1, dsys, dtiles, ntiles, rpt, st, evs[4 * i + 2], evs[4 * i + 3]);
+        launch_pcg_phase<VT>(0, dsys, ptiles, ntiles, rpt, st, evs[4 * i], evs[4 * i + 1]);
+        launch_pcg_phase<VT>(1, dsys, ptiles, ntiles, rpt, st, evs[4 * i + 2], evs[4 * i + 3]);
       }
       HIPCHK(hipEventSynchronize(evs[4 * w - 1]));
       for (int i = 0; i < w; ++i) {
@@ -598,7 +599,7 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
       launch_pcg_check<VT>(dsys, nsys, st);
     } else {
       auto issue = [&]() {
-        for (int i = 0; i < w; ++i) launch_pcg_iter<VT>(dsys, dtiles, ntiles, rpt, st);
+        for (int i = 0; i < w; ++i) launch_pcg_iter<VT>(dsys, ptiles, ntiles, rpt, st);
         launch_pcg_check<VT>(dsys, nsys, st);
       };
       if (!(graph && launch_window_graph(*graph, st, dsys, w, rpt, issue))) issue();

@@ -23,6 +23,8 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device.h"
 #include "reduce.h"
 
@@ -42,8 +44,7 @@ struct SysView {
 };
 
 template <class VT>
-__device__ __forceinline__ SysView<VT> view(const PcgSys<VT>* __restrict__ sys, int i) {
-  const PcgSys<VT>& S = sys[i];
+__device__ __forceinline__ SysView<VT> view(const PcgSys<VT>& S) {
   SysView<VT> v;
   v.n = S.n;
   v.ntiles = S.ntiles;
@@ -130,7 +131,7 @@ __global__ void __launch_bounds__(256) k_pcg_init(const PcgSys<VT>* __restrict__
   __shared__ double red[4];
   __shared__ VT lds[kSpmvLdsCap];
   const TileRef tr = tiles[xcd_block(blockIdx.x, gridDim.x)];
-  const SysView<VT> S = view(sys, tr.sys);
+  const SysView<VT> S = view(sys[tr.sys]);
   const int n = S.n;
   const gptr<const double> h0 = S.h0, h1 = S.h1, h2 = S.h2;
   const bool hist = S.has_hist;
@@ -180,13 +181,18 @@ __global__ void __launch_bounds__(256) k_pcg_init(const PcgSys<VT>* __restrict__
 // chunk's nonzeros coalesced (lane l takes entries s0 + l + 64 m) together with the z and p_old
 // gathers; the products go to the wave's LDS slice and each lane sums its own row in column
 // order. Columns are read as int16 offsets from the chunk's first row when they fit.
-constexpr int kWaveCap = 640;   // nonzeros of a 64-row chunk held in registers (10 per lane)
-constexpr int kWaveM = kWaveCap / 64;
-
-template <class VT>
+//
+// W: a workgroup of 256 R threads, one row each, the tile's p.q summed in the R-rows-per-thread order
+// (tile_tree_wide), so results equal the 256-thread form's bit for bit. The 256-thread form walks
+// its R sub-rounds one after another, each waiting for entries and then gathers; the wide form has
+// all 4 R chunks of a tile in flight, which a system of few tiles needs (launch_pcg_phase).
+template <class VT, bool W>
 struct Chunk {
+  // nonzeros of a 64-row chunk held in registers: 10 per lane; 9 in the wide form, whose 16 waves'
+  // products then take 72 KB of LDS and two workgroups fit a CU
+  static constexpr int kM = W ? 9 : 10, kCap = 64 * kM;
   int s0, e0;
-  VT v[kWaveM], zc[kWaveM], pc[kWaveM];
+  VT v[kM], zc[kM], pc[kM];
 };
 
 template <class VT>
@@ -195,47 +201,46 @@ __device__ __forceinline__ int col_of(const SysView<VT>& S, int kk, int base64) 
 }
 
 // s0, e0: the chunk's first entry and the entry after its last (rowptr at r0w and r0w + 64)
-template <class VT>
+template <class VT, bool W>
 __device__ __forceinline__ void load_chunk(const SysView<VT>& S, gptr<const VT> po, int r0w, int lane, int s0, int e0,
-                                           Chunk<VT>& c) {
+                                           Chunk<VT, W>& c) {
   c.s0 = s0;
   c.e0 = e0;
-  if (c.e0 - c.s0 > kWaveCap) return;
+  if (c.e0 - c.s0 > c.kCap) return;
+  int col[c.kM];
 #pragma unroll
-  for (int m = 0; m < kWaveM; ++m) {
+  for (int m = 0; m < c.kM; ++m) {
     const int kk = c.s0 + lane + 64 * m;
     if (kk < c.e0) {
-      const int col = col_of(S, kk, r0w);
+      col[m] = col_of(S, kk, r0w);
       c.v[m] = S.val[kk];
-      c.zc[m] = S.z[col];
-      c.pc[m] = po[col];
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < c.kM; ++m) {
+    const int kk = c.s0 + lane + 64 * m;
+    if (kk < c.e0) {
+      c.zc[m] = S.z[col[m]];
+      c.pc[m] = po[col[m]];
     }
   }
 }
 
-template <class VT, int R>
-__global__ void __launch_bounds__(256) k_pcg_phase_a(const PcgSys<VT>* __restrict__ sys,
-                                                     const TileRef* __restrict__ tiles) {
-  __shared__ double red[4];
-  __shared__ VT lds[4 * kWaveCap];
-  const TileRef tr = tiles[xcd_block(blockIdx.x, gridDim.x)];
-  const SysView<VT> S = view(sys, tr.sys);
+template <class VT, int R, bool W>
+__device__ __forceinline__ void pcg_phase_a_body(const SysView<VT>& S, int tile, double* red, VT* lds) {
+  constexpr int kCap = Chunk<VT, W>::kCap, J = W ? 1 : R;
   gptr<PcgState> st = S.st;
-  if (load_done(st) >= 0) return;
-  const int k = st->k;
   const int n = S.n;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const gptr<VT> pn = (k & 1) ? S.pb : S.pa;
-  const gptr<const VT> po = (k & 1) ? S.pa : S.pb;
-  const int base = tr.tile * kTpb * R;
+  const int base = tile * kTpb * R;
   // FP64: the row pointers of every sub-round first: they depend on nothing, so each sub-round's
   // chunk then waits for two memory steps (entries, then gathers) instead of three. FP32 loads them
   // per sub-round: its registers would otherwise drop it from 7 to 5 waves per SIMD, which its
   // batched launches of small systems need more.
-  constexpr bool kPre = sizeof(VT) == 8;
-  int cs0[R], ce0[R], ra[R], rb[R];
+  constexpr bool kPre = W || sizeof(VT) == 8;
+  int cs0[J], ce0[J], ra[J], rb[J];
 #pragma unroll
-  for (int j = 0; j < R; ++j) {
+  for (int j = 0; j < J; ++j) {
     const int r0w = base + j * kTpb + w * 64;
     cs0[j] = ce0[j] = ra[j] = rb[j] = 0;
     if (kPre && r0w < n) {
@@ -248,6 +253,10 @@ __global__ void __launch_bounds__(256) k_pcg_phase_a(const PcgSys<VT>* __restric
       }
     }
   }
+  if (load_done(st) >= 0) return;
+  const int k = st->k;
+  const gptr<VT> pn = (k & 1) ? S.pb : S.pa;
+  const gptr<const VT> po = (k & 1) ? S.pa : S.pb;
   // a sub-round's first and end entries and the thread's row range (FP32: loaded here)
   auto rows_of = [&](int j, int r0w) {
     if (!kPre) {
@@ -260,23 +269,29 @@ __global__ void __launch_bounds__(256) k_pcg_phase_a(const PcgSys<VT>* __restric
       }
     }
   };
-  Chunk<VT> c;
+  const gptr<const VT> z = S.z;
+  Chunk<VT, W> c;
   const int r00 = base + w * 64;
+  VT zi0 = 0, pi0 = 0;  // the thread's own row (wide form: its only one)
   if (r00 < n) {
     rows_of(0, r00);
     load_chunk(S, po, r00, lane, cs0[0], ce0[0], c);
+    if (W && r00 + lane < n) {
+      zi0 = z[r00 + lane];
+      pi0 = po[r00 + lane];
+    }
   }
-  const double rz_cur = final_reduce(S.part_rz, S.ntiles, red);
+  const double rz_cur = W ? final_reduce_lo(S.part_rz, S.ntiles, red) : final_reduce(S.part_rz, S.ntiles, red);
   double beta = 0.0;
   if (k > 0) {
     const double rz_old = st->rho[(k - 1) & 1];
     beta = (rz_old == 0.0) ? 0.0 : rz_cur / rz_old;
   }
-  if (tr.tile == 0) {
+  if (tile == 0) {
     // workgroup 0: atol = rtol ||b|| at k = 0 (pcg_solver.py:928-930, 1089-1095), otherwise the
     // stopping test of iteration k-1 (pcg_loop.cpp:405-412)
     if (k == 0) {
-      const double bb = final_reduce(S.part_bb, S.ntiles, red);
+      const double bb = W ? final_reduce_lo(S.part_bb, S.ntiles, red) : final_reduce(S.part_bb, S.ntiles, red);
       if (threadIdx.x == 0) {
         const double atol = st->rtol * sqrt(bb);
         st->bb = bb;
@@ -289,7 +304,7 @@ __global__ void __launch_bounds__(256) k_pcg_phase_a(const PcgSys<VT>* __restric
     } else {
       const int it = k - 1;
       if ((it + 1) % st->check_every == 0 || it == st->maxiter - 1) {
-        const double rr = final_reduce(S.part_rr, S.ntiles, red);
+        const double rr = W ? final_reduce_lo(S.part_rr, S.ntiles, red) : final_reduce(S.part_rr, S.ntiles, red);
         if (threadIdx.x == 0) {
           st->rr_last = rr;
           if (rr <= st->atol2) st->done = k;
@@ -302,11 +317,10 @@ __global__ void __launch_bounds__(256) k_pcg_phase_a(const PcgSys<VT>* __restric
     }
   }
   const VT bv = (VT)beta;
-  const gptr<const VT> z = S.z;
-  VT* my = lds + w * kWaveCap;
+  VT* my = lds + w * kCap;
   double pq = 0.0;
 #pragma unroll
-  for (int j = 0; j < R; ++j) {
+  for (int j = 0; j < J; ++j) {
     const int r0w = base + j * kTpb + w * 64;
     if (r0w >= n) break;
     if (j > 0) {
@@ -315,9 +329,9 @@ __global__ void __launch_bounds__(256) k_pcg_phase_a(const PcgSys<VT>* __restric
     }
     const int i = r0w + lane;
     VT q = (VT)0;
-    if (c.e0 - c.s0 <= kWaveCap) {
+    if (c.e0 - c.s0 <= kCap) {
 #pragma unroll
-      for (int m = 0; m < kWaveM; ++m) {
+      for (int m = 0; m < c.kM; ++m) {
         const int kk = c.s0 + lane + 64 * m;
         if (kk < c.e0) my[kk - c.s0] = c.v[m] * (c.zc[m] + bv * c.pc[m]);
       }
@@ -335,51 +349,71 @@ __global__ void __launch_bounds__(256) k_pcg_phase_a(const PcgSys<VT>* __restric
       }
     }
     if (i < n) {
-      const VT pi = z[i] + bv * po[i];
+      const VT pi = (W ? zi0 : z[i]) + bv * (W ? pi0 : po[i]);
       pn[i] = pi;
       S.q[i] = q;
-      pq += (double)pi * (double)q;
+      const double t = (double)pi * (double)q;
+      if (W)
+        pq = t;
+      else
+        pq += t;
     }
   }
-  pq = block_tree(pq, red);
-  if (threadIdx.x == 0) S.part_pq[tr.tile] = pq;
+  // the wide form's row values pass through the first 64 words of each wave's own product slice
+  if (W)
+    pq = tile_tree_wide<R, kCap * (int)sizeof(VT) / 8>(pq, reinterpret_cast<double*>(lds), red);
+  else
+    pq = block_tree(pq, red);
+  if (threadIdx.x == 0) S.part_pq[tile] = pq;
+}
+
+// The launch table names each workgroup's system and tile; one system (tiles = NULL) needs none.
+template <class VT, int R, bool W>
+__global__ void __launch_bounds__(W ? kTpb * R : kTpb) k_pcg_phase_a(const PcgSys<VT>* __restrict__ sys,
+                                                                     const TileRef* __restrict__ tiles) {
+  __shared__ double red[4];
+  __shared__ __align__(8) VT lds[(W ? 4 * R : 4) * Chunk<VT, W>::kCap];
+  const int b = xcd_block(blockIdx.x, gridDim.x);
+  const TileRef tr = tiles ? tiles[b] : TileRef{0, b};
+  pcg_phase_a_body<VT, R, W>(view(sys[tr.sys]), tr.tile, red, lds);
 }
 
 // ------------------------------------------------------------------ phase B
 // f_update_xrz (pcg_solver.py:253-276): alpha = rz / pq (0 if pq == 0). The row loads are
-// issued before the scalar reduction, which only the arithmetic waits for.
-template <class VT, int R>
-__global__ void __launch_bounds__(256) k_pcg_phase_b(const PcgSys<VT>* __restrict__ sys,
-                                                     const TileRef* __restrict__ tiles) {
-  __shared__ double red[4];
-  const TileRef tr = tiles[blockIdx.x];
-  const SysView<VT> S = view(sys, tr.sys);
+// issued before the scalar reduction, which only the arithmetic waits for. W as in phase A.
+template <class VT, int R, bool W>
+__device__ __forceinline__ void pcg_phase_b_body(const SysView<VT>& S, int tile, double* red, double* lrows) {
+  constexpr int J = W ? 1 : R;
   gptr<PcgState> st = S.st;
-  if (load_done(st) >= 0) return;
-  const int k = st->kk;
   const int n = S.n;
-  const gptr<const VT> p = (k & 1) ? S.pb : S.pa;
-  const int base = tr.tile * kTpb * R;
-  VT xv[R], pv[R], rv[R], qv[R], dv[R];
+  const int base = tile * kTpb * R;
+  VT xv[J], pv[J], rv[J], qv[J], dv[J];
 #pragma unroll
-  for (int j = 0; j < R; ++j) {
+  for (int j = 0; j < J; ++j) {
     const int i = base + j * kTpb + threadIdx.x;
     if (i < n) {
       xv[j] = S.x[i];
-      pv[j] = p[i];
       rv[j] = S.r[i];
       qv[j] = S.q[i];
       dv[j] = S.invd[i];
     }
   }
-  const double pq = final_reduce(S.part_pq, S.ntiles, red);
+  if (load_done(st) >= 0) return;
+  const int k = st->kk;
+  const gptr<const VT> p = (k & 1) ? S.pb : S.pa;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int i = base + j * kTpb + threadIdx.x;
+    if (i < n) pv[j] = p[i];
+  }
+  const double pq = W ? final_reduce_lo(S.part_pq, S.ntiles, red) : final_reduce(S.part_pq, S.ntiles, red);
   const double rz = st->rho[k & 1];
   const double alpha = (pq != 0.0) ? rz / pq : 0.0;
-  if (tr.tile == 0 && threadIdx.x == 0) st->k = k + 1;
+  if (tile == 0 && threadIdx.x == 0) st->k = k + 1;
   const VT av = (VT)alpha;
   double rr = 0.0, rzs = 0.0;
 #pragma unroll
-  for (int j = 0; j < R; ++j) {
+  for (int j = 0; j < J; ++j) {
     const int i = base + j * kTpb + threadIdx.x;
     if (i < n) {
       S.x[i] = xv[j] + av * pv[j];
@@ -387,16 +421,36 @@ __global__ void __launch_bounds__(256) k_pcg_phase_b(const PcgSys<VT>* __restric
       const VT zi = dv[j] * ri;
       S.r[i] = ri;
       S.z[i] = zi;
-      rr += (double)ri * (double)ri;
-      rzs += (double)ri * (double)zi;
+      const double a = (double)ri * (double)ri, b = (double)ri * (double)zi;
+      if (W) {
+        rr = a;
+        rzs = b;
+      } else {
+        rr += a;
+        rzs += b;
+      }
     }
   }
-  rr = block_tree(rr, red);
-  rzs = block_tree(rzs, red);
-  if (threadIdx.x == 0) {
-    S.part_rr[tr.tile] = rr;
-    S.part_rz[tr.tile] = rzs;
+  if (W) {
+    rr = tile_tree_wide<R>(rr, lrows, red);
+    rzs = tile_tree_wide<R>(rzs, lrows, red);
+  } else {
+    rr = block_tree(rr, red);
+    rzs = block_tree(rzs, red);
   }
+  if (threadIdx.x == 0) {
+    S.part_rr[tile] = rr;
+    S.part_rz[tile] = rzs;
+  }
+}
+
+template <class VT, int R, bool W>
+__global__ void __launch_bounds__(W ? kTpb * R : kTpb) k_pcg_phase_b(const PcgSys<VT>* __restrict__ sys,
+                                                                     const TileRef* __restrict__ tiles) {
+  __shared__ double red[4];
+  __shared__ double lrows[W ? kTpb * R : 1];
+  const TileRef tr = tiles ? tiles[blockIdx.x] : TileRef{0, (int)blockIdx.x};
+  pcg_phase_b_body<VT, R, W>(view(sys[tr.sys]), tr.tile, red, lrows);
 }
 
 // ------------------------------------------------------------------ window-end stopping test
@@ -406,7 +460,7 @@ __global__ void __launch_bounds__(256) k_pcg_phase_b(const PcgSys<VT>* __restric
 template <class VT>
 __global__ void __launch_bounds__(256) k_pcg_check(const PcgSys<VT>* __restrict__ sys) {
   __shared__ double red[4];
-  const SysView<VT> S = view(sys, blockIdx.x);
+  const SysView<VT> S = view(sys[blockIdx.x]);
   gptr<PcgState> st = S.st;
   if (load_done(st) >= 0) return;
   const int k = st->k;
@@ -426,7 +480,7 @@ template <class VT, int R>
 __global__ void __launch_bounds__(256) k_pcg_finish(const PcgSys<VT>* __restrict__ sys,
                                                     const TileRef* __restrict__ tiles) {
   const TileRef tr = tiles[blockIdx.x];
-  const SysView<VT> S = view(sys, tr.sys);
+  const SysView<VT> S = view(sys[tr.sys]);
   if (!S.st->zero) return;
   const int base = tr.tile * kTpb * R;
   for (int j = 0; j < R; ++j) {
@@ -444,7 +498,7 @@ __global__ void __launch_bounds__(256) k_true_residual(const PcgSys<double>* __r
   __shared__ double red[4];
   __shared__ double lds[kSpmvLdsCap];
   const TileRef tr = tiles[xcd_block(blockIdx.x, gridDim.x)];
-  const SysView<double> S = view(sys, tr.sys);
+  const SysView<double> S = view(sys[tr.sys]);
   const int n = S.n;
   const gptr<const double> xv = G(xv_);
   const gptr<double> rvec = G(rvec_);
@@ -479,7 +533,7 @@ __global__ void __launch_bounds__(256) k_residual_batch(const PcgSys<double>* __
   __shared__ double red[4];
   __shared__ double lds[kSpmvLdsCap];
   const TileRef tr = tiles[xcd_block(blockIdx.x, gridDim.x)];
-  const SysView<double> S = view(sys, tr.sys);
+  const SysView<double> S = view(sys[tr.sys]);
   const int n = S.n;
   const gptr<const double> xv = S.x;
   auto xf = [&](int c) -> double { return xv[c]; };
@@ -590,37 +644,57 @@ void launch_pcg_init(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, in
   GSH_DISPATCH_R(rpt, k_pcg_init, VT, dim3(ntiles), dim3(kTpb), 0, s, sys, tiles);
 }
 
-template <class VT>
-void launch_pcg_iter(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s) {
-  if (ntiles <= 0) return;
-  GSH_DISPATCH_R(rpt, k_pcg_phase_a, VT, dim3(ntiles), dim3(kTpb), 0, s, sys, tiles);
-  GSH_DISPATCH_R(rpt, k_pcg_phase_b, VT, dim3(ntiles), dim3(kTpb), 0, s, sys, tiles);
+// Calls f with R as a constant.
+template <class F>
+static void with_rpt(int rpt, F&& f) {
+  switch (rpt) {
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    case 8: f(std::integral_constant<int, 8>()); break;
+    default: f(std::integral_constant<int, 4>()); break;
+  }
 }
 
-// Launch with kernel start/end stamps in e0/e1 (hipExtLaunchKernelGGL), for profiling.
-#define GSH_DISPATCH_RX(rpt, KER, VT, E0, E1, GRID, STREAM, ...)                                                \
-  switch (rpt) {                                                                                             \
-    case 1: hipExtLaunchKernelGGL(KER<VT, 1>, dim3(GRID), dim3(kTpb), 0, STREAM, E0, E1, 0, __VA_ARGS__); break;  \
-    case 2: hipExtLaunchKernelGGL(KER<VT, 2>, dim3(GRID), dim3(kTpb), 0, STREAM, E0, E1, 0, __VA_ARGS__); break;  \
-    case 8: hipExtLaunchKernelGGL(KER<VT, 8>, dim3(GRID), dim3(kTpb), 0, STREAM, E0, E1, 0, __VA_ARGS__); break;  \
-    default: hipExtLaunchKernelGGL(KER<VT, 4>, dim3(GRID), dim3(kTpb), 0, STREAM, E0, E1, 0, __VA_ARGS__); break; \
-  }
+// With e0/e1 the runtime stamps the kernel's start and end (hipExtLaunchKernelGGL), for profiling;
+// without them a plain launch, which stream capture records.
+template <class... A>
+static void launch_stamped(void (*ker)(A...), int grid, int block, hipStream_t s, hipEvent_t e0, hipEvent_t e1,
+                           A... a) {
+  if (e0 || e1)
+    hipExtLaunchKernelGGL(ker, dim3(grid), dim3(block), 0, s, e0, e1, 0, a...);
+  else
+    hipLaunchKernelGGL(ker, dim3(grid), dim3(block), 0, s, a...);
+}
+
+// Wide workgroups (R = 2, 4) up to 512 tiles, two for every CU: below that the tiles' serial
+// sub-rounds leave the chip waiting, above it the narrow form's row pointers, loaded ahead for R
+// sub-rounds, keep more in flight per register. Microseconds per Jacobi iteration, wide against
+// narrow, at R = 4: 16,000 rows 15.1 against 24.3, 66,887 14.8 against 24.2, 501,264 (490 tiles) 30.0
+// against 33.5, 1,048,576 (1,024 tiles) 53.7 against 42.3; at R = 2: 66,887 13.2 against 16.3,
+// 501,264 (980 tiles) 28.7 against 26.0.
+constexpr int kWideTiles = 512;
 
 template <class VT>
 void launch_pcg_phase(int which, const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s,
                       hipEvent_t e0, hipEvent_t e1) {
   if (ntiles <= 0) return;
-  if (!e0 && !e1) {
-    if (which == 0) {
-      GSH_DISPATCH_R(rpt, k_pcg_phase_a, VT, dim3(ntiles), dim3(kTpb), 0, s, sys, tiles);
-    } else {
-      GSH_DISPATCH_R(rpt, k_pcg_phase_b, VT, dim3(ntiles), dim3(kTpb), 0, s, sys, tiles);
-    }
-  } else if (which == 0) {
-    GSH_DISPATCH_RX(rpt, k_pcg_phase_a, VT, e0, e1, ntiles, s, sys, tiles);
-  } else {
-    GSH_DISPATCH_RX(rpt, k_pcg_phase_b, VT, e0, e1, ntiles, s, sys, tiles);
-  }
+  with_rpt(rpt, [&](auto r) {
+    constexpr int R = decltype(r)::value;
+    auto run = [&](auto wide) {
+      constexpr bool W = decltype(wide)::value;
+      launch_stamped(which == 0 ? k_pcg_phase_a<VT, R, W> : k_pcg_phase_b<VT, R, W>, ntiles, W ? kTpb * R : kTpb, s, e0,
+                     e1, sys, tiles);
+    };
+    if constexpr (R == 2 || R == 4)
+      if (ntiles <= kWideTiles) return run(std::true_type());
+    run(std::false_type());
+  });
+}
+
+template <class VT>
+void launch_pcg_iter(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s) {
+  launch_pcg_phase<VT>(0, sys, tiles, ntiles, rpt, s);
+  launch_pcg_phase<VT>(1, sys, tiles, ntiles, rpt, s);
 }
 
 template <class VT>
@@ -644,7 +718,7 @@ template void launch_pcg_iter<float>(const PcgSys<float>*, const TileRef*, int, 
 template void launch_pcg_phase<double>(int, const PcgSys<double>*, const TileRef*, int, int, hipStream_t, hipEvent_t,
                                        hipEvent_t);
 template void launch_pcg_phase<float>(int, const PcgSys<float>*, const TileRef*, int, int, hipStream_t, hipEvent_t,
-                                      hipEvent_t);
+                                       hipEvent_t);
 template void launch_pcg_check<double>(const PcgSys<double>*, int, hipStream_t);
 template void launch_pcg_check<float>(const PcgSys<float>*, int, hipStream_t);
 template void launch_pcg_finish<double>(const PcgSys<double>*, const TileRef*, int, int, hipStream_t);

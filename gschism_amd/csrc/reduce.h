@@ -69,15 +69,17 @@ __device__ __forceinline__ double block_tree_lo(double v, double* red) {
 // The partial of a tile of 256 * R rows whose workgroup has 256 * R threads, one row each, in the
 // order of a 256-thread workgroup with R rows per thread: lane position t adds the values of rows
 // t, t + 256, ..., t + 256 (R - 1) to 0.0 in that order, then block_tree. rows holds 256 * R
-// doubles of LDS; v is the thread's own row value.
-template <int R>
+// doubles of LDS; v is the thread's own row value. Wave w keeps its 64 values from rows[w * S] on
+// (S = 64: contiguous; larger: the first words of a slice the wave owns).
+template <int R, int S = 64>
 __device__ __forceinline__ double tile_tree_wide(double v, double* rows, double* red) {
-  rows[threadIdx.x] = v;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  rows[w * S + lane] = v;
   __syncthreads();
   double acc = 0.0;
   if (threadIdx.x < kTpb) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) acc += rows[j * kTpb + threadIdx.x];
+    for (int j = 0; j < R; ++j) acc += rows[(4 * j + w) * S + lane];
   }
   return block_tree_lo(acc, red);
 }

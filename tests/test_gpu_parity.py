@@ -662,3 +662,26 @@ def test_step_call_argument_errors(ctx):
     mesh.momentum(p)
     assert np.isfinite(mesh.get(L.F_SIDE_U2)).all()
     mesh.close()
+
+
+@pytest.mark.parametrize("rpt", [2, 4])
+@pytest.mark.parametrize("half", [4, 5])
+def test_wide_phases_and_long_chunks(ctx, rpt, half):
+    """Banded rows of 9 and 11 entries: 64-row chunks of exactly 576 nonzeros, the most the wide phases
+    hold in registers, and of 704, summed row by row; a last tile of a few rows. FP64 bit for bit."""
+    n = 2 * 256 * rpt + 37
+    rows = np.repeat(np.arange(n), 2 * half + 1)
+    cols = rows + np.tile(np.arange(-half, half + 1), n)
+    on = (cols >= 0) & (cols < n)
+    rows, cols = rows[on], cols[on].astype(np.int32)
+    ip = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    val = np.where(rows == cols, 2.0 * half + 0.5, -1.0 / (1.0 + np.abs(rows - cols)))
+    b = cases.normal(41, n)
+    s = core.Solver(None, ctx=ctx, indptr=ip, indices=cols)
+    s.set_tuning(rpt)
+    s.set_values(val)
+    x, it, st = s.solve(b, rtol=1e-12, maxiter=500, check_every=10)
+    xo, ito, _, _ = O.pcg(ip, cols, val, b, rtol=1e-12, maxiter=500, check_every=10, rows_per_thread=rpt)
+    assert st == 0 and it == ito
+    assert_bitwise(x, xo, f"banded solve, half width {half}, {rpt} rows per thread")
+    s.close()
