@@ -25,7 +25,10 @@ CXX = shutil.which("g++") or "g++"
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-fast-math", "-Wall",
           "-Wno-unused-function", f"-I{INCLUDE}", f"-I{CSRC}"]
 HIP_FLAGS = ["-x", "hip", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
-             "-packed-fp32-ops", "-fno-gpu-rdc"]
+             "-packed-fp32-ops", "-fno-gpu-rdc",
+             # kernel arguments arrive in scalar registers with the dispatch instead of being read
+             # from host memory by every workgroup's first instructions
+             "-mllvm", "-amdgpu-kernarg-preload-count=16"]
 HOST_SOURCES = ["gen.cpp", "topology.cpp", "ssor_layout.cpp", "grid_io.cpp"]
 HIP_SOURCES = ["mesh_kernels.hip", "pcg_kernels.hip", "ssor_kernels.hip", "block_kernels.hip", "api.hip"]
 HEADERS = ["host_mesh.h", "abi_util.h", "context.h", "device.h", "reduce.h", "ssor_layout.h"]
