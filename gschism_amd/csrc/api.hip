@@ -93,6 +93,11 @@ __global__ void k_extrapolate(double* __restrict__ x, const double* __restrict__
   if (i < n) x[i] = (3.0 * h0[i] - 3.0 * h1[i]) + h2[i];
 }
 
+__global__ void k_fill_words(uint64_t* __restrict__ p, int count) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < count) p[i] = 0;
+}
+
 __global__ void k_pack_uvw(const double* __restrict__ in, double* __restrict__ out, int64_t cnt) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= cnt) return;
@@ -235,6 +240,11 @@ struct gsh_solver {
   PcgSys<double>* ds = nullptr;
   TileRef* dtiles = nullptr;   // tiles of this system alone
   double* red2 = nullptr;      // scratch for two reduced scalars
+  // whole-solve launches (launch_pcg_run): exchange words, the next launch's first epoch, and the
+  // pattern's longest row and largest |column - row|
+  uint64_t* run_words = nullptr;
+  uint32_t run_epoch = 1;
+  int32_t max_row = 0, band = 0;
   // mixed precision
   float* val32 = nullptr;
   double* r64 = nullptr;
@@ -305,6 +315,11 @@ static void solver_alloc(gsh_solver* s, int32_t n, int64_t nnz, const std::vecto
   s->ds = P.alloc<PcgSys<double>>(1);
   s->dtiles = P.alloc<TileRef>(nt);
   s->red2 = P.alloc<double>(2);
+  s->run_words = P.alloc<uint64_t>(kRunWords);
+  for (int32_t i = 0; i < n; ++i) {
+    s->max_row = std::max(s->max_row, indptr[i + 1] - indptr[i]);
+    for (int32_t k = indptr[i]; k < indptr[i + 1]; ++k) s->band = std::max(s->band, std::abs(indices[k] - i));
+  }
   if (s->precision == GSH_PREC_MIXED) {
     s->val32 = P.alloc<float>(nnz);
     s->r64 = P.alloc<double>(n);
@@ -541,12 +556,14 @@ struct PhaseTimes {
 
 // The iteration loop itself: dgather (device, 2 * nsys states) stages the window readbacks and
 // the final states land in the context's pinned slots 0..nsys-1. It allocates nothing when the
-// pinned slots already hold 2 * nsys states and no profile is asked for.
+// pinned slots already hold 2 * nsys states and no profile is asked for. solo: the solver of a
+// single system whose pattern was counted on the host (its small systems run whole in a launch).
+constexpr int kRunIters = 512;  // iterations of a launch at most (milliseconds, so time limits hold)
 template <class VT>
 static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const TileRef* dtiles, int ntiles, int rpt,
                          double rtol, int maxiter, int check_every, double timeout_s, PcgState* dgather,
                          const TileRef* dinit_tiles, int ninit_tiles, PhaseTimes* prof, const double* rtols_dev,
-                         WindowGraph* graph) {
+                         WindowGraph* graph, gsh_solver* solo) {
   hipStream_t st = ctx->stream;
   if (check_every < 1) check_every = 1;
   if (timeout_s <= 0.0) timeout_s = 60.0;
@@ -558,6 +575,30 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
   else
     launch_pcg_init<VT>(dsys, dtiles, ntiles, rpt, st);
   HIPCHK(hipGetLastError());
+  if (solo && !prof && !(graph && graph->enabled) && pcg_run_fits(ntiles, rpt, solo->max_row, solo->band)) {
+    // a small system: hundreds of iterations per launch, which stops itself at the passing test
+    const auto t0 = Clock::now();
+    for (int issued = 0;;) {
+      const int w = std::min(kRunIters, maxiter - issued);
+      if (solo->run_epoch > 0xffff0000u) {  // the words start again at epoch 0, as when they were allocated
+        hipLaunchKernelGGL(k_fill_words, dim3((kRunWords + 255) / 256), dim3(256), 0, st, solo->run_words, kRunWords);
+        solo->run_epoch = 1;
+      }
+      launch_pcg_run<VT>(dsys, ntiles, rpt, solo->run_words, solo->run_epoch, solo->band, w, st);
+      solo->run_epoch += (uint32_t)w + 1;
+      issued += w;
+      launch_pcg_finish<VT>(dsys, dtiles, ntiles, rpt, st);
+      hipLaunchKernelGGL(k_gather_states<VT>, dim3(1), dim3(64), 0, st, dsys, 1, dgather);
+      HIPCHK(hipMemcpyAsync(slots, dgather, sizeof(PcgState), hipMemcpyDeviceToHost, st));
+      HIPCHK(hipEventRecord(ctx->ev[0], st));
+      HIPCHK(hipGetLastError());
+      wait_event(ctx->ev[0], timeout_s, "PCG launch");
+      if (slots[0].pad0) throw Error(GSH_E_DEVICE, "PCG: the workgroups of a launch did not meet");
+      if (slots[0].done >= 0 || issued >= maxiter) return;
+      if (std::chrono::duration<double>(Clock::now() - t0).count() > timeout_s)
+        throw Error(GSH_E_TIMEOUT, "PCG: time limit exceeded while issuing iterations");
+    }
+  }
   int issued = 0, window = 0;
   int inflight[2], nflight = 0;  // windows pending readback (slot = window & 1), oldest first
   bool all_done = false;
@@ -629,11 +670,12 @@ template <class VT>
 static void run_pcg(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const TileRef* dtiles, int ntiles, int rpt,
                     double rtol, int maxiter, int check_every, double timeout_s, PcgOutcome& out,
                     const TileRef* dinit_tiles = nullptr, int ninit_tiles = -1, PhaseTimes* prof = nullptr,
-                    const double* rtols_dev = nullptr, WindowGraph* graph = nullptr) {
+                    const double* rtols_dev = nullptr, WindowGraph* graph = nullptr,
+                    gsh_solver* solo = nullptr) {
   StreamBuffers tmp(ctx->stream);
   PcgState* dgather = tmp.alloc<PcgState>(2 * (size_t)nsys);
   run_pcg_core<VT>(ctx, dsys, nsys, dtiles, ntiles, rpt, rtol, maxiter, check_every, timeout_s, dgather, dinit_tiles,
-                   ninit_tiles, prof, rtols_dev, graph);
+                   ninit_tiles, prof, rtols_dev, graph, solo);
   const PcgState* slots = ctx->pinned;
   out.st.assign(slots, slots + nsys);
 }
@@ -1038,7 +1080,7 @@ static void run_mixed(gsh_ctx* ctx, gsh_solver* const* S, int count, double rtol
       HIPCHK(hipMemcpyAsync(dtl, stl.data(), sizeof(TileRef) * stl.size(), hipMemcpyHostToDevice, st));
       HIPCHK(hipMemcpyAsync(drt, rts.data(), sizeof(double) * ns, hipMemcpyHostToDevice, st));
       run_pcg<float>(ctx, d32s, ns, dtl, (int)stl.size(), rpt, rtol, maxiter, check_every, timeout_s, o, nullptr, -1,
-                     nullptr, drt);
+                     nullptr, drt, nullptr, ns == 1 ? S[sub[0]] : nullptr);
       launch_refine_batch(d64s, d32s, dtl, (int)stl.size(), rpt, st);
     }
     for (int j = 0; j < ns; ++j) {
@@ -2049,7 +2091,7 @@ int gsh_solver_solve(gsh_solver* s, const double* b_host, double* x_host, double
     } else {
       PcgOutcome o;
       run_pcg<double>(s->ctx, s->ds, 1, s->dtiles, s->ntiles, s->rpt, rtol, maxiter, check_every, timeout_s, o,
-                      nullptr, -1, nullptr, nullptr, &s->wg_jacobi);
+                      nullptr, -1, nullptr, nullptr, &s->wg_jacobi, s);
       const PcgState& r = o.st[0];
       iters = iters_of(r, maxiter);
       status = (r.done >= 0) ? 0 : GSH_W_MAXITER;
@@ -2133,7 +2175,7 @@ int gsh_pcg_solve_static(gsh_ctx* ctx, int32_t n, int64_t nnz, const int32_t* in
     hipLaunchKernelGGL(k_static_desc, dim3(1), dim3(1), 0, st, h, dsys);
     HIPCHK(hipGetLastError());
     run_pcg_core<double>(ctx, dsys, 1, dtiles, ntiles, kStaticRpt, rtol, maxiter, check_every, timeout_s, dgather,
-                         nullptr, -1, nullptr, nullptr, nullptr);
+                         nullptr, -1, nullptr, nullptr, nullptr, nullptr);
     const PcgState r = ctx->pinned[0];
     if (iters_out) *iters_out = iters_of(r, maxiter);
     if (status_out) *status_out = (r.done >= 0) ? 0 : GSH_W_MAXITER;

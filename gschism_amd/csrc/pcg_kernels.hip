@@ -95,6 +95,7 @@ __global__ void k_pcg_reset(const PcgSys<VT>* sys, int nsys, double rtol, int ma
   st->bb = 0.0;
   st->rho[0] = 0.0;
   st->rho[1] = 0.0;
+  st->pad0 = 0;
 }
 
 // ------------------------------------------------------------------ CSR row sums (block staged)
@@ -453,6 +454,310 @@ __global__ void __launch_bounds__(W ? kTpb * R : kTpb) k_pcg_phase_b(const PcgSy
   pcg_phase_b_body<VT, R, W>(view(sys[tr.sys]), tr.tile, red, lrows);
 }
 
+// ------------------------------------------------------------------ whole solve in one launch
+// Many iterations of one small system in one launch: one workgroup of 256 R threads per tile, one
+// row per thread. The row's matrix entries, x, r, z and the inverse diagonal stay in registers, p of
+// the tile and of the rows its columns reach (the halo: within the matrix bandwidth of the tile)
+// in LDS, where every workgroup updates its own copy of the halo's p from z. So per iteration the
+// workgroups exchange two tile sums (p.q; r.r and r.z) and z of the halo. Arithmetic, partial trees
+// and stopping rule are those of the two phases, and so are the bits.
+//
+// The exchange: agent-scope relaxed atomic stores and loads, which no XCD's L2 answers from a stale
+// line. A double travels as two 64-bit words of (epoch, 32 bits), each word whole in itself; every
+// workgroup polls all tiles' words until they carry the exchange's epoch, which is both the sum's
+// transport and the grid barrier, in one trip. z is performed (s_waitcnt) before the r.r, r.z words
+// that announce it. The words of p.q are not overwritten before all have read them: the next p.q
+// comes after an r.r, r.z exchange, which each workgroup enters when it has read p.q, and likewise
+// the other way round.
+//
+// Why: an iteration of the phases on a small system is two launches, each of which waits for its
+// dispatch and for five dependent loads before its first product: 12-15 us at 384 to 66,887 rows,
+// where the matrix and vectors would take 1-3 us from the caches. Here (us per iteration, R = 4):
+// 384 rows (one workgroup, no exchange) 4.2 against 12.4 with the solve's set-up, 16,000 rows 6.1
+// against 15.1, 66,887 rows 6.6 against 14.8, 128,000 rows 7.0 against 17. Up to kRunTiles workgroups: an exchange takes 1.2 us among 32, 2.3 among 128, and
+// 128 never take more than a quarter of the chip's workgroup slots, so that solves on other streams
+// stay resident beside them.
+constexpr int kRunTiles = 128;
+constexpr int kRunRow = 12;     // entries of a row held in registers
+constexpr int kRunWin = 6144;   // p of the tile and its halo, words of LDS
+constexpr int kSpin = 1 << 24;  // polls before a launch gives up (tens of seconds)
+
+template <class T>
+__device__ __forceinline__ T ld_agent(gptr<const T> p) {
+  if constexpr (sizeof(T) == 8) {
+    const uint64_t v = __hip_atomic_load((gptr<const uint64_t>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(T, v);
+  } else {
+    const uint32_t v = __hip_atomic_load((gptr<const uint32_t>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(T, v);
+  }
+}
+template <class T>
+__device__ __forceinline__ void st_agent(gptr<T> p, T x) {
+  if constexpr (sizeof(T) == 8)
+    __hip_atomic_store((gptr<uint64_t>)p, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    __hip_atomic_store((gptr<uint32_t>)p, __builtin_bit_cast(uint32_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The tile partials of N sums at once, in the R-rows-per-thread order (tile_tree_wide), returned to
+// every thread. rows: N x 256 R words, red: N x 4. With drain, the workgroup's earlier stores are
+// performed when it returns.
+template <int R, int N>
+__device__ __forceinline__ void run_tile_sums(double (&v)[N], double* rows, double* red, bool drain) {
+  const int tid = threadIdx.x, w = tid >> 6;
+#pragma unroll
+  for (int a = 0; a < N; ++a) rows[a * kTpb * R + tid] = v[a];
+  __syncthreads();
+  if (tid < kTpb) {
+#pragma unroll
+    for (int a = 0; a < N; ++a) {
+      double acc = 0.0;
+#pragma unroll
+      for (int j = 0; j < R; ++j) acc += rows[a * kTpb * R + j * kTpb + tid];
+      acc = wave_tree(acc);
+      if ((tid & 63) == 0) red[4 * a + w] = acc;
+    }
+  }
+  if (drain) {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < N; ++a) v[a] = (red[4 * a] + red[4 * a + 1]) + (red[4 * a + 2] + red[4 * a + 3]);
+}
+
+// Sums over the T <= 128 tile partials (thread t holds tile t's) in final_reduce's order.
+template <int N>
+__device__ __forceinline__ void run_totals(double (&v)[N], double* red) {
+  const int tid = threadIdx.x, w = tid >> 6;
+  if (w < 4) {
+#pragma unroll
+    for (int a = 0; a < N; ++a) {
+      const double u = wave_tree(0.0 + v[a]);
+      if ((tid & 63) == 0) red[4 * a + w] = u;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < N; ++a) v[a] = (red[4 * a] + red[4 * a + 1]) + (red[4 * a + 2] + red[4 * a + 3]);
+}
+
+// Publishes this tile's N partials (v, the same in every thread) and returns in v of thread t < T
+// tile t's, 0 in the others. False in a thread that gave up.
+template <int N>
+__device__ __forceinline__ bool run_exchange(double (&v)[N], gptr<uint64_t> words, int tile, int T, uint32_t epoch) {
+  const int tid = threadIdx.x;
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  if (tid < 2 * N) {
+    double x = v[0];
+#pragma unroll
+    for (int a = 1; a < N; ++a)
+      if ((tid >> 1) == a) x = v[a];
+    const uint64_t bits = __builtin_bit_cast(uint64_t, x);
+    const uint32_t half = (tid & 1) ? (uint32_t)(bits >> 32) : (uint32_t)bits;
+    st_agent(words + (int64_t)tile * 2 * N + tid, ((uint64_t)epoch << 32) | half);
+  }
+  bool ok = true;
+  if (tid < T) {
+    uint64_t u[2 * N];
+    for (int spin = 0;;) {
+#pragma unroll
+      for (int a = 0; a < 2 * N; ++a) u[a] = ld_agent((gptr<const uint64_t>)words + (int64_t)tid * 2 * N + a);
+      bool all = true;
+#pragma unroll
+      for (int a = 0; a < 2 * N; ++a) all = all && (uint32_t)(u[a] >> 32) == epoch;
+      if (all) break;
+      if (++spin == kSpin) {
+        ok = false;
+        break;
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < N; ++a) v[a] = __builtin_bit_cast(double, (u[2 * a] & 0xffffffffull) | (u[2 * a + 1] << 32));
+  } else {
+#pragma unroll
+    for (int a = 0; a < N; ++a) v[a] = 0.0;
+  }
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  return ok;
+}
+
+// words: 6 x 128 exchange words of the solver; epoch0: the launch's first epoch, above every earlier
+// launch's; band: the largest |column - row|; iters: iterations at most.
+template <class VT, int R, bool SOLO>
+__global__ void __launch_bounds__(kTpb * R) k_pcg_run(const PcgSys<VT>* __restrict__ sys, uint64_t* __restrict__ words_,
+                                                      uint32_t epoch0, int band, int iters) {
+  constexpr int kRows = kTpb * R;
+  __shared__ double red[8], redt[8], rows[2 * kRows];
+  __shared__ int stuck;
+  __shared__ VT win[SOLO ? kRows : kRunWin];
+  const SysView<VT> S = view(*sys);
+  gptr<PcgState> st = S.st;
+  const gptr<uint64_t> wpq = G(words_), wrr = wpq + 2 * kRunTiles;
+  const int n = S.n, T = S.ntiles, tile = blockIdx.x, tid = threadIdx.x;
+  const int base = tile * kRows, i = base + tid;
+  const bool in = i < n;
+  const int lo = SOLO ? 0 : max(0, base - band), hi = SOLO ? n : min(n, base + kRows + band);
+  const int below = base - lo, halo = (hi - lo) - (min(n, base + kRows) - base);
+  // halo word h: rows below the tile, then rows above it
+  auto halo_row = [&](int h) { return h < below ? lo + h : base + kRows + (h - below); };
+  if (tid == 0) stuck = 0;
+  if (load_done(st) >= 0) return;
+  const int check_every = st->check_every, maxiter = st->maxiter;
+  int k = st->k;
+  const gptr<const VT> pold = (k & 1) ? S.pa : S.pb;
+  VT v[kRunRow];
+  int c[kRunRow];
+  VT x = 0, r = 0, z = 0, p = 0, invd = 0;
+  int len = 0;
+  if (in) {
+    const int a = S.rowptr[i];
+    len = S.rowptr[i + 1] - a;
+#pragma unroll
+    for (int m = 0; m < kRunRow; ++m) {
+      v[m] = 0;
+      c[m] = i - lo;
+      if (m < len) {
+        v[m] = S.val[a + m];
+        c[m] = S.col[a + m] - lo;
+      }
+    }
+    x = S.x[i];
+    r = S.r[i];
+    z = S.z[i];
+    p = pold[i];
+    invd = S.invd[i];
+    win[i - lo] = p;
+  }
+  if (!SOLO)
+    for (int h = tid; h < halo; h += kRows) {
+      const int row = halo_row(h);
+      win[row - lo] = pold[row];
+    }
+  double rz_cur, rz_old = 0.0, rr_last = st->rr_last, atol2;
+  double part[2] = {tid < T ? S.part_rz[tid] : 0.0, (k == 0 && tid < T) ? S.part_bb[tid] : 0.0};
+  run_totals(part, redt);
+  rz_cur = part[0];
+  int done = -1;
+  if (k == 0) {  // atol = rtol ||b|| (pcg_solver.py:928-930, 1089-1095)
+    const double atol = st->rtol * sqrt(part[1]);
+    atol2 = atol * atol;
+    if (tile == 0 && tid == 0) {
+      st->bb = part[1];
+      st->atol2 = atol2;
+      if (atol == 0.0) {
+        st->zero = 1;
+        st->done = 0;
+      }
+    }
+    if (atol == 0.0) return;
+  } else {
+    atol2 = st->atol2;
+    rz_old = st->rho[(k - 1) & 1];
+  }
+  uint32_t epoch = epoch0;
+  double t2[2] = {0.0, 0.0};
+  for (int it = 0; it < iters; ++it) {
+    // phase A(k): p = z + beta p on the window, q = A p
+    const VT bv = (VT)((k > 0 && rz_old != 0.0) ? rz_cur / rz_old : 0.0);
+    if (!SOLO)
+      for (int h0 = tid; h0 < halo; h0 += 4 * kRows) {
+        VT zh[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int h = h0 + u * kRows;
+          // the first launch iteration reads what an earlier launch stored, all others a neighbour's
+          zh[u] = h < halo ? ld_agent((gptr<const VT>)S.z + halo_row(h)) : (VT)0;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int h = h0 + u * kRows;
+          if (h < halo) {
+            const int j = halo_row(h) - lo;
+            win[j] = zh[u] + bv * win[j];
+          }
+        }
+      }
+    if (in) {
+      p = z + bv * p;
+      win[i - lo] = p;
+    }
+    __syncthreads();
+    VT q = 0;
+    if (in) {
+      VT pw[kRunRow];
+#pragma unroll
+      for (int m = 0; m < kRunRow; ++m) pw[m] = win[c[m]];
+#pragma unroll
+      for (int m = 0; m < kRunRow; ++m)
+        if (m < len) q += v[m] * pw[m];
+    }
+    double t1[1] = {in ? (double)p * (double)q : 0.0};
+    run_tile_sums<R>(t1, rows, red, false);
+    if (!SOLO) {
+      if (!run_exchange(t1, wpq, tile, T, epoch)) stuck = 1;
+    } else if (tid != 0) {
+      t1[0] = 0.0;
+    }
+    run_totals(t1, redt);
+    // phase B(k)
+    const double pq = t1[0];
+    const VT av = (VT)((pq != 0.0) ? rz_cur / pq : 0.0);
+    t2[0] = t2[1] = 0.0;
+    if (in) {
+      x = x + av * p;
+      r = r - av * q;
+      z = invd * r;
+      if (!SOLO) st_agent(S.z + i, z);
+      t2[0] = (double)r * (double)r;
+      t2[1] = (double)r * (double)z;
+    }
+    run_tile_sums<R>(t2, rows, red, !SOLO);
+    double s2[2] = {t2[0], t2[1]};
+    if (!SOLO) {
+      if (!run_exchange(s2, wrr, tile, T, epoch)) stuck = 1;
+    } else if (tid != 0) {
+      s2[0] = s2[1] = 0.0;
+    }
+    run_totals(s2, redt);
+    if (!SOLO && stuck) break;  // set before run_totals' barrier, so the same in every thread
+    ++epoch;
+    rz_old = rz_cur;
+    rz_cur = s2[1];
+    ++k;
+    if (k % check_every == 0 || k == maxiter) {
+      rr_last = s2[0];
+      if (rr_last <= atol2) {
+        done = k;
+        break;
+      }
+    }
+  }
+  if (!SOLO && stuck) {
+    if (tid == 0) st->pad0 = 1;
+    return;
+  }
+  if (in) {
+    S.x[i] = x;
+    S.r[i] = r;
+    S.z[i] = z;
+    ((k & 1) ? S.pa : S.pb)[i] = p;
+  }
+  if (tid == 0) {
+    S.part_rr[tile] = t2[0];
+    S.part_rz[tile] = t2[1];
+    if (tile == 0) {
+      st->rho[(k - 1) & 1] = rz_old;
+      st->rr_last = rr_last;
+      st->k = k;
+      st->kk = k - 1;
+      if (done >= 0) st->done = done;
+    }
+  }
+}
+
 // ------------------------------------------------------------------ window-end stopping test
 // The test of iteration k-1 normally runs at the start of phase A(k); at the end of a window of
 // launches this kernel runs it (one workgroup per system) so the host sees the flag at once.
@@ -697,6 +1002,25 @@ void launch_pcg_iter(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, in
   launch_pcg_phase<VT>(1, sys, tiles, ntiles, rpt, s);
 }
 
+bool pcg_run_fits(int ntiles, int rpt, int max_row, int band) {
+  return ntiles >= 1 && ntiles <= kRunTiles && (rpt == 1 || rpt == 2 || rpt == 4) && max_row <= kRunRow &&
+         (ntiles == 1 || kTpb * rpt + 2 * (int64_t)band <= kRunWin);
+}
+
+template <class VT>
+void launch_pcg_run(const PcgSys<VT>* sys, int ntiles, int rpt, uint64_t* words, uint32_t epoch, int band, int iters,
+                    hipStream_t s) {
+  with_rpt(rpt, [&](auto r) {
+    constexpr int R = decltype(r)::value;
+    if constexpr (R <= 4) {
+      if (ntiles == 1)
+        launch_stamped(k_pcg_run<VT, R, true>, 1, kTpb * R, s, nullptr, nullptr, sys, words, epoch, band, iters);
+      else
+        launch_stamped(k_pcg_run<VT, R, false>, ntiles, kTpb * R, s, nullptr, nullptr, sys, words, epoch, band, iters);
+    }
+  });
+}
+
 template <class VT>
 void launch_pcg_check(const PcgSys<VT>* sys, int nsys, hipStream_t s) {
   if (nsys <= 0) return;
@@ -719,6 +1043,8 @@ template void launch_pcg_phase<double>(int, const PcgSys<double>*, const TileRef
                                        hipEvent_t);
 template void launch_pcg_phase<float>(int, const PcgSys<float>*, const TileRef*, int, int, hipStream_t, hipEvent_t,
                                        hipEvent_t);
+template void launch_pcg_run<double>(const PcgSys<double>*, int, int, uint64_t*, uint32_t, int, int, hipStream_t);
+template void launch_pcg_run<float>(const PcgSys<float>*, int, int, uint64_t*, uint32_t, int, int, hipStream_t);
 template void launch_pcg_check<double>(const PcgSys<double>*, int, hipStream_t);
 template void launch_pcg_check<float>(const PcgSys<float>*, int, hipStream_t);
 template void launch_pcg_finish<double>(const PcgSys<double>*, const TileRef*, int, int, hipStream_t);

@@ -685,3 +685,31 @@ def test_wide_phases_and_long_chunks(ctx, rpt, half):
     assert st == 0 and it == ito
     assert_bitwise(x, xo, f"banded solve, half width {half}, {rpt} rows per thread")
     s.close()
+
+
+@pytest.mark.parametrize("rpt,n,maxiter", [(4, 1, 50), (4, 1023, 200), (4, 1024, 200), (4, 1025, 200), (1, 257, 1100),
+                                           (2, 5000, 1100), (4, 131072, 40), (4, 131073, 40), (1, 300, 7)])
+def test_small_systems_in_one_launch(ctx, rpt, n, maxiter):
+    """Systems around one tile and around the most tiles that run whole in a launch; 1,100 iterations
+    take three launches, which resume each other; stops at maxiter off the check interval; twice, the
+    second time from the history of the first. FP64 bit for bit."""
+    rows = np.repeat(np.arange(n), 5)
+    cols = rows + np.tile([-37, -1, 0, 1, 37], n)
+    on = (cols >= 0) & (cols < n)
+    rows, cols = rows[on], cols[on].astype(np.int32)
+    ip = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    val = np.where(rows == cols, 4.0 + 1e-6 * (rows % 7), -1.0)
+    hist = [np.zeros(n)] * 3
+    s = core.Solver(None, ctx=ctx, indptr=ip, indices=cols)
+    s.set_tuning(rpt)
+    s.set_values(val)
+    print(f"[gpu] one-launch solve, n={n}, {rpt} rows per thread", flush=True)
+    for rep in range(2):
+        b = cases.normal(50 + rep, n)
+        x, it, st = s.solve(b, rtol=1e-14, maxiter=maxiter, check_every=10)
+        xo, ito, _, _ = O.pcg(ip, cols, val, b, hist=hist, rtol=1e-14, maxiter=maxiter, check_every=10,
+                              rows_per_thread=rpt, nthreads=8)
+        assert it == ito
+        assert_bitwise(x, xo, f"solution {rep}")
+        hist = [xo] + hist[:2]
+    s.close()
