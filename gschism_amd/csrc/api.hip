@@ -492,6 +492,35 @@ static void solver_roll(gsh_solver* s) {
 }
 
 // ---------------------------------------------------------------------- PCG driver
+// Whole-solve launches wait for their own workgroups, so those of all streams together must fit the
+// device: the solves of this process hold slots of it while they run, and a solve that gets none
+// takes the launches per phase. (Other processes are not counted; see the launches' bounded wait.)
+struct RunSlots {
+  static constexpr int kSlots = 256;  // workgroups of up to 1,024 threads resident on any device here
+  static std::atomic<int>& used(int device) {
+    static std::atomic<int> u[64];
+    return u[device & 63];
+  }
+  std::atomic<int>* u = nullptr;
+  int n = 0;
+  RunSlots(int device, int wgs) {
+    if (wgs <= 0) return;
+    std::atomic<int>& a = used(device);
+    if (a.fetch_add(wgs) + wgs > kSlots) {
+      a.fetch_sub(wgs);
+      return;
+    }
+    u = &a;
+    n = wgs;
+  }
+  ~RunSlots() {
+    if (u) u->fetch_sub(n);
+  }
+  RunSlots(const RunSlots&) = delete;
+  RunSlots& operator=(const RunSlots&) = delete;
+  explicit operator bool() const { return u != nullptr; }
+};
+
 struct PcgOutcome {
   std::vector<PcgState> st;
 };
@@ -559,6 +588,7 @@ struct PhaseTimes {
 // pinned slots already hold 2 * nsys states and no profile is asked for. solo: the solver of a
 // single system whose pattern was counted on the host (its small systems run whole in a launch).
 constexpr int kRunIters = 512;  // iterations of a launch at most (milliseconds, so time limits hold)
+constexpr uint32_t kRunEpochs = 0xffff0000u;  // last first epoch of a launch before the words are cleared
 template <class VT>
 static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const TileRef* dtiles, int ntiles, int rpt,
                          double rtol, int maxiter, int check_every, double timeout_s, PcgState* dgather,
@@ -575,13 +605,15 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
   else
     launch_pcg_init<VT>(dsys, dtiles, ntiles, rpt, st);
   HIPCHK(hipGetLastError());
-  if (solo && !prof && !(graph && graph->enabled) && pcg_run_fits(ntiles, rpt, solo->max_row, solo->band)) {
+  const bool fits = solo && !prof && !(graph && graph->enabled) && pcg_run_fits(ntiles, rpt, solo->max_row, solo->band);
+  if (const RunSlots held(ctx->device, fits ? ntiles : 0); held) {
     // a small system: hundreds of iterations per launch, which stops itself at the passing test
     const auto t0 = Clock::now();
     for (int issued = 0;;) {
       const int w = std::min(kRunIters, maxiter - issued);
-      if (solo->run_epoch > 0xffff0000u) {  // the words start again at epoch 0, as when they were allocated
-        hipLaunchKernelGGL(k_fill_words, dim3((kRunWords + 255) / 256), dim3(256), 0, st, solo->run_words, kRunWords);
+      if (solo->run_epoch > kRunEpochs) {  // the words start again at epoch 0, as when they were allocated
+        hipLaunchKernelGGL(k_fill_words, dim3((kRunWords + 255) / 256), dim3(256), 0, st, solo->run_words,
+                           kRunWords);
         solo->run_epoch = 1;
       }
       launch_pcg_run<VT>(dsys, ntiles, rpt, solo->run_words, solo->run_epoch, solo->band, w, st);
@@ -593,11 +625,13 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
       HIPCHK(hipEventRecord(ctx->ev[0], st));
       HIPCHK(hipGetLastError());
       wait_event(ctx->ev[0], timeout_s, "PCG launch");
-      if (slots[0].pad0) throw Error(GSH_E_DEVICE, "PCG: the workgroups of a launch did not meet");
+      if (slots[0].pad0) break;  // its workgroups did not meet: the phases solve it, from the start
       if (slots[0].done >= 0 || issued >= maxiter) return;
       if (std::chrono::duration<double>(Clock::now() - t0).count() > timeout_s)
         throw Error(GSH_E_TIMEOUT, "PCG: time limit exceeded while issuing iterations");
     }
+    launch_pcg_reset<VT>(dsys, nsys, rtol, maxiter, check_every, st, rtols_dev);
+    launch_pcg_init<VT>(dsys, dtiles, ntiles, rpt, st);
   }
   int issued = 0, window = 0;
   int inflight[2], nflight = 0;  // windows pending readback (slot = window & 1), oldest first

@@ -474,31 +474,14 @@ __global__ void __launch_bounds__(W ? kTpb * R : kTpb) k_pcg_phase_b(const PcgSy
 // dispatch and for five dependent loads before its first product: 12-15 us at 384 to 66,887 rows,
 // where the matrix and vectors would take 1-3 us from the caches. Here (us per iteration, R = 4):
 // 384 rows (one workgroup, no exchange) 4.2 against 12.4 with the solve's set-up, 16,000 rows 6.1
-// against 15.1, 66,887 rows 6.6 against 14.8, 128,000 rows 7.0 against 17. Up to kRunTiles workgroups: an exchange takes 1.2 us among 32, 2.3 among 128, and
-// 128 never take more than a quarter of the chip's workgroup slots, so that solves on other streams
-// stay resident beside them.
+// against 15.1, 66,887 rows 6.6 against 14.8, 128,000 rows 7.0 against 17. Up to kRunTiles
+// workgroups: an exchange takes 1.2 us among 32, 2.3 among 128, and at one workgroup of 1,024 threads
+// per CU two such launches are resident together (the host admits no more, RunSlots). A launch whose
+// workgroups do not become resident together all the same (another process's solve) gives up after
+// kRunSpin polls and leaves the solve to the phases.
 constexpr int kRunTiles = 128;
 constexpr int kRunRow = 12;     // entries of a row held in registers
 constexpr int kRunWin = 6144;   // p of the tile and its halo, words of LDS
-constexpr int kSpin = 1 << 24;  // polls before a launch gives up (tens of seconds)
-
-template <class T>
-__device__ __forceinline__ T ld_agent(gptr<const T> p) {
-  if constexpr (sizeof(T) == 8) {
-    const uint64_t v = __hip_atomic_load((gptr<const uint64_t>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return __builtin_bit_cast(T, v);
-  } else {
-    const uint32_t v = __hip_atomic_load((gptr<const uint32_t>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return __builtin_bit_cast(T, v);
-  }
-}
-template <class T>
-__device__ __forceinline__ void st_agent(gptr<T> p, T x) {
-  if constexpr (sizeof(T) == 8)
-    __hip_atomic_store((gptr<uint64_t>)p, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else
-    __hip_atomic_store((gptr<uint32_t>)p, __builtin_bit_cast(uint32_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // The tile partials of N sums at once, in the R-rows-per-thread order (tile_tree_wide), returned to
 // every thread. rows: N x 256 R words, red: N x 4. With drain, the workgroup's earlier stores are
@@ -519,10 +502,7 @@ __device__ __forceinline__ void run_tile_sums(double (&v)[N], double* rows, doub
       if ((tid & 63) == 0) red[4 * a + w] = acc;
     }
   }
-  if (drain) {
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0);
-  }
+  if (drain) wait_stores();
   __syncthreads();
 #pragma unroll
   for (int a = 0; a < N; ++a) v[a] = (red[4 * a] + red[4 * a + 1]) + (red[4 * a + 2] + red[4 * a + 3]);
@@ -555,9 +535,7 @@ __device__ __forceinline__ bool run_exchange(double (&v)[N], gptr<uint64_t> word
 #pragma unroll
     for (int a = 1; a < N; ++a)
       if ((tid >> 1) == a) x = v[a];
-    const uint64_t bits = __builtin_bit_cast(uint64_t, x);
-    const uint32_t half = (tid & 1) ? (uint32_t)(bits >> 32) : (uint32_t)bits;
-    st_agent(words + (int64_t)tile * 2 * N + tid, ((uint64_t)epoch << 32) | half);
+    st_agent(words + (int64_t)tile * 2 * N + tid, run_word(x, tid & 1, epoch));
   }
   bool ok = true;
   if (tid < T) {
@@ -569,13 +547,13 @@ __device__ __forceinline__ bool run_exchange(double (&v)[N], gptr<uint64_t> word
 #pragma unroll
       for (int a = 0; a < 2 * N; ++a) all = all && (uint32_t)(u[a] >> 32) == epoch;
       if (all) break;
-      if (++spin == kSpin) {
+      if (++spin == kRunSpin) {
         ok = false;
         break;
       }
     }
 #pragma unroll
-    for (int a = 0; a < N; ++a) v[a] = __builtin_bit_cast(double, (u[2 * a] & 0xffffffffull) | (u[2 * a + 1] << 32));
+    for (int a = 0; a < N; ++a) v[a] = run_value(u[2 * a], u[2 * a + 1]);
   } else {
 #pragma unroll
     for (int a = 0; a < N; ++a) v[a] = 0.0;

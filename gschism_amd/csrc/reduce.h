@@ -84,6 +84,43 @@ __device__ __forceinline__ double tile_tree_wide(double v, double* rows, double*
   return block_tree_lo(acc, red);
 }
 
+// Agent-scope relaxed accesses for what the workgroups of one launch exchange: written through to
+// where every XCD sees them, read past lines that may be stale. A store is performed when
+// s_waitcnt says so (wait_stores).
+template <class T>
+__device__ __forceinline__ T ld_agent(gptr<const T> p) {
+  if constexpr (sizeof(T) == 8) {
+    const uint64_t v = __hip_atomic_load((gptr<const uint64_t>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(T, v);
+  } else {
+    const uint32_t v = __hip_atomic_load((gptr<const uint32_t>)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(T, v);
+  }
+}
+template <class T>
+__device__ __forceinline__ void st_agent(gptr<T> p, T x) {
+  if constexpr (sizeof(T) == 8)
+    __hip_atomic_store((gptr<uint64_t>)p, __builtin_bit_cast(uint64_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+    __hip_atomic_store((gptr<uint32_t>)p, __builtin_bit_cast(uint32_t, x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void wait_stores() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0);
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+constexpr int kRunSpin = 1 << 16;  // polls before a workgroup gives up on the others (tens of milliseconds)
+
+// A double as two 64-bit words of (epoch, 32 bits): each word is whole in itself, so a reader knows
+// from the epochs when it has the value.
+__device__ __forceinline__ uint64_t run_word(double v, int half, uint32_t epoch) {
+  const uint64_t bits = __builtin_bit_cast(uint64_t, v);
+  return ((uint64_t)epoch << 32) | (half ? (uint32_t)(bits >> 32) : (uint32_t)bits);
+}
+__device__ __forceinline__ double run_value(uint64_t w0, uint64_t w1) {
+  return __builtin_bit_cast(double, (w0 & 0xffffffffull) | (w1 << 32));
+}
+
 // Orders LDS writes before reads among the lanes of one wave.
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

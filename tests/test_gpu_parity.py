@@ -713,3 +713,39 @@ def test_small_systems_in_one_launch(ctx, rpt, n, maxiter):
         assert_bitwise(x, xo, f"solution {rep}")
         hist = [xo] + hist[:2]
     s.close()
+
+
+def test_concurrent_one_launch_solves(ctx):
+    """Four contexts solving at once, together more workgroups than may wait for each other on the
+    device: some take the phases, all return the same bits, three times in a row."""
+    import concurrent.futures as cf
+
+    n = 131072
+    rows = np.repeat(np.arange(n), 3)
+    cols = rows + np.tile([-1, 0, 1], n)
+    on = (cols >= 0) & (cols < n)
+    rows, cols = rows[on], cols[on].astype(np.int32)
+    ip = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    val = np.where(rows == cols, 2.01, -1.0)
+    b = cases.normal(61, n)
+    xo, ito, _, _ = O.pcg(ip, cols, val, b, rtol=1e-10, maxiter=400, check_every=10, rows_per_thread=4, nthreads=8)
+
+    def run(i):
+        c = core.Context(0)
+        s = core.Solver(None, ctx=c, indptr=ip, indices=cols)
+        s.set_values(val)
+        out = []
+        for _ in range(3):
+            s.reset_history()
+            x, it, _ = s.solve(b, rtol=1e-10, maxiter=400, check_every=10)
+            out.append((x, it))
+        s.close()
+        c.close()
+        return out
+
+    print("[gpu] four concurrent solves", flush=True)
+    with cf.ThreadPoolExecutor(4) as ex:
+        for out in ex.map(run, range(4)):
+            for x, it in out:
+                assert it == ito
+                assert_bitwise(x, xo, "concurrent solve")
