@@ -1439,6 +1439,11 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.kb = P.upload(hm.kb);
     d.sigma = P.upload(hm.sigma);
     d.vmode = hm.vmode;
+    d.flat = hm.vmode == 0 && hm.sigma[nv - 1] == 0.0 && std::all_of(hm.kb.begin(), hm.kb.end(), [](int32_t k) { return k == 0; });
+    if (hm.vmode != 0) {
+      d.zn = P.alloc<double>((int64_t)n * nv);
+      d.nkz = P.alloc<int32_t>(n);
+    }
     if (hm.vmode == 1) d.sig_node = P.upload(hm.sig_node);
     if (hm.vmode == 2) {
       d.ztot = P.upload(hm.ztot);
@@ -1463,6 +1468,11 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.etype = P.upload(std::vector<int8_t>(n, -1));
     d.elem = P.upload(erec);
     d.area = P.upload(m->geo.area);
+    {
+      std::vector<double2> ai(ne);
+      for (int32_t e = 0; e < ne; ++e) ai[e] = make_double2(m->geo.area[e], 1.0 / m->geo.area[e]);
+      d.area_inv = P.upload(ai);
+    }
     d.gradphi = P.upload(m->geo.gradphi);
     d.elem_wet = P.alloc<int8_t>(ne);
     d.elem_kb = P.alloc<int32_t>(ne);

@@ -25,6 +25,7 @@ struct DMesh {
   // sigma per level, 1 = ivcor 1 with a sigma per node and level, 2 = ivcor 2 (SZ)
   int32_t vmode;
   int32_t bt_stage;         // backtracking stages each workgroup's element patch in LDS (0: off)
+  int32_t flat;             // vmode 0, kb = 0 at every node and the last sigma exactly 0
   int32_t izlev;            // nz - 1: the level at -min(h, h_s) (vmode 2)
   double h_s, h_c;          // (vmode 2)
   const double* sig_node;   // [n][nvrt] (vmode 1)
@@ -41,6 +42,8 @@ struct DMesh {
   double* elbc;
   double* uvw;              // [n][nvrt][4]: u, v, w, 0
   double2* nrec;            // [n][2]: (x, y), (eta2, depth), packed for the backtracking gathers
+  double* zn;               // [n][nvrt] z columns for the backtracking search (vmode 1, 2)
+  int32_t* nkz;             // [n] kb, with a flag where the column decreases (vmode 1, 2)
   double* eta_lev;          // [n] eta2 of the last level update (the node z levels follow it)
   int8_t* node_wet;
   int8_t* etype;            // [n] elevation BC type of each open node (-1: the step parameter iettype)
@@ -51,6 +54,7 @@ struct DMesh {
   // elements
   const int4* elem;         // [ne][2]: (n0, n1, n2, s0), (s1, s2, -, -)
   const double* area;
+  const double2* area_inv;  // [ne]: area, 1 / area
   const double* gradphi;    // [ne][3][2]
   int8_t* elem_wet;
   int32_t* elem_kb;

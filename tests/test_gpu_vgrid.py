@@ -149,3 +149,49 @@ def test_run_like_case_from_files(ctx, tmp_path):
     _full_chain(ctx, mesh, om, p)
     st = mesh.get(L.F_BSTATUS)
     assert (st & L.BT_OPEN_EXIT).any() or (st & L.BT_SLIDE).any()
+
+
+@pytest.mark.parametrize("grid", ["sz", "lsc2"])
+@pytest.mark.parametrize("state", ["low-water", "depth-only", "list"])
+def test_backtrack_columns(ctx, grid, state):
+    """The vertical search on kept z columns: water so low that some SZ columns decrease with the
+    level (searched in full), depths changed without a level update (element bottom levels of the
+    old bed), and short lists of start points (no columns kept)."""
+    spec = cases.CaseSpec(f"columns-{grid}", 40, 28, 400.0, nvrt=13, depth=10.0, substeps=6)
+    data = cases.make_case(spec)
+    depth = _basin_depth(data.xy)
+    if grid == "sz":
+        vg = core.VGrid(2, nz=3, h_s=40.0, h_c=10.0, theta_b=0.3, theta_f=6.0, ztot=np.array([-160.0, -80.0, -40.0]),
+                        sigma_s=np.linspace(-1.0, 0.0, spec.nvrt - 2))
+        mesh, om, p = _setup_vgrid(ctx, spec, depth, vg)
+    else:
+        expo = 1.0 + 0.7 * np.sin(np.arange(spec.n))
+        sn = -1.0 + np.linspace(0.0, 1.0, spec.nvrt)[None, :] ** expo[:, None]
+        kb = np.clip((8 - np.maximum(depth, 0.0) / 12.0).astype(np.int32), 0, 8)
+        mesh, om, p = _setup_vgrid(ctx, spec, depth, core.VGrid(1, sigma_node=sn), kb=kb)
+    h = mesh.topology(L.T_DEPTH)
+    sides = levs = None
+    if state == "low-water":
+        eta = np.where(h > 28.0, -24.0 - 0.01 * (np.arange(mesh.n) % 11), 0.0)
+        for x in (mesh, om):
+            x.set(L.F_ETA2, eta)
+        mesh.update_levels(p)
+        om.levels(p)
+    elif state == "depth-only":
+        d2 = np.where((h > 12.0) & (h < 38.0), h * 0.9 + 1.0, h)  # no bottom level of the SZ grid moves
+        mesh.set(L.F_DEPTH, d2)
+        om.set(L.F_DEPTH, d2)
+    print(f"[gpu] backtracking columns, {grid}, {state}", flush=True)
+    if state == "list":
+        rng = np.random.default_rng(11)
+        sides = rng.integers(0, mesh.ns, 300).astype(np.int32)
+        levs = rng.integers(0, mesh.nvrt, 300).astype(np.int32)
+        mesh.backtrack_list(p, sides, levs)
+        om.backtrack(p, sides, levs)
+        for f in (L.F_FOOT, L.F_BTU, L.F_BSTATUS):
+            assert_bitwise(mesh.get(f)[sides, levs], om.get(f)[sides, levs], f"field {f}")
+        return
+    mesh.backtrack(p)
+    om.backtrack(p, nthreads=8)
+    for f in (L.F_FOOT, L.F_BTU, L.F_BSTATUS):
+        assert_bitwise(mesh.get(f), om.get(f), f"field {f}")
