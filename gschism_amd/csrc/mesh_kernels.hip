@@ -16,6 +16,8 @@ namespace gsh {
 #define GSH_BT_OPEN_EXIT 8
 #define GSH_BT_SLIDE 16
 
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
 constexpr double kSmall = 1.0e-7;  // meshdata.h:10
 
 // Node::compZCoord (meshdata.cu:1744-1807) at level k of a wet node with elevation eta, depth h
@@ -184,6 +186,16 @@ __device__ __forceinline__ double div_by(double a, double b, double y) {
   const double q0 = a * y;
   const double q1 = __builtin_fma(__builtin_fma(-b, q0, a), y, q0);
   return __builtin_fma(__builtin_fma(-b, q1, a), y, q1);
+}
+
+// a / 3.0, correctly rounded as the division is, in four operations instead of eleven: a RN(1/3) is
+// within an ulp, one Newton correction then rounds correctly (Markstein; its remainder is a multiple
+// of the smallest subnormal, so exact at any size), and the fixup gives the division's zeros,
+// infinities and NaN.
+__device__ __forceinline__ double third(double a) {
+  constexpr double y = 1.0 / 3.0;
+  const double q = a * y;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-3.0, q, a), y, q), 3.0, a);
 }
 
 // LDS-staged element patch (k_backtrack with ST = true): every element the walk and the
@@ -1075,57 +1087,55 @@ void launch_rhs(const DMesh& m, const StepArgs& a, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------- momentum (the step after the solve)
-// The inverse of stage_rows: `rows` LDS rows of `row_len` values (stride `stride`) to one
-// contiguous span of HBM, with flat coalesced stores.
-__device__ __forceinline__ void unstage_rows(double* __restrict__ dst, const double* __restrict__ src, int stride,
-                                             int row_len, int rows) {
-  const int total = rows * row_len;
-  const float inv = 1.0f / (float)row_len;
-  for (int i = threadIdx.x; i < total; i += blockDim.x) {
-    int j;
-    const int g = split_row(i, inv, row_len, j);
-    dst[i] = src[g * stride + j];
-  }
-}
-
 // Side::grad2 (meshdata.cu:1363-1398) of eta1 over the side's elements that are wet (isDry of
 // the last level update) and of eta2 over those wet by eta2 (Element::isDry2, meshdata.cu:774-778:
 // a node with eta2 + depth <= h0 makes its element dry), each the mean of the element gradients
-// (Element::grad2, meshdata.h:1105-1114).
-__device__ __forceinline__ void side_eta_grads(const DMesh& m, const int4 sr, double h0, double& g1x, double& g1y,
-                                               double& g2x, double& g2y) {
-  g1x = g1y = g2x = g2y = 0.0;
-  int c1 = 0, c2 = 0;
-  const int es[2] = {sr.z, sr.w};
+// (Element::grad2, meshdata.h:1105-1114). Lane c of the side's two (adjacent) lanes reads and forms
+// element c's gradients; the lanes then exchange the components the other one sums.
+struct SideElem {  // element c of a side: its gradient coefficients, its nodes and whether it is wet
+  bool there, wet;
+  double2 p[3];
+  double f1[3], f2[3], h[3];
+};
+
+__device__ __forceinline__ SideElem side_elem_load(const DMesh& m, int e) {
+  SideElem q;
+  q.there = e >= 0;
+  e = max(e, 0);
+  const int4 r0 = m.elem[2 * (int64_t)e];
+  const double2* gp = reinterpret_cast<const double2*>(m.gradphi) + 3 * (int64_t)e;
+  q.wet = m.elem_wet[e] != 0;
+  const int nd[3] = {r0.x, r0.y, r0.z};
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int e = es[j];
-    if (e < 0) continue;
-    const int4 r0 = m.elem[2 * e];
-    const double* gp = m.gradphi + 6 * (int64_t)e;
-    const double p0x = gp[0], p0y = gp[1], p1x = gp[2], p1y = gp[3], p2x = gp[4], p2y = gp[5];
-    if (m.elem_wet[e]) {
-      const double f0 = m.eta1[r0.x], f1 = m.eta1[r0.y], f2 = m.eta1[r0.z];
-      g1x += f0 * p0x + f1 * p1x + f2 * p2x;
-      g1y += f0 * p0y + f1 * p1y + f2 * p2y;
-      ++c1;
-    }
-    const double f0 = m.eta2[r0.x], f1 = m.eta2[r0.y], f2 = m.eta2[r0.z];
-    const bool dry2 = f0 + m.depth[r0.x] <= h0 || f1 + m.depth[r0.y] <= h0 || f2 + m.depth[r0.z] <= h0;
-    if (!dry2) {
-      g2x += f0 * p0x + f1 * p1x + f2 * p2x;
-      g2y += f0 * p0y + f1 * p1y + f2 * p2y;
-      ++c2;
-    }
+  for (int j = 0; j < 3; ++j) {
+    q.p[j] = gp[j];
+    q.f1[j] = m.eta1[nd[j]];
+    q.f2[j] = m.eta2[nd[j]];
+    q.h[j] = m.depth[nd[j]];
   }
-  if (c1 > 0) {
-    g1x = g1x * (1.0 / c1);
-    g1y = g1y * (1.0 / c1);
-  }
-  if (c2 > 0) {
-    g2x = g2x * (1.0 / c2);
-    g2y = g2y * (1.0 / c2);
-  }
+  return q;
+}
+
+// The mean over the elements of one component; x, y: this lane's element's gradient, in: it counts.
+__device__ __forceinline__ double side_grad_mean(double x, double y, bool in, int c) {
+  const double own = c ? y : x, other = __shfl_xor(c ? x : y, 1, 64);
+  const bool oin = __shfl_xor((int)in, 1, 64) != 0;
+  const bool in0 = c ? oin : in, in1 = c ? in : oin;
+  double g = 0.0;
+  if (in0) g += c ? other : own;
+  if (in1) g += c ? own : other;
+  const int n = (int)in0 + (int)in1;
+  return n > 0 ? g * (1.0 / n) : g;
+}
+
+__device__ __forceinline__ void side_eta_grads(const SideElem& q, double h0, int c, double& g1, double& g2) {
+  const double x1 = q.f1[0] * q.p[0].x + q.f1[1] * q.p[1].x + q.f1[2] * q.p[2].x;
+  const double y1 = q.f1[0] * q.p[0].y + q.f1[1] * q.p[1].y + q.f1[2] * q.p[2].y;
+  g1 = side_grad_mean(x1, y1, q.there && q.wet, c);
+  const bool dry2 = q.f2[0] + q.h[0] <= h0 || q.f2[1] + q.h[1] <= h0 || q.f2[2] + q.h[2] <= h0;
+  const double x2 = q.f2[0] * q.p[0].x + q.f2[1] * q.p[1].x + q.f2[2] * q.p[2].x;
+  const double y2 = q.f2[0] * q.p[0].y + q.f2[1] * q.p[1].y + q.f2[2] * q.p[2].y;
+  g2 = side_grad_mean(x2, y2, q.there && !dry2, c);
 }
 
 // solveMomentumEquations (meshdata.cu:5074-5352) for one side, barotropic, itur=0 (dfv = dfv0),
@@ -1134,105 +1144,122 @@ __device__ __forceinline__ void side_eta_grads(const DMesh& m, const int4 sr, do
 // zc and u are the side's rows in LDS; u holds btu on entry and u2 on exit. The 3D case is
 // tridag_sch<2> (meshdata.cu:3665-3711) with the coefficients formed on the fly: the forward
 // sweep keeps u_j in the btu slot k-1 and gam_j in the zc slot k-1 (both dead once row j is
-// formed), the back substitution runs over those slots, and the result moves up one slot.
+// formed), and the back substitution moves each result up one slot, clamped.
 // Component c (0: x, 1: y) of one side's momentum solve, by one of the side's two lanes (adjacent
 // lanes of one wave): both lanes compute the shared coefficients identically (the Thomas pivots,
 // written to the same zc slots with the same values, in lockstep) and each solves its own
 // component. The free-slip projection needs both components and runs in lane 0 after a wave
 // fence. Every value has the operands and order of the one-lane form.
-__device__ void momentum_side(const DMesh& m, const StepArgs& a, int s, int c, double* zc, double* u) {
-  const int nv = m.nvrt;
-  const int kb = m.side_kb[s];
-  const int4 sr = m.side[s];
-  const double rx = a.rmaxvel, ry = a.rmaxvel * 1.013;
-  const double rc = c ? ry : rx;
-  if (!m.side_wet[s]) {
+// Few waves fit (24 bytes of LDS per side and level), so a wave must not wait for LDS at each level:
+// both sweeps read kMomAhead levels before the arithmetic that needs them.
+constexpr int kMomAhead = 4;
+
+struct MomSide {  // what a side's solve reads besides its rows
+  int kb;
+  bool wet;
+  double g1, g2, grav3, Cd, hhat, chi;  // g1, g2: the lane's component of the two gradients
+};
+
+__device__ __forceinline__ void momentum_side(int nv, const StepArgs& a, const MomSide& q, int c, double* zc, double* u) {
+  const int kb = q.kb;
+  const double rc = c ? a.rmaxvel * 1.013 : a.rmaxvel;
+  if (!q.wet) {
     for (int k = 0; k < nv; ++k) u[2 * k + c] = 0.0;
+    return;
+  }
+  const double dt = a.dt, th = a.theta;
+  if (kb == nv - 2) {
+    const double htot = zc[nv - 1] - zc[kb];
+    const double hc = u[2 * (nv - 1) + c] + dt * (0.0 - q.grav3 * ((1.0 - th) * q.g1 + th * q.g2));
+    const double vc = fmin(fmax(hc * q.hhat / htot, -rc), rc);
+    for (int k = 0; k < nv; ++k) u[2 * k + c] = vc;
   } else {
-    double g1x, g1y, g2x, g2y;
-    side_eta_grads(m, sr, a.h0, g1x, g1y, g2x, g2y);
-    const double g1 = c ? g1y : g1x, g2 = c ? g2y : g2x;
-    const double grav3 = 0.5 * (m.grav2[sr.x] + m.grav2[sr.y]);
-    const double Cd = 0.5 * (m.cd[sr.x] + m.cd[sr.y]);
-    const double dt = a.dt, th = a.theta;
-    if (kb == nv - 2) {
-      const double htot = zc[nv - 1] - zc[kb];
-      const double hhat = m.hhat[s];
-      const double hc = u[2 * (nv - 1) + c] + dt * (0.0 - grav3 * ((1.0 - th) * g1 + th * g2));
-      const double vc = fmin(fmax(hc * hhat / htot, -rc), rc);
-      for (int k = 0; k < nv; ++k) u[2 * k + c] = vc;
-    } else {
-      const double G = grav3 * (th * g2 + (1.0 - th) * g1);
-      const double chi2 = m.chi[s], dfv0 = a.dfv0;
-      double zm = zc[kb], z0 = zc[kb + 1];         // zc[k-1], zc[k]
-      double bm = u[2 * kb + c], b0 = u[2 * kb + 2 + c];  // btu[k-1], btu[k] of this component
-      double bet = 1.0, cprev = 0.0, up = 0.0;
-      // dz/6, dz/3 and dt dfv0 / dz of layer (k, k+1); the next row reuses them for its layer
-      // (k-1, k), whose dz is the same difference of the same two levels
-      double d6p = 0.0, d3p = 0.0, tp = 0.0;
-      for (int k = kb + 1; k < nv; ++k) {
-        const bool top = k < nv - 1;
-        const double zp = top ? zc[k + 1] : 0.0;
-        const double bp = top ? u[2 * (k + 1) + c] : 0.0;
-        const double dz_0 = z0 - zm;
-        const double dz_1 = top ? zp - z0 : 0.0;
-        double aj = 0.0, bj = 0.0, cj = 0.0, d6 = 0.0, d3 = 0.0, tq = 0.0;
-        if (top) {
-          tq = dt * dfv0 / dz_1;
-          d3 = dz_1 / 3.0;
-          d6 = d3 * 0.5;  // = dz_1 / 6.0 exactly: halving commutes with rounding for normal values
-          cj += d6 - tq;
-          bj += d3 + tq;
-        }
-        if (k > kb + 1) {
-          aj += d6p - tp;
-          bj += d3p + tp;
-        } else {
-          bj += dt * chi2;
-        }
-        double dz = 0.0;
-        dz += dz_1;
-        if (k > kb + 1) dz += dz_0;
-        double q = -(0.5 * dz) * dt * G;
-        if (top) q += d6 * (2.0 * b0 + bp);
-        if (k > kb + 1) q += d6p * (2.0 * b0 + bm);
-        d6p = d6;
-        d3p = d3;
-        tp = tq;
-        double uk;
-        if (k == kb + 1) {
-          bet = bj;
-          uk = q / bet;
-        } else {
+    const double G = q.grav3 * (th * q.g2 + (1.0 - th) * q.g1);
+    const double td = dt * a.dfv0;
+    // dz/6, dz/3 and dt dfv0 / dz of layer (k, k+1); the next row reuses them for its layer
+    // (k-1, k), whose dz is the same difference of the same two levels. dz/6 = (dz/3) 0.5
+    // exactly: halving commutes with rounding for normal values.
+    double zm = zc[kb], z0 = zc[kb + 1], zp = zc[kb + 2];                               // zc[k-1], zc[k], zc[k+1]
+    double bm = u[2 * kb + c], b0 = u[2 * (kb + 1) + c], bp = u[2 * (kb + 2) + c];  // btu of this component
+    // row kb + 1 (never the top one)
+    double dzp = zp - z0;
+    double tp = td / dzp, d3p = third(dzp), d6p = d3p * 0.5;
+    double bet = (d3p + tp) + dt * q.chi;
+    double cprev = d6p - tp;
+    double up = (-(0.5 * dzp) * dt * G + d6p * (2.0 * b0 + bp)) / bet;
+    u[2 * kb + c] = up;
+    zm = z0, z0 = zp, bm = b0, b0 = bp;
+    // rows kb + 2 .. nv - 2
+    for (int k0 = kb + 2; k0 < nv - 1; k0 += kMomAhead) {
+      double zb[kMomAhead], bb[kMomAhead];
+#pragma unroll
+      for (int j = 0; j < kMomAhead; ++j) {
+        const int k = min(k0 + 1 + j, nv - 1);
+        zb[j] = zc[k];
+        bb[j] = u[2 * k + c];
+      }
+#pragma unroll
+      for (int j = 0; j < kMomAhead; ++j) {
+        const int k = k0 + j;
+        if (k < nv - 1) {
+          zp = zb[j];
+          bp = bb[j];
+          const double dz_1 = zp - z0;
+          const double tq = td / dz_1, d3 = third(dz_1), d6 = d3 * 0.5;
+          const double aj = d6p - tp;
+          const double bj = (d3 + tq) + (d3p + tp);
+          double r = -(0.5 * (dz_1 + dzp)) * dt * G;
+          r += d6 * (2.0 * b0 + bp);
+          r += d6p * (2.0 * b0 + bm);
           const double gam = cprev / bet;
           bet = bj - aj * gam;
-          uk = (q - aj * up) / bet;
+          up = (r - aj * up) / bet;
           zc[k - 1] = gam;
+          u[2 * (k - 1) + c] = up;
+          cprev = d6 - tq;
+          dzp = dz_1, tp = tq, d3p = d3, d6p = d6;
+          z0 = zp, bm = b0, b0 = bp;
         }
-        u[2 * (k - 1) + c] = uk;
-        up = uk;
-        cprev = cj;
-        zm = z0;
-        z0 = zp;
-        bm = b0;
-        b0 = bp;
       }
-      // back substitution: u_j (slot kb + j) -= gam_{j+1} (zc slot kb + j + 1) u_{j+1}
-      for (int k = nv - 3; k >= kb; --k) {
-        const double gam = zc[k + 1];
-        up = u[2 * k + c] - gam * up;
-        u[2 * k + c] = up;
+    }
+    // row nv - 1
+    {
+      const double aj = d6p - tp, bj = d3p + tp;
+      double r = -(0.5 * dzp) * dt * G;
+      r += d6p * (2.0 * b0 + bm);
+      const double gam = cprev / bet;
+      bet = bj - aj * gam;
+      up = (r - aj * up) / bet;
+      zc[nv - 2] = gam;
+    }
+    // back substitution: u_j (slot kb + j) -= gam_{j+1} (zc slot kb + j + 1) u_{j+1}, each value
+    // clamped into the slot above, whose own value has been read
+    u[2 * (nv - 1) + c] = fmin(fmax(up, -rc), rc);
+    for (int k0 = nv - 3; k0 >= kb; k0 -= kMomAhead) {
+      double gb[kMomAhead], ub[kMomAhead];
+#pragma unroll
+      for (int j = 0; j < kMomAhead; ++j) {
+        const int k = max(k0 - j, kb);
+        gb[j] = zc[k + 1];
+        ub[j] = u[2 * k + c];
       }
-      for (int k = nv - 1; k > kb; --k) u[2 * k + c] = fmin(fmax(u[2 * (k - 1) + c], -rc), rc);
+#pragma unroll
+      for (int j = 0; j < kMomAhead; ++j) {
+        const int k = k0 - j;
+        if (k >= kb) {
+          up = ub[j] - gb[j] * up;
+          u[2 * (k + 1) + c] = fmin(fmax(up, -rc), rc);
+        }
+      }
     }
-    // bottom condition, imm = 0
-    if (Cd == 0.0) {
-      u[2 * kb + c] = u[2 * (kb + 1) + c];
-    } else if (kb < nv - 2) {
-      u[2 * kb + c] = 0.0;
-    }
-    for (int k = 0; k < kb; ++k) u[2 * k + c] = 0.0;
   }
+  // bottom condition, imm = 0
+  if (q.Cd == 0.0) {
+    u[2 * kb + c] = u[2 * (kb + 1) + c];
+  } else if (kb < nv - 2) {
+    u[2 * kb + c] = 0.0;
+  }
+  for (int k = 0; k < kb; ++k) u[2 * k + c] = 0.0;
 }
 
 // The free-slip projection of a land side (side_type 1), both components, by the side's lane 0
@@ -1254,26 +1281,75 @@ __device__ void momentum_free_slip(const DMesh& m, int s, double* u) {
   }
 }
 
-// A workgroup of 64 takes g <= 32 consecutive sides: their zc and btu rows come into LDS with flat
-// coalesced loads, two lanes per side solve in LDS (one component each), the u2 rows leave with
-// flat stores.
-__global__ void __launch_bounds__(64) k_momentum(DMesh m, StepArgs a, int g) {
+// A wave takes g <= 32 consecutive sides: their zc and btu rows come into LDS with flat coalesced
+// loads, two lanes per side solve in LDS (one component each), the u2 rows leave with flat stores.
+// 24 KB of LDS allow six waves on a CU, so what a wave waits for is what the kernel takes: all its
+// loads (kMomItems of either array per lane, and the records of its sides) are in flight together
+// (of 25 us a wave, 16 went into loads waited for in turn; 645,122 sides x 31 levels: 387 -> 186 us,
+// 4.3 TB/s; now half the time is the serial sweep, four divisions a level).
+// Strides: zs odd and us = 2 zs spread the sides' reads of one level over the banks.
+constexpr int kMomItems = 16;
+constexpr int kMomLds = 24 * 1024;
+
+
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) k_momentum(DMesh m, StepArgs a, int g) {
   extern __shared__ double lds[];
-  const int nv = m.nvrt;
-  const int zs = nv | 1, us = (2 * nv) | 1;
-  double* Lz = lds;
-  double* Lu = lds + g * zs;
+  const int nv = m.nvrt, zs = nv | 1, us = 2 * zs;
+  double* Lu = lds;
+  double* Lz = lds + g * us;
   const int s0 = blockIdx.x * g;
   const int gc = min(g, m.ns - s0);
-  stage_rows(Lz, zs, m.zc + (int64_t)s0 * nv, nv, gc);
-  stage_rows(Lu, us, m.btu + 2 * (int64_t)s0 * nv, 2 * nv, gc);
-  __syncthreads();
-  const int t = threadIdx.x, sl = t >> 1, c = t & 1;  // two lanes per side
-  if (sl < gc) momentum_side(m, a, s0 + sl, c, Lz + sl * zs, Lu + sl * us);
+  const int total = gc * nv;  // <= 64 kMomItems
+  const int t = threadIdx.x, sl = t >> 1, c = t & 1;
+  const float inv = 1.0f / (float)nv;
+  const double* zc = m.zc + (int64_t)s0 * nv;
+  const f64x2* btu = reinterpret_cast<const f64x2*>(m.btu) + (int64_t)s0 * nv;
+  const int s = s0 + min(sl, gc - 1);
+  const int4 sr = m.side[s];
+  __builtin_amdgcn_sched_barrier(0);  // the compiler would move each load down to its use
+  double z[kMomItems];
+  f64x2 b[kMomItems];
+  // past the end the last item is read and written again
+#pragma unroll
+  for (int j = 0; j < kMomItems; ++j) {
+    const int i = min(t + 64 * j, total - 1);
+    z[j] = zc[i];
+    b[j] = btu[i];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  const SideElem el = side_elem_load(m, c ? sr.w : sr.z);
+  MomSide q;
+  q.kb = m.side_kb[s];
+  q.wet = m.side_wet[s] != 0;
+  q.hhat = m.hhat[s];
+  q.chi = m.chi[s];
+  const double gr0 = m.grav2[sr.x], gr1 = m.grav2[sr.y], cd0 = m.cd[sr.x], cd1 = m.cd[sr.y];
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < kMomItems; ++j) {
+    int k;
+    const int r = split_row(min(t + 64 * j, total - 1), inv, nv, k);
+    Lz[r * zs + k] = z[j];
+    *reinterpret_cast<f64x2*>(Lu + r * us + 2 * k) = b[j];
+  }
+  q.grav3 = 0.5 * (gr0 + gr1);
+  q.Cd = 0.5 * (cd0 + cd1);
+  side_eta_grads(el, a.h0, c, q.g1, q.g2);
+  wave_lds_sync();
+  if (sl < gc) momentum_side(nv, a, q, c, Lz + sl * zs, Lu + sl * us);
   wave_lds_sync();
   if (sl < gc && c == 0) momentum_free_slip(m, s0 + sl, Lu + sl * us);
-  __syncthreads();
-  unstage_rows(m.su2 + 2 * (int64_t)s0 * nv, Lu, us, 2 * nv, gc);
+  wave_lds_sync();
+  f64x2* out = reinterpret_cast<f64x2*>(m.su2) + (int64_t)s0 * nv;
+#pragma unroll
+  for (int j = 0; j < kMomItems; ++j) {
+    const int i = t + 64 * j;
+    if (i < total) {
+      int k;
+      const int r = split_row(i, inv, nv, k);
+      out[i] = *reinterpret_cast<const f64x2*>(Lu + r * us + 2 * k);
+    }
+  }
 }
 
 // shapiroFilter1 + shapiroFilter2 (meshdata.cu:5456-5518) in one pass that writes every side's
@@ -1353,10 +1429,9 @@ void launch_shapiro(const DMesh& m, double shapiro0, double* out, hipStream_t st
 
 void launch_momentum(const DMesh& m, const StepArgs& a, hipStream_t st) {
   if (m.ns <= 0) return;
-  // sides per workgroup: one per two lanes, as many as 24 KB of LDS holds (measured best against
-  // 16-64 KB and 32-256 threads at 3.1M sides x 31 levels)
-  const int row = 8 * ((m.nvrt | 1) + ((2 * m.nvrt) | 1));
-  const int g = max(1, min(32, (24 * 1024) / row));
+  // sides per wave: one per two lanes, as many as 24 KB of LDS and kMomItems loads a lane hold
+  const int row = 24 * (m.nvrt | 1);
+  const int g = max(1, min(32, min(kMomLds / row, 64 * kMomItems / m.nvrt)));
   hipLaunchKernelGGL(k_momentum, dim3((unsigned)((m.ns + g - 1) / g)), dim3(64), (size_t)g * row, st, m, a, g);
 }
 
