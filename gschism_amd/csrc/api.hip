@@ -1498,6 +1498,15 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.chi = P.alloc<double>(ns);
     d.ball_ptr = P.upload(t.ball_ptr);
     d.ball_elem = P.upload(t.ball_elem);
+    {
+      std::vector<int4> br(t.ball_elem.size());
+      for (size_t j = 0; j < br.size(); ++j) {
+        const int32_t e = t.ball_elem[j], l = t.ball_loc[j];
+        const int32_t* es = &t.elside[3 * (size_t)e];  // side c lies opposite corner c
+        br[j] = make_int4(e, es[l], es[(l + 1) % 3], es[(l + 2) % 3]);
+      }
+      d.ball_rec = P.upload(br);
+    }
     d.ball_loc = P.upload(t.ball_loc);
     d.ball_slot = P.upload(ball_slot);
     d.nbr_ptr = P.upload(t.nbr_ptr);

@@ -84,6 +84,7 @@ struct DMesh {
   const int32_t* ball_ptr;
   const int32_t* ball_elem;
   const int8_t* ball_loc;
+  const int4* ball_rec;      // [ball]: element, the sides opposite the node and the next corner, and (first entry) the one after
   const int16_t* ball_slot;  // [ball][2]: CSR slots of the two other element nodes
   const int32_t* nbr_ptr;
   const int32_t* nbr_node;

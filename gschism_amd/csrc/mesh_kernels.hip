@@ -782,73 +782,84 @@ void launch_backtrack(const DMesh& mesh, const StepArgs& a, const int32_t* ls, c
 // wave reads consecutive levels of the same side and element rows.
 __device__ __forceinline__ double clamp_vel(double x, double hi) { return fmin(fmax(x, -hi), hi); }
 
+// Each ball is counter-clockwise, so the spoke s2 of one entry is the next entry's s3 (ball_rec.w
+// holds the first entry's s3): a node with m elements reads 2 m + 1 side rows instead of 3 m.
 // The workgroup's threads cover the levels of a few consecutive nodes, whose balls are one
-// contiguous range of the ball arrays: its entries (element, area, wet flag and the three side
-// ids) are staged in LDS once, up to kNvCap of them (the rest read from global memory, the same
-// values), so each (node, level) thread only gathers its level's w and u2.
+// contiguous range of the ball arrays: its entries (record, and the area, negative where the
+// element is dry) are staged in LDS once, up to kNvCap of them (the rest read from global memory,
+// the same values), so each (node, level) thread only gathers its level's w and u2, kNvBatch entries'
+// loads at a time. Bound by the first-level cache: its misses stall it 60 % of the time (215,683 nodes
+// x 31 levels: 240 -> 205 us, 3.1 TB/s; 3 entries at a time 213, 2 230; workgroups of consecutive
+// nodes on one XCD 210).
 constexpr int kNvCap = 512;
+constexpr int kNvBatch = 4;  // ball entries whose loads are in flight together
 
 __global__ void __launch_bounds__(256) k_nodal_velocity(DMesh m, double rx, double ry) {
+  __shared__ int4 Lrec[kNvCap];
   __shared__ double Larea[kNvCap];
-  __shared__ int Le[kNvCap], Ls1[kNvCap], Ls2[kNvCap], Ls3[kNvCap];
-  __shared__ int8_t Lwet[kNvCap];
+  __shared__ f64x2 Lout[512];
   const uint64_t t0 = (uint64_t)blockIdx.x * blockDim.x;
   const uint32_t nv = (uint32_t)m.nvrt;
   const uint64_t total = (uint64_t)m.n * nv;
   auto node_of = [&](uint64_t tt) { return (tt < 0xffffffffull) ? (int)((uint32_t)tt / nv) : (int)(tt / nv); };
-  // sides (r0.w, r1.x, r1.y) are opposite corners 0, 1, 2; s1 is the side opposite the node
-  auto sides_of = [&](int e, int l, int& s1, int& s2, int& s3) {
-    const int4 r0 = m.elem[2 * e], r1 = m.elem[2 * e + 1];
-    s1 = (l == 0) ? r0.w : ((l == 1) ? r1.x : r1.y);
-    s2 = (l == 0) ? r1.x : ((l == 1) ? r1.y : r0.w);
-    s3 = (l == 0) ? r1.y : ((l == 1) ? r0.w : r1.x);
-  };
   const int ifirst = node_of(t0), ilast = node_of(min(t0 + blockDim.x, total) - 1);
   const int jb = m.ball_ptr[ifirst];
   const int nst = min(m.ball_ptr[ilast + 1] - jb, kNvCap);
+  auto area_of = [&](int e) {
+    const double a = m.area[e];
+    const int wet = m.elem_wet[e];
+    return wet ? a : -a;
+  };
   for (int q = threadIdx.x; q < nst; q += blockDim.x) {
-    const int e = m.ball_elem[jb + q];
-    Le[q] = e;
-    Larea[q] = m.area[e];
-    Lwet[q] = m.elem_wet[e];
-    sides_of(e, m.ball_loc[jb + q], Ls1[q], Ls2[q], Ls3[q]);
+    const int4 r = m.ball_rec[jb + q];
+    Lrec[q] = r;
+    Larea[q] = area_of(r.x);
   }
-  __syncthreads();
-  const uint64_t t = t0 + threadIdx.x;
-  if (t >= total) return;
+  const uint64_t t = min(t0 + threadIdx.x, total - 1);
   const int i = node_of(t);
   const int k = (int)(t - (uint64_t)i * nv);
   const int j0 = m.ball_ptr[i], j1 = m.ball_ptr[i + 1];
   const bool node_wet = m.node_wet[i] != 0;
   const bool above = k >= m.kb[i];
-  const double2* su = reinterpret_cast<const double2*>(m.su2);
+  __syncthreads();
+  const double2* su = reinterpret_cast<const double2*>(m.su2) + k;
+  const double* ew = m.ew + k;
   // one pass over the ball; each sum keeps its own ball-order sequence of additions
   double asum = 0.0, ws = 0.0, sx = 0.0, sy = 0.0;
   int count = 0;
-  for (int j = j0; j < j1; ++j) {
-    const int q = j - jb;
-    const bool staged = q < nst;
-    const int e = staged ? Le[q] : m.ball_elem[j];
-    const double a = staged ? Larea[q] : m.area[e];
-    asum += a;
-    if (above) ws += m.ew[(int64_t)e * nv + k] * a;
-    if (!(staged ? Lwet[q] : m.elem_wet[e]) || !node_wet) continue;
-    ++count;
-    if (!above) continue;
-    int s1, s2, s3;
-    if (staged) {
-      s1 = Ls1[q];
-      s2 = Ls2[q];
-      s3 = Ls3[q];
-    } else {
-      sides_of(e, m.ball_loc[j], s1, s2, s3);
+  auto pass = [&](auto rec, auto area) {
+    if (j0 >= j1) return;
+    double2 u3 = su[(int64_t)rec(j0).w * nv];
+    for (int j = j0; j < j1; j += kNvBatch) {
+      double2 u1[kNvBatch] = {}, u2[kNvBatch] = {};
+      double w[kNvBatch] = {};
+#pragma unroll
+      for (int q = 0; q < kNvBatch; ++q)
+        if (j + q < j1) {
+          const int4 r = rec(j + q);
+          u1[q] = su[(int64_t)r.y * nv];
+          u2[q] = su[(int64_t)r.z * nv];
+          w[q] = ew[(int64_t)r.x * nv];
+        }
+#pragma unroll
+      for (int q = 0; q < kNvBatch; ++q)
+        if (j + q < j1) {
+          const double as = area(j + q), a = fabs(as);
+          asum += a;
+          ws += w[q] * a;
+          if (as > 0.0 && node_wet) {
+            ++count;
+            sx += clamp_vel(u2[q].x + u3.x - u1[q].x, rx);
+            sy += clamp_vel(u2[q].y + u3.y - u1[q].y, ry);
+          }
+          u3 = u2[q];
+        }
     }
-    const double2 u1 = su[(int64_t)s1 * nv + k];
-    const double2 u2 = su[(int64_t)s2 * nv + k];
-    const double2 u3 = su[(int64_t)s3 * nv + k];
-    sx += clamp_vel(u2.x + u3.x - u1.x, rx);
-    sy += clamp_vel(u2.y + u3.y - u1.y, ry);
-  }
+  };
+  if (j1 - jb <= nst)
+    pass([&](int j) { return Lrec[j - jb]; }, [&](int j) { return Larea[j - jb]; });
+  else
+    pass([&](int j) { return m.ball_rec[j]; }, [&](int j) { return area_of(m.ball_rec[j].x); });
   double ux = 0.0, uy = 0.0, w = 0.0;
   if (above) {
     w = (1.0 / asum) * ws;
@@ -857,7 +868,17 @@ __global__ void __launch_bounds__(256) k_nodal_velocity(DMesh m, double rx, doub
       uy = sy * (1.0 / count);
     }
   }
-  reinterpret_cast<double4*>(m.uvw)[t] = make_double4(ux, uy, w, 0.0);
+  // a lane's record is 32 bytes: through LDS each store of a wave covers one contiguous KB (two
+  // stores of every other 16 bytes write each line twice)
+  f64x2* mine = Lout + 128 * (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  mine[2 * lane] = f64x2{ux, uy};
+  mine[2 * lane + 1] = f64x2{w, 0.0};
+  wave_lds_sync();
+  const uint64_t c0 = 2 * t0 + 128 * (threadIdx.x >> 6) + lane;
+  f64x2* out = reinterpret_cast<f64x2*>(m.uvw);
+  if (c0 < 2 * total) out[c0] = mine[lane];
+  if (c0 + 64 < 2 * total) out[c0 + 64] = mine[lane + 64];
 }
 
 void launch_nodal_velocity(const DMesh& m, double rmaxvel, hipStream_t st) {
