@@ -1485,6 +1485,12 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.side_cx = P.upload(m->geo.side_cx);
     d.side_cy = P.upload(m->geo.side_cy);
     d.side_len = P.upload(m->geo.side_len);
+    {
+      std::vector<double4> sg(ns);
+      for (int32_t s = 0; s < ns; ++s)
+        sg[s] = make_double4(m->geo.side_nx[s], m->geo.side_ny[s], m->geo.side_len[s], (double)srec[s].z);
+      d.side_geo = P.upload(sg);
+    }
     d.side_kb = P.alloc<int32_t>(ns);
     d.side_wet = P.alloc<int8_t>(ns);
     d.zc = P.alloc<double>((int64_t)ns * nv);

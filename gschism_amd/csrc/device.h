@@ -69,6 +69,7 @@ struct DMesh {
   const double* side_cx;
   const double* side_cy;
   const double* side_len;
+  const double4* side_geo;  // [ns]: unit normal x, y, length, element 0 (as a value)
   int32_t* side_kb;
   int8_t* side_wet;
   double* zc;               // [ns][nvrt]

@@ -1486,15 +1486,22 @@ void launch_momentum(const DMesh& m, const StepArgs& a, hipStream_t st) {
 // meshdata.cu:559-631); phase 2, one thread per element: the running top flux
 // top_l = -side_l - bottom_l, bottom_l+1 = -top_l, in the reference's order; phase 3, one thread
 // per (element, level): w = (top - horizontal) / (n_z A), stored with coalesced writes.
+// 55 % of the time is VALU issue (a square root, four divisions and the geometry of each face), the
+// rest the three loads one after the other before phase 1's values are there: the side normals come
+// from the mesh (DMesh::side_geo), the level function has no branches (VM), and the bottom velocity
+// is phase 1's own (645,122 sides x 31 levels: 308 -> 219 us, 2.2 TB/s).
 
 // Per-element values that every level of phase 1 reads: node positions and level data, side
 // normals (populateSides, meshdata.cu:2283-2287), orientation signs, lengths and bottom levels.
 struct VvElem {
   double px[3], py[3], eta[3], h[3];
   double snx[3], sny[3], sign[3], slen[3];
+  double area;
   int nkb[3], s[3], skb[3], dry[3], nd[3];
+  int kb;  // the element's bottom level, nvrt when it is dry
 };
 
+template <int VM>
 __global__ void __launch_bounds__(256) k_vertical_velocity(DMesh m, double h0, int E) {
   extern __shared__ double lds[];
   const int nv = m.nvrt, nvp = nv - 1;
@@ -1510,122 +1517,136 @@ __global__ void __launch_bounds__(256) k_vertical_velocity(DMesh m, double h0, i
     const int el = t / 3, j = t - 3 * el;
     const int e = e0 + el;
     VvElem& q = Lel[el];
-    const int4 r0 = m.elem[2 * e], r1 = m.elem[2 * e + 1];
-    const int nd[3] = {r0.x, r0.y, r0.z};
-    const int sd[3] = {r0.w, r1.x, r1.y};
-    {
-      const int i = nd[j];
-      q.px[j] = m.x[i];
-      q.py[j] = m.y[i];
-      q.eta[j] = m.eta_lev[i];
-      q.h[j] = m.depth[i];
-      q.nkb[j] = m.kb[i];
-      q.nd[j] = i;
-      q.dry[j] = q.eta[j] + q.h[j] <= h0;  // isDry2 at the level update
-      const int s = sd[j];
-      const int4 sr = m.side[s];
-      const double vx = -(m.y[sr.x] - m.y[sr.y]), vy = m.x[sr.x] - m.x[sr.y];
-      const double ql = sqrt(vx * vx + vy * vy);
-      q.snx[j] = vx / ql;
-      q.sny[j] = vy / ql;
-      q.sign[j] = (sr.z == e) ? 1.0 : -1.0;
-      q.slen[j] = m.side_len[s];
-      q.s[j] = s;
-      q.skb[j] = m.side_kb[s];
+    const int* er = reinterpret_cast<const int*>(m.elem + 2 * (int64_t)e);  // nodes 0-2, sides 0-2
+    const int i = er[j], s = er[3 + j];
+    const double4 sg = m.side_geo[s];
+    const double eta = m.eta_lev[i], h = m.depth[i];
+    q.px[j] = m.x[i];
+    q.py[j] = m.y[i];
+    q.eta[j] = eta;
+    q.h[j] = h;
+    q.nkb[j] = m.kb[i];
+    q.nd[j] = i;
+    q.dry[j] = eta + h <= h0;  // isDry2 at the level update
+    q.snx[j] = sg.x;
+    q.sny[j] = sg.y;
+    q.slen[j] = sg.z;
+    q.sign[j] = sg.w == (double)e ? 1.0 : -1.0;
+    q.s[j] = s;
+    q.skb[j] = m.side_kb[s];
+    const int wet = m.elem_wet[e], kb = m.elem_kb[e];
+    const double area = m.area[e];
+    if (j == 0) {
+      q.area = area;
+      q.kb = wet ? kb : nv;
     }
   }
   __syncthreads();
+  const float inv = 1.0f / (float)nvp;
   for (int idx = threadIdx.x; idx < ec * nvp; idx += blockDim.x) {
-    const int el = idx / nvp, l = idx - el * nvp;
-    const int e = e0 + el;
-    if (!m.elem_wet[e] || l < m.elem_kb[e]) continue;
+    int l;
+    const int el = split_row(idx, inv, nvp, l);
     const VvElem& q = Lel[el];
+    if (l < q.kb) continue;
+    double2 ut[3], ul[3];
+    double zt[3], zl[3], sg[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      // the face's sigma: its level's, its nodes' from their beds up, or (SZ) its sigma, C and Z level
+      if (VM == 0) sg[j] = m.sigma[l + 1];
+      if (VM == 1) sg[j] = m.sig_node[(int64_t)q.nd[j] * nv + max(l + 1, q.nkb[j])];
+      if (VM == 2) sg[j] = j == 0 ? m.ssig[max(l + 1 - m.izlev, 0)] : (j == 1 ? m.cs[max(l + 1 - m.izlev, 0)] : m.ztot[min(l + 1, m.izlev)]);
+      const int64_t row = (int64_t)q.s[j] * nv;
+      const int kt = max(l + 1, q.skb[j]), kl = max(l, q.skb[j]);
+      const double2* u2 = reinterpret_cast<const double2*>(m.su2) + row;
+      ut[j] = u2[kt];
+      ul[j] = u2[kl];
+      zt[j] = m.zc[row + kt];
+      zl[j] = m.zc[row + kl];
+    }
+    if (l == q.kb) {
+      // w at the bottom: -grad(h) . u there (kl is then the side's own bottom level)
+      const double* gp = m.gradphi + 6 * (int64_t)(e0 + el);
+      const double ghx = q.h[0] * gp[0] + q.h[1] * gp[2] + q.h[2] * gp[4];
+      const double ghy = q.h[0] * gp[1] + q.h[1] * gp[3] + q.h[2] * gp[5];
+      const double ubx = third(ul[0].x + ul[1].x + ul[2].x + 0.0), uby = third(ul[0].y + ul[1].y + ul[2].y + 0.0);
+      const double bottomW = -(ghx * ubx + ghy * uby);
+      Lbw[el] = 0.0 + bottomW;
+    }
     // the face at level l+1 (node levels clamped to each node's bed), zcoord of the level update
     double pz[3];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
+      const double eta = q.eta[j], h = q.h[j];
       const int k = max(l + 1, q.nkb[j]);
-      pz[j] = q.dry[j] ? 0.0 : z_wet(m, q.nd[j], q.eta[j], q.h[j], q.nkb[j], k);
+      double z;
+      if (VM == 2) {  // z_wet's SZ branch as selects
+        const double hm = fmin(h, m.h_s);
+        const double zs = hm <= m.h_c ? sg[0] * (hm + eta) + eta : eta * (1.0 + sg[0]) + m.h_c * sg[0] + (hm - m.h_c) * sg[1];
+        z = k < m.izlev ? sg[2] : zs;
+        z = k == q.nkb[j] ? -h : z;
+        z = k == m.izlev ? -hm : z;
+        z = k == nv - 1 ? eta : z;
+      } else {
+        z = (eta + h) * sg[j] + eta;
+        z = k <= q.nkb[j] ? -h : (k == nv - 1 ? eta : z);
+      }
+      pz[j] = q.dry[j] ? 0.0 : z;
     }
     const double n20x = q.px[2] - q.px[0], n20y = q.py[2] - q.py[0], n20z = pz[2] - pz[0];
     const double n10x = q.px[1] - q.px[0], n10y = q.py[1] - q.py[0], n10z = pz[1] - pz[0];
     const double nx = (n10y) * (n20z) - (n20y) * (n10z);
     const double ny = (n20x) * (n10z) - (n10x) * (n20z);
-    const double nz = 2.0 * m.area[e];
+    const double nz = 2.0 * q.area;
     const double len = sqrt(nx * nx + ny * ny + nz * nz);
     const double ta = 0.5 * len;
     const double inv_len = 1.0 / len;
     const double tnx = nx * inv_len, tny = ny * inv_len, tnz = nz * inv_len;
-    double sf = 0.0, vx[3], vy[3];
+    double sf = 0.0;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-      const int s = q.s[j], kbs = q.skb[j];
-      const int kt = max(l + 1, kbs), kl = max(l, kbs);
-      const double2* u2 = reinterpret_cast<const double2*>(m.su2) + (int64_t)s * nv;
-      const double* zc = m.zc + (int64_t)s * nv;
-      const double2 ut = u2[kt], ul = u2[kl];
-      const double ucx = 0.5 * (ut.x + ul.x), ucy = 0.5 * (ut.y + ul.y);
-      const double sideArea = q.slen[j] * (zc[kt] - zc[kl]);
+      const double ucx = 0.5 * (ut[j].x + ul[j].x), ucy = 0.5 * (ut[j].y + ul[j].y);
+      const double sideArea = q.slen[j] * (zt[j] - zl[j]);
       sf += q.sign[j] * (ucx * q.snx[j] + ucy * q.sny[j]) * sideArea;
-      vx[j] = ut.x;
-      vy[j] = ut.y;
     }
-    const double utx = (vx[0] + vx[1] + vx[2] + 0.0) / 3, uty = (vy[0] + vy[1] + vy[2] + 0.0) / 3;
+    const double utx = third(ut[0].x + ut[1].x + ut[2].x + 0.0), uty = third(ut[0].y + ut[1].y + ut[2].y + 0.0);
     Lsf[idx] = sf;
     Lth[idx] = (utx * tnx + uty * tny) * ta;
     Lden[idx] = tnz * ta;
   }
   __syncthreads();
   if (threadIdx.x < ec) {
-    const int el = threadIdx.x, e = e0 + el;
-    if (m.elem_wet[e]) {
-      const VvElem& q = Lel[el];
-      const int kb = m.elem_kb[e];
-      const double* gp = m.gradphi + 6 * (int64_t)e;
-      const double ghx = q.h[0] * gp[0] + q.h[1] * gp[2] + q.h[2] * gp[4];
-      const double ghy = q.h[0] * gp[1] + q.h[1] * gp[3] + q.h[2] * gp[5];
-      double bx[3], by[3];
+    const int el = threadIdx.x;
+    // the running sums in level order; the side fluxes of 8 levels are read ahead so that
+    // the dependent additions do not wait for LDS one at a time
+    double bottom = 0.0;
+    double* row = Lsf + el * nvp;
+    for (int l0 = Lel[el].kb; l0 < nvp; l0 += 8) {
+      double f[8];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double2 u = reinterpret_cast<const double2*>(m.su2)[(int64_t)q.s[j] * nv + q.skb[j]];
-        bx[j] = u.x;
-        by[j] = u.y;
-      }
-      const double ubx = (bx[0] + bx[1] + bx[2] + 0.0) / 3, uby = (by[0] + by[1] + by[2] + 0.0) / 3;
-      const double bottomW = -(ghx * ubx + ghy * uby);
-      Lbw[el] = 0.0 + bottomW;
-      // the running sums in level order; the side fluxes of 8 levels are read ahead so that
-      // the dependent additions do not wait for LDS one at a time
-      double bottom = 0.0;
-      double* row = Lsf + el * nvp;
-      for (int l0 = kb; l0 < nvp; l0 += 8) {
-        double f[8];
+      for (int u = 0; u < 8; ++u) f[u] = (l0 + u < nvp) ? row[l0 + u] : 0.0;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) f[u] = (l0 + u < nvp) ? row[l0 + u] : 0.0;
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (l0 + u < nvp) {
-            const double top = -f[u] - bottom;
-            row[l0 + u] = top;
-            bottom = -top;
-          }
-      }
+      for (int u = 0; u < 8; ++u)
+        if (l0 + u < nvp) {
+          const double top = -f[u] - bottom;
+          row[l0 + u] = top;
+          bottom = -top;
+        }
     }
   }
   __syncthreads();
   double* w = m.ew + (int64_t)e0 * nv;
+  const float invn = 1.0f / (float)nv;
   for (int idx = threadIdx.x; idx < ec * nv; idx += blockDim.x) {
-    const int el = idx / nv, k = idx - el * nv;
-    const int e = e0 + el;
+    int k;
+    const int el = split_row(idx, invn, nv, k);
+    const int kb = Lel[el].kb;
     double v = 0.0;
-    if (m.elem_wet[e]) {
-      const int kb = m.elem_kb[e];
-      if (k == kb) {
-        v = Lbw[el];
-      } else if (k > kb) {
-        const int j = el * nvp + k - 1;
-        v = (Lsf[j] - Lth[j]) / Lden[j];
-      }
+    if (k == kb) {
+      v = Lbw[el];
+    } else if (k > kb) {
+      const int j = el * nvp + k - 1;
+      v = (Lsf[j] - Lth[j]) / Lden[j];
     }
     w[idx] = v;
   }
@@ -1634,11 +1655,21 @@ __global__ void __launch_bounds__(256) k_vertical_velocity(DMesh m, double h0, i
 void launch_vertical_velocity(const DMesh& m, double h0, hipStream_t st) {
   if (m.ne <= 0 || m.nvrt < 2) return;
   const int nvp = m.nvrt - 1;
-  // elements per workgroup: about one thread per (element, level), within 32 KB of LDS
+  // elements per workgroup: four (element, level) items a thread, within 32 KB of LDS (215,683 nodes x
+  // 31 levels: one item 359 us, two 238, four 219, eight 224); one item where four would leave fewer
+  // than two workgroups a CU (24 x 16 nodes x 8 levels 9.1 us with four, 5.8 with one; 200 x 80 x 31,
+  // just above the line, 20.0 and 24.4)
   const size_t per_elem = 8 * (3 * (size_t)nvp + 1) + sizeof(VvElem);
-  const int E = max(1, min(256 / nvp, (int)((32 * 1024) / per_elem)));
+  auto elems = [&](int items) { return max(1, min(items * 256 / nvp, (int)((32 * 1024) / per_elem))); };
+  const int E = m.ne >= 512 * elems(4) ? elems(4) : elems(1);
   const size_t lds = per_elem * E;
-  hipLaunchKernelGGL(k_vertical_velocity, dim3((unsigned)((m.ne + E - 1) / E)), dim3(256), lds, st, m, h0, E);
+  auto go = [&](auto ker) { hipLaunchKernelGGL(ker, dim3((unsigned)((m.ne + E - 1) / E)), dim3(256), lds, st, m, h0, E); };
+  if (m.vmode == 0)
+    go(k_vertical_velocity<0>);
+  else if (m.vmode == 1)
+    go(k_vertical_velocity<1>);
+  else
+    go(k_vertical_velocity<2>);
 }
 
 // ---------------------------------------------------------------- a11+a12: assembly + BC

@@ -749,3 +749,35 @@ def test_concurrent_one_launch_solves(ctx):
             for x, it in out:
                 assert it == ito
                 assert_bitwise(x, xo, "concurrent solve")
+
+
+@pytest.mark.parametrize("nvrt", [2, 3, 4, 5, 6, 7, 10, 33, 64, 65])
+def test_velocity_kernels_level_edges(ctx, nvrt):
+    """Momentum, Shapiro filter, vertical and nodal velocity around their unrolled levels, items per
+    thread and staged ball entries (at two levels a workgroup's nodes have more than are staged), with
+    node-varying bottom levels and an island's dry sides."""
+    spec = cases.CaseSpec(f"levels-{nvrt}", 41, 29, 400.0, nvrt=nvrt, depth=10.0, substeps=4)
+    mesh, om, p = _setup(ctx, spec, kb_fn=lambda d: (np.arange(d.size) % max(1, min(5, nvrt - 1))).astype(np.int32),
+                         depth_fn=_island_depth)
+    rng = np.random.default_rng(nvrt)
+    btu = rng.normal(0.0, 0.4, (mesh.ns, nvrt, 2))
+    eta_old = mesh.get(L.F_ETA2)
+    p.ishapiro, p.shapiro0 = 1, 0.5
+    print(f"[gpu] velocity kernels nvrt={nvrt} ns={mesh.ns}", flush=True)
+    for m in (mesh, om):
+        m.set(L.F_BTU, btu)
+    mesh.rhs_producers(p)
+    om.rhs(p)
+    for m in (mesh, om):
+        m.set(L.F_ETA1, eta_old)
+        m.set(L.F_ETA2, eta_old + 0.02)
+    mesh.momentum(p)
+    om.momentum(p)
+    assert_bitwise(mesh.get(L.F_SIDE_U2), om.get(L.F_SIDE_U2), f"filtered side velocity, {nvrt} levels")
+    mesh.vertical_velocity(p)
+    om.vertical_velocity()
+    assert_bitwise(mesh.get(L.F_ELEM_W), om.get(L.F_ELEM_W), f"element w, {nvrt} levels")
+    mesh.nodal_velocity(p)
+    om.nodal_velocity(p)
+    assert_bitwise(mesh.get(L.F_NODE_UVW), om.get(L.F_NODE_UVW), f"nodal velocity, {nvrt} levels")
+    mesh.close()
