@@ -303,6 +303,10 @@ struct ZSigma {
   NodeZ q0, q1, q2;
   const double* sig;
   int nv;
+  __device__ __forceinline__ double3 nodes(int M) const {
+    const double sM = sig[F ? M : max(M, 0)];
+    return {zlev<F>(q0, sM, M, nv), zlev<F>(q1, sM, M, nv), zlev<F>(q2, sM, M, nv)};
+  }
   __device__ __forceinline__ double operator()(double s0, double s1, double s2, int M) const {
     const double sM = sig[F ? M : max(M, 0)];
     return s0 * zlev<F>(q0, sM, M, nv) + s1 * zlev<F>(q1, sM, M, nv) + s2 * zlev<F>(q2, sM, M, nv) + 0.0;
@@ -319,6 +323,7 @@ struct ZColumns {
     if (q.x + q.y <= h0) return 0.0;
     return (M <= kb) ? -q.y : z_wet(m, node, q.x, q.y, kb, M);
   }
+  __device__ __forceinline__ double3 nodes(int M) const { return {level(n0, M), level(n1, M), level(n2, M)}; }
   __device__ __forceinline__ double operator()(double s0, double s1, double s2, int M) const {
     return s0 * level(n0, M) + s1 * level(n1, M) + s2 * level(n2, M) + 0.0;
   }
@@ -332,7 +337,7 @@ struct ZColumns {
 // and zR; otherwise one step down or up. A point at or below the bed, next to it (h <= bed, where
 // z_h is z_L0), or at or above the surface takes the end that the full search finds first. A wave
 // holds the levels of about two sides, the bed's and the surface's among them, so without these two
-// rules every wave ran the full search's probes in every substep. (1,048,576 nodes x 32 levels, one
+// rules every wave ran the full search's probes in every substep. (1,048,576 nodes x 31 levels, one
 // sigma per level: 9.72 -> 8.58 ms a pass with the F variant and div_by; SZ grid 301x173 602 -> 282 us
 // and per-node sigma 417x263 1419 -> 823 us, both with k_pack_levels, whose full search had evaluated
 // the level functions at every probe.)
@@ -397,26 +402,39 @@ __device__ __forceinline__ void z_bracket(const Z& z, double s0, double s1, doub
   }
 }
 
+// What the last interpolation of a start point read: the element, its area and reciprocal, and the
+// z and velocities of its nodes at the two levels of the vertical bracket. Most substeps stay in
+// their prism, and then read nothing: every operand is here, in the operations of the full search.
+// It takes 58 registers: three waves a SIMD instead of four (four spill: 16.8 ms against 7.5, two 9.8),
+// and 64 % of the time is VALU issue. 1,048,576 nodes x 31 levels 8.58 -> 7.48 ms (8.36 with only the
+// last interpolation spared), per-node sigma 417x263 841 -> 685 us.
+struct BtCell {
+  int e = -1;  // -1: none
+  int L = 0, R = 0;
+  bool kept = false;  // the bracket's values hold, and the column's levels do not decrease
+  double2 area;
+  double3 zL, zR;                      // per node
+  double3 u0, u1, u2, v0, v1, v2;      // (u, v, w) of nodes 0-2 at L, and at R
+};
+
 // Element::interpolateVelocities for triangles, ics=1 (meshdata.cu:1209-1291) with
 // computeShapeCoords(fiAnywhere) (meshdata.cu:990-1043); g is element e's geometry.
 // hint: the lower level of the previous vertical bracket (updated here).
 // rc: element e's staged record (ST), else NULL.
 template <int VM, bool ST, bool F>
 __device__ void interp_velocity(const DMesh& m, const double* sig, double h0, int e, const ElemGeom& g,
-                                const StElem* rc, double px, double py, double pz, double& uo, double& vo,
+                                const StElem* rc, BtCell& c, double px, double py, double pz, double& uo, double& vo,
                                 double& wo, int& hint) {
   const int n0 = g.n0, n1 = g.n1, n2 = g.n2;
   const double x0 = g.x0, y0 = g.y0, x1 = g.x1, y1 = g.y1, x2 = g.x2, y2 = g.y2;
-  const double a0 = signed_area(px, py, x1, y1, x2, y2), a1 = signed_area(x0, y0, px, py, x2, y2);
-  double s0, s1;
-  if (ST && rc) {
-    s0 = a0 / rc->area;
-    s1 = a1 / rc->area;
-  } else {
-    const double2 ar = m.area_inv[ux(e)];
-    s0 = div_by(a0, ar.x, ar.y);
-    s1 = div_by(a1, ar.x, ar.y);
+  if (c.e != e) {
+    c.e = e;
+    c.kept = false;
+    c.area = m.area_inv[ux(e)];
   }
+  const double a0 = signed_area(px, py, x1, y1, x2, y2), a1 = signed_area(x0, y0, px, py, x2, y2);
+  double s0 = div_by(a0, c.area.x, c.area.y);
+  double s1 = div_by(a1, c.area.x, c.area.y);
   double s2 = 1.0 - s0 - s1;
   const double tmin = fmin(s0, fmin(s1, s2));
   if (tmin < 0.0) {
@@ -428,34 +446,66 @@ __device__ void interp_velocity(const DMesh& m, const double* sig, double h0, in
   }
   const int nv = m.nvrt;
   const bool st = ST && rc;
-  const int L0 = F ? -1 : (st ? rc->ekb : m.elem_kb[ux(e)]) - 1, R0 = nv - 1;
-  int L, R, kb0, kb1, kb2;
-  double w1, w2;
-  if constexpr (VM == 0) {
-    const ZSigma<F> z{st ? st_node_z(*rc, 0) : node_z<F>(m, n0), st ? st_node_z(*rc, 1) : node_z<F>(m, n1),
-                      st ? st_node_z(*rc, 2) : node_z<F>(m, n2), sig, nv};
-    kb0 = z.q0.kb, kb1 = z.q1.kb, kb2 = z.q2.kb;
-    // F: level 0 is the bed, as -1 is
-    z_bracket(z, s0, s1, s2, pz, F ? 0 : L0, min(kb0, min(kb1, kb2)), R0, true, hint, L, R, w1, w2);
-  } else {
-    // kb with a flag where the node's column is not non-decreasing (k_pack_levels), or is not kept
-    const int f0 = m.zn ? m.nkz[ux(n0)] : m.kb[ux(n0)], f1 = m.zn ? m.nkz[ux(n1)] : m.kb[ux(n1)],
-              f2 = m.zn ? m.nkz[ux(n2)] : m.kb[ux(n2)];
-    kb0 = f0 & kKbMask, kb1 = f1 & kKbMask, kb2 = f2 & kKbMask;
-    z_bracket(ZColumns{m, h0, n0, n1, n2}, s0, s1, s2, pz, L0, min(kb0, min(kb1, kb2)), R0,
-              m.zn && !((f0 | f1 | f2) & ~kKbMask), hint, L, R, w1, w2);
+  // F: level 0 is the bed, as -1 is
+  const int R0 = nv - 1;
+  double w1 = 1.0, w2 = 0.0;
+  bool hit = false;
+  if (c.kept) {
+    // the kept bracket: strictly inside two neighbouring levels, or the whole column (L0, R0) with the
+    // point at or beyond an end: then z_bracket ends in it, with the same weights
+    const double zL = s0 * c.zL.x + s1 * c.zL.y + s2 * c.zL.z + 0.0, zR = s0 * c.zR.x + s1 * c.zR.y + s2 * c.zR.z + 0.0;
+    const bool whole = c.R - c.L > 1;
+    if (!whole) {
+      hit = zL < pz && pz < zR;
+      if (hit) {
+        w2 = (pz - zL) / (zR - zL);
+        w1 = 1.0 - w2;
+      }
+    } else if (pz <= zL) {
+      hit = true;
+    } else if (pz >= zR) {
+      hit = true;
+      w1 = 0.0;
+      w2 = 1.0;
+    }
   }
-  // the three nodes' level rows (64-bit row offsets), then two levels of each
-  const double4* U = reinterpret_cast<const double4*>(m.uvw);
-  const double4* u0 = U + (uint64_t)ux(n0) * ux(nv);
-  const double4* u1 = U + (uint64_t)ux(n1) * ux(nv);
-  const double4* u2 = U + (uint64_t)ux(n2) * ux(nv);
-  auto at = [](int level, int kb) { return ux(F ? level : max(level, kb)); };
-  const double4 l0 = u0[at(L, kb0)], l1 = u1[at(L, kb1)], l2 = u2[at(L, kb2)];
-  const double4 r0 = u0[at(R, kb0)], r1 = u1[at(R, kb1)], r2 = u2[at(R, kb2)];
-  const double uL = s0 * l0.x + s1 * l1.x + s2 * l2.x + 0.0, vL = s0 * l0.y + s1 * l1.y + s2 * l2.y + 0.0;
-  const double uR = s0 * r0.x + s1 * r1.x + s2 * r2.x + 0.0, vR = s0 * r0.y + s1 * r1.y + s2 * r2.y + 0.0;
-  const double wL = s0 * l0.z + s1 * l1.z + s2 * l2.z + 0.0, wR = s0 * r0.z + s1 * r1.z + s2 * r2.z + 0.0;
+  if (!hit) {
+    int L, R, kb0, kb1, kb2;
+    const int L0 = F ? 0 : (st ? rc->ekb : m.elem_kb[ux(e)]) - 1;
+    if constexpr (VM == 0) {
+      const ZSigma<F> z{st ? st_node_z(*rc, 0) : node_z<F>(m, n0), st ? st_node_z(*rc, 1) : node_z<F>(m, n1),
+                        st ? st_node_z(*rc, 2) : node_z<F>(m, n2), sig, nv};
+      kb0 = z.q0.kb, kb1 = z.q1.kb, kb2 = z.q2.kb;
+      z_bracket(z, s0, s1, s2, pz, L0, min(kb0, min(kb1, kb2)), R0, true, hint, L, R, w1, w2);
+      c.kept = true;
+      c.zL = z.nodes(L);
+      c.zR = z.nodes(R);
+    } else {
+      // kb with a flag where the node's column is not non-decreasing (k_pack_levels), or is not kept
+      const int f0 = m.zn ? m.nkz[ux(n0)] : m.kb[ux(n0)], f1 = m.zn ? m.nkz[ux(n1)] : m.kb[ux(n1)],
+                f2 = m.zn ? m.nkz[ux(n2)] : m.kb[ux(n2)];
+      kb0 = f0 & kKbMask, kb1 = f1 & kKbMask, kb2 = f2 & kKbMask;
+      const ZColumns z{m, h0, n0, n1, n2};
+      const bool mono = m.zn && !((f0 | f1 | f2) & ~kKbMask);
+      z_bracket(z, s0, s1, s2, pz, L0, min(kb0, min(kb1, kb2)), R0, mono, hint, L, R, w1, w2);
+      c.kept = mono;
+      c.zL = z.nodes(L);
+      c.zR = z.nodes(R);
+    }
+    c.L = L;
+    c.R = R;
+    // the three nodes' level rows (64-bit row offsets), then two levels of each
+    const double4* U = reinterpret_cast<const double4*>(m.uvw);
+    auto at = [&](int node, int level, int kb) {
+      const double4 q = U[(uint64_t)ux(node) * ux(nv) + ux(F ? level : max(level, kb))];
+      return double3{q.x, q.y, q.z};
+    };
+    c.u0 = at(n0, L, kb0), c.u1 = at(n1, L, kb1), c.u2 = at(n2, L, kb2);
+    c.v0 = at(n0, R, kb0), c.v1 = at(n1, R, kb1), c.v2 = at(n2, R, kb2);
+  }
+  const double uL = s0 * c.u0.x + s1 * c.u1.x + s2 * c.u2.x + 0.0, vL = s0 * c.u0.y + s1 * c.u1.y + s2 * c.u2.y + 0.0;
+  const double uR = s0 * c.v0.x + s1 * c.v1.x + s2 * c.v2.x + 0.0, vR = s0 * c.v0.y + s1 * c.v1.y + s2 * c.v2.y + 0.0;
+  const double wL = s0 * c.u0.z + s1 * c.u1.z + s2 * c.u2.z + 0.0, wR = s0 * c.v0.z + s1 * c.v1.z + s2 * c.v2.z + 0.0;
   uo = w1 * uL + w2 * uR;
   vo = w1 * vL + w2 * vR;
   wo = w1 * wL + w2 * wR;
@@ -553,7 +603,11 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
   ElemGeom geo;  // set by every walk before its first use
   int slot = -1;  // geo's staged slot (ST)
   bool geo_valid = false;
+  BtCell cell;
+  double fu = 0.0, fv = 0.0;  // the interpolated velocity at the last point, where there is one
+  bool interpolated = false;
   while (true) {
+    interpolated = false;
     const double dtb = fmin(dtbk, time_rm);
     xtx = x0x - dtb * uix;
     xty = x0y - dtb * uiy;
@@ -603,7 +657,9 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
       const double len = sqrt(v2x * v2x + v2y * v2y);
       const double tx = v2x / len, ty = v2y / len;
       double iu, iv, iw;
-      interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, rc, xtx, xty, xtz, iu, iv, iw, hint);
+      interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, rc, cell, xtx, xty, xtz, iu, iv, iw, hint);
+      fu = iu;
+      fv = iv;
       const double d = iu * tx + iv * ty;
       uix = tx * d;
       uiy = ty * d;
@@ -611,8 +667,11 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
       status |= GSH_BT_SLIDE;
     } else {
       time_rm -= dtb;
-      interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, rc, xtx, xty, xtz, uix, uiy, uiz, hint);
+      interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, rc, cell, xtx, xty, xtz, uix, uiy, uiz, hint);
+      fu = uix;
+      fv = uiy;
     }
+    interpolated = true;
     if (time_rm <= 0.0) break;
     if (uix * uix + uiy * uiy <= a.velmin2) {
       ux = uix;
@@ -635,9 +694,14 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
     t2 = t1;
     t1 = time_rm;
   }
-  double iw;
-  interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, (ST && slot >= 0) ? rec + slot : nullptr, xtx, xty, xtz, ux, uy, iw,
-                          hint);
+  // the velocity at the last point: already interpolated unless the walk stuck or left the mesh there
+  ux = fu;
+  uy = fv;
+  if (!interpolated) {
+    double iw;
+    interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, (ST && slot >= 0) ? rec + slot : nullptr, cell, xtx, xty, xtz, ux,
+                               uy, iw, hint);
+  }
   foot = cur;
 }
 
@@ -648,8 +712,8 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
 // ST: the workgroup first stages its element patch in LDS (all sides and levels, no list).
 // F: a mesh with kb = 0 at every node whose last sigma is 0 (VM = 0).
 template <int VM, bool ST, bool F>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) k_backtrack(DMesh m, StepArgs a, const int32_t* list_side,
-                                                   const int32_t* list_lev, int32_t count) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8)))
+k_backtrack(DMesh m, StepArgs a, const int32_t* list_side, const int32_t* list_lev, int32_t count) {
   __shared__ double sig[VM == 0 ? 1024 : 1];
   __shared__ int st_key[ST ? kStSlots : 1];
   __shared__ StElem st_rec[ST ? kStSlots : 1];
