@@ -187,6 +187,13 @@ __global__ void __launch_bounds__(256) k_pcg_init(const PcgSys<VT>* __restrict__
 // (tile_tree_wide), so results equal the 256-thread form's bit for bit. The 256-thread form walks
 // its R sub-rounds one after another, each waiting for entries and then gathers; the wide form has
 // all 4 R chunks of a tile in flight, which a system of few tiles needs (launch_pcg_phase).
+//
+// What the two forms load first differs. The wide one, a single wait chain per thread, requests the
+// row pointers before the done test and every column before the first gather. The narrow one runs
+// where many waves share a SIMD, and among a batch's finished systems: it tests done first, and its
+// FP32 chunk takes each entry's column and gathers together, which keeps it at 71 registers and 7
+// waves a SIMD (with every column held at once 76 and 6: batched mixed Jacobi solves of 16 x 501,264
+// rows 19.3 ms against 16.8, of 96 systems of 5,000 to 200,000 rows 12.6 against 11.8).
 template <class VT, bool W>
 struct Chunk {
   // nonzeros of a 64-row chunk held in registers: 10 per lane; 9 in the wide form, whose 16 waves'
@@ -208,6 +215,19 @@ __device__ __forceinline__ void load_chunk(const SysView<VT>& S, gptr<const VT> 
   c.s0 = s0;
   c.e0 = e0;
   if (c.e0 - c.s0 > c.kCap) return;
+  if constexpr (!W) {
+#pragma unroll
+    for (int m = 0; m < c.kM; ++m) {
+      const int kk = c.s0 + lane + 64 * m;
+      if (kk < c.e0) {
+        const int col = col_of(S, kk, r0w);
+        c.v[m] = S.val[kk];
+        c.zc[m] = S.z[col];
+        c.pc[m] = po[col];
+      }
+    }
+    return;
+  }
   int col[c.kM];
 #pragma unroll
   for (int m = 0; m < c.kM; ++m) {
@@ -234,6 +254,7 @@ __device__ __forceinline__ void pcg_phase_a_body(const SysView<VT>& S, int tile,
   const int n = S.n;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int base = tile * kTpb * R;
+  if (!W && load_done(st) >= 0) return;
   // FP64: the row pointers of every sub-round first: they depend on nothing, so each sub-round's
   // chunk then waits for two memory steps (entries, then gathers) instead of three. FP32 loads them
   // per sub-round: its registers would otherwise drop it from 7 to 5 waves per SIMD, which its
@@ -254,7 +275,7 @@ __device__ __forceinline__ void pcg_phase_a_body(const SysView<VT>& S, int tile,
       }
     }
   }
-  if (load_done(st) >= 0) return;
+  if (W && load_done(st) >= 0) return;
   const int k = st->k;
   const gptr<VT> pn = (k & 1) ? S.pb : S.pa;
   const gptr<const VT> po = (k & 1) ? S.pa : S.pb;
@@ -388,6 +409,7 @@ __device__ __forceinline__ void pcg_phase_b_body(const SysView<VT>& S, int tile,
   gptr<PcgState> st = S.st;
   const int n = S.n;
   const int base = tile * kTpb * R;
+  if (!W && load_done(st) >= 0) return;
   VT xv[J], pv[J], rv[J], qv[J], dv[J];
 #pragma unroll
   for (int j = 0; j < J; ++j) {
@@ -399,7 +421,7 @@ __device__ __forceinline__ void pcg_phase_b_body(const SysView<VT>& S, int tile,
       dv[j] = S.invd[i];
     }
   }
-  if (load_done(st) >= 0) return;
+  if (W && load_done(st) >= 0) return;
   const int k = st->kk;
   const gptr<const VT> p = (k & 1) ? S.pb : S.pa;
 #pragma unroll

@@ -1,0 +1,40 @@
+"""What the compiler gives the kernels whose speed hangs on their occupancy, from its own
+kernel-resource-usage remarks on this library's sources (no GPU)."""
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from gschism_amd import build
+
+
+def _usage(source, tmp_path):
+    """{demangled kernel name: {"VGPRs": .., "Occupancy": .., "ScratchSize": ..}} of one source."""
+    cmd = [build.HIPCC, *build.COMMON, *build.HIP_FLAGS, "-Rpass-analysis=kernel-resource-usage", "--cuda-device-only",
+           "-c", str(build.CSRC / source), "-o", str(tmp_path / "device.o")]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    names = subprocess.run(["c++filt"], input=r.stderr, capture_output=True, text=True).stdout
+    out, cur = {}, None
+    for line in names.splitlines():
+        m = re.search(r"remark: +Function Name: (?:void )?(.*?)\(", line)
+        if m:
+            cur = out.setdefault(m.group(1), {})
+        m = re.search(r"remark: +(VGPRs|Occupancy|ScratchSize)[^:]*: (\d+)", line)
+        if m and cur is not None:
+            cur[m.group(1)] = int(m.group(2))
+    return out
+
+
+@pytest.mark.skipif(not (shutil.which(build.HIPCC) and shutil.which("c++filt")), reason="needs hipcc and c++filt")
+def test_narrow_jacobi_phases_keep_their_waves(tmp_path):
+    """Batched and large Jacobi solves run the 256-thread phases at as many waves a SIMD as their
+    registers give: 7 for the FP32 phase A (71 VGPRs), 4 for FP64 up to 4 rows per thread."""
+    u = _usage("pcg_kernels.hip", tmp_path)
+    for rpt in (1, 2, 4, 8):
+        assert u[f"gsh::k_pcg_phase_a<float, {rpt}, false>"]["Occupancy"] >= 7
+        assert u[f"gsh::k_pcg_phase_a<double, {rpt}, false>"]["Occupancy"] >= (3 if rpt == 8 else 4)
+    for name, k in u.items():
+        if "k_pcg_phase" in name or "k_pcg_run" in name:
+            assert k["ScratchSize"] == 0, name
