@@ -1439,7 +1439,10 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.kb = P.upload(hm.kb);
     d.sigma = P.upload(hm.sigma);
     d.vmode = hm.vmode;
-    d.flat = hm.vmode == 0 && hm.sigma[nv - 1] == 0.0 && std::all_of(hm.kb.begin(), hm.kb.end(), [](int32_t k) { return k == 0; });
+    d.sig_mono = hm.vmode == 0 && std::all_of(hm.sigma.begin() + 1, hm.sigma.end() - 1,
+                                              [](double s) { return s >= -1.0 && s <= 0.0; });
+    d.flat = d.sig_mono && hm.sigma[nv - 1] == 0.0 &&
+             std::all_of(hm.kb.begin(), hm.kb.end(), [](int32_t k) { return k == 0; });
     if (hm.vmode != 0) {
       d.zn = P.alloc<double>((int64_t)n * nv);
       d.nkz = P.alloc<int32_t>(n);

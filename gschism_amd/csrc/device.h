@@ -25,7 +25,8 @@ struct DMesh {
   // sigma per level, 1 = ivcor 1 with a sigma per node and level, 2 = ivcor 2 (SZ)
   int32_t vmode;
   int32_t bt_stage;         // backtracking stages each workgroup's element patch in LDS (0: off)
-  int32_t flat;             // vmode 0, kb = 0 at every node and the last sigma exactly 0
+  int32_t sig_mono;         // vmode 0, every sigma between the first and the last in [-1, 0]: levels do not decrease
+  int32_t flat;             // sig_mono, kb = 0 at every node and the last sigma exactly 0
   int32_t izlev;            // nz - 1: the level at -min(h, h_s) (vmode 2)
   double h_s, h_c;          // (vmode 2)
   const double* sig_node;   // [n][nvrt] (vmode 1)

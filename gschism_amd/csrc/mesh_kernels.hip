@@ -708,7 +708,8 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
 // backtrackAllNodes (meshdata.cu:3547-3660), one thread per (side, level): consecutive
 // lanes are consecutive levels of one side, so the nodal [node][level] gathers of a wave
 // fall on a few contiguous cache lines.
-// VM: the vertical coordinate system (DMesh::vmode); 0, one sigma per level, keeps it in LDS.
+// VM: 0, one sigma per level (kept in LDS) and levels that do not decrease in any wet column; 1, each
+// node's own levels (DMesh::vmode 1 and 2, and 0 where levels may decrease).
 // ST: the workgroup first stages its element patch in LDS (all sides and levels, no list).
 // F: a mesh with kb = 0 at every node whose last sigma is 0 (VM = 0).
 template <int VM, bool ST, bool F>
@@ -822,11 +823,14 @@ void launch_backtrack(const DMesh& mesh, const StepArgs& a, const int32_t* ls, c
   const dim3 grid((unsigned)((total + 255) / 256));
   const bool stage = m.bt_stage != 0 && !ls;
   auto go = [&](auto ker) { hipLaunchKernelGGL(ker, grid, dim3(256), 0, st, m, a, ls, ll, count); };
-  if (m.vmode == 0 && stage)
+  // One sigma per level: a wet node's levels do not decrease where 0 <= h0 < H and every sigma between
+  // bed and surface lies in [-1, 0], which VM = 0 relies on. Outside that, VM = 1 searches in full.
+  const bool sigma = m.vmode == 0 && m.sig_mono && a.h0 >= 0.0;
+  if (sigma && stage)
     go(k_backtrack<0, true, false>);
-  else if (m.vmode == 0 && m.flat)
+  else if (sigma && m.flat)
     go(k_backtrack<0, false, true>);
-  else if (m.vmode == 0)
+  else if (sigma)
     go(k_backtrack<0, false, false>);
   else if (stage)
     go(k_backtrack<1, true, false>);

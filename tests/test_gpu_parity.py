@@ -781,3 +781,44 @@ def test_velocity_kernels_level_edges(ctx, nvrt):
     om.nodal_velocity(p)
     assert_bitwise(mesh.get(L.F_NODE_UVW), om.get(L.F_NODE_UVW), f"nodal velocity, {nvrt} levels")
     mesh.close()
+
+
+@pytest.mark.parametrize("staged", [False, True])
+@pytest.mark.parametrize("levels", ["above-surface", "below-bed", "below-bed-kb", "land-below-h0"])
+def test_backtrack_levels_out_of_order(ctx, levels, staged):
+    """Columns whose levels decrease somewhere: sigma above 0 or below -1 between the bed and the
+    surface, and nodes of negative depth that a negative h0 calls wet. The bracket search may then
+    not start from an earlier bracket: feet, velocities and flags of the full search."""
+    w = np.linspace(0.0, 1.0, 13)
+    sigma = -1.0 + w
+    kb, h0, depth = None, None, lambda xy: np.full(xy.shape[0], 10.0) + 3e-4 * xy[:, 0]
+    if levels == "above-surface":
+        sigma = -1.0 + 1.6 * w
+    elif levels == "land-below-h0":
+        h0, flat = -100.0, depth
+        depth = lambda xy: flat(xy) - np.where(np.hypot(xy[:, 0] - 8000.0, xy[:, 1] - 5000.0) < 2500.0, 13.0, 0.0)
+    else:
+        sigma = -1.8 + 1.8 * w
+        kb = np.arange(40 * 28, dtype=np.int32) % 4 if levels == "below-bed-kb" else None
+    spec = cases.CaseSpec(f"levels-{levels}", 40, 28, 400.0, nvrt=sigma.size, depth=10.0, substeps=6)
+    data = cases.make_case(spec)
+    mesh = core.Mesh(ctx, data.xy, data.elnode, depth(data.xy), sigma, open_bnd=data.open_bnd, kb=kb)
+    eta, uvw, su2 = cases.initial_state(spec, mesh.topology(L.T_XY), cases.side_centres(mesh), data.sigma)
+    uvw[..., 2] += 0.004 * cases.normal(5, uvw[..., 2].size).reshape(uvw[..., 2].shape)
+    p = cases.step_params(spec)
+    if h0 is not None:
+        p.h0 = h0
+    om = oracle_mesh_for(mesh, sigma)
+    for m in (mesh, om):
+        m.set(L.F_ETA2, eta)
+        m.set(L.F_NODE_UVW, uvw)
+        m.set(L.F_SIDE_U2, su2)
+    mesh.update_levels(p)
+    om.levels(p)
+    mesh.set_backtrack_staging(staged)
+    print(f"[gpu] backtracking, {levels}, staged {staged}", flush=True)
+    mesh.backtrack(p)
+    om.backtrack(p, nthreads=8)
+    for f in (L.F_FOOT, L.F_BTU, L.F_BSTATUS):
+        assert_bitwise(mesh.get(f), om.get(f), f"field {f}")
+    mesh.close()
