@@ -1377,18 +1377,23 @@ __device__ void momentum_free_slip(const DMesh& m, int s, double* u) {
 // (of 25 us a wave, 16 went into loads waited for in turn; 645,122 sides x 31 levels: 387 -> 186 us,
 // 4.3 TB/s; now half the time is the serial sweep, four divisions a level).
 // Strides: zs odd and us = 2 zs spread the sides' reads of one level over the banks.
+// NI, the items of either array per lane, is a power of two up to kMomItems with g sides' rows in 64 NI
+// items: 32 sides of few levels would otherwise read and write their last item many times over, at two
+// waves a SIMD (156,000 sides, 16 items / as many as they need: 2 levels 16.7 / 11.1 us, 5 levels 21.1 /
+// 15.8, 8 levels 25.6 / 19.9; 840,000 sides x 16 levels 149 with 8 items).
 constexpr int kMomItems = 16;
 constexpr int kMomLds = 24 * 1024;
 
-
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) k_momentum(DMesh m, StepArgs a, int g) {
+template <int NI>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, NI < kMomItems ? 8 : 2)))
+k_momentum(DMesh m, StepArgs a, int g) {
   extern __shared__ double lds[];
   const int nv = m.nvrt, zs = nv | 1, us = 2 * zs;
   double* Lu = lds;
   double* Lz = lds + g * us;
   const int s0 = blockIdx.x * g;
   const int gc = min(g, m.ns - s0);
-  const int total = gc * nv;  // <= 64 kMomItems
+  const int total = gc * nv;  // <= 64 NI
   const int t = threadIdx.x, sl = t >> 1, c = t & 1;
   const float inv = 1.0f / (float)nv;
   const double* zc = m.zc + (int64_t)s0 * nv;
@@ -1396,11 +1401,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
   const int s = s0 + min(sl, gc - 1);
   const int4 sr = m.side[s];
   __builtin_amdgcn_sched_barrier(0);  // the compiler would move each load down to its use
-  double z[kMomItems];
-  f64x2 b[kMomItems];
+  double z[NI];
+  f64x2 b[NI];
   // past the end the last item is read and written again
 #pragma unroll
-  for (int j = 0; j < kMomItems; ++j) {
+  for (int j = 0; j < NI; ++j) {
     const int i = min(t + 64 * j, total - 1);
     z[j] = zc[i];
     b[j] = btu[i];
@@ -1415,7 +1420,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
   const double gr0 = m.grav2[sr.x], gr1 = m.grav2[sr.y], cd0 = m.cd[sr.x], cd1 = m.cd[sr.y];
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int j = 0; j < kMomItems; ++j) {
+  for (int j = 0; j < NI; ++j) {
     int k;
     const int r = split_row(min(t + 64 * j, total - 1), inv, nv, k);
     Lz[r * zs + k] = z[j];
@@ -1431,7 +1436,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
   wave_lds_sync();
   f64x2* out = reinterpret_cast<f64x2*>(m.su2) + (int64_t)s0 * nv;
 #pragma unroll
-  for (int j = 0; j < kMomItems; ++j) {
+  for (int j = 0; j < NI; ++j) {
     const int i = t + 64 * j;
     if (i < total) {
       int k;
@@ -1542,7 +1547,18 @@ void launch_momentum(const DMesh& m, const StepArgs& a, hipStream_t st) {
   // sides per wave: one per two lanes, as many as 24 KB of LDS and kMomItems loads a lane hold
   const int row = 24 * (m.nvrt | 1);
   const int g = max(1, min(32, min(kMomLds / row, 64 * kMomItems / m.nvrt)));
-  hipLaunchKernelGGL(k_momentum, dim3((unsigned)((m.ns + g - 1) / g)), dim3(64), (size_t)g * row, st, m, a, g);
+  auto go = [&](auto ker) {
+    hipLaunchKernelGGL(ker, dim3((unsigned)((m.ns + g - 1) / g)), dim3(64), (size_t)g * row, st, m, a, g);
+  };
+  const int items = (g * m.nvrt + 63) / 64;
+  if (items <= 2)
+    go(k_momentum<2>);
+  else if (items <= 4)
+    go(k_momentum<4>);
+  else if (items <= 8)
+    go(k_momentum<8>);
+  else
+    go(k_momentum<kMomItems>);
 }
 
 // ---------------------------------------------------------------- vertical velocity

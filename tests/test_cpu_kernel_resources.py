@@ -27,7 +27,10 @@ def _usage(source, tmp_path):
     return out
 
 
-@pytest.mark.skipif(not (shutil.which(build.HIPCC) and shutil.which("c++filt")), reason="needs hipcc and c++filt")
+needs_compiler = pytest.mark.skipif(not (shutil.which(build.HIPCC) and shutil.which("c++filt")), reason="needs hipcc and c++filt")
+
+
+@needs_compiler
 def test_narrow_jacobi_phases_keep_their_waves(tmp_path):
     """Batched and large Jacobi solves run the 256-thread phases at as many waves a SIMD as their
     registers give: 7 for the FP32 phase A (71 VGPRs), 4 for FP64 up to 4 rows per thread."""
@@ -38,3 +41,13 @@ def test_narrow_jacobi_phases_keep_their_waves(tmp_path):
     for name, k in u.items():
         if "k_pcg_phase" in name or "k_pcg_run" in name:
             assert k["ScratchSize"] == 0, name
+
+
+@needs_compiler
+def test_momentum_of_few_levels_keeps_its_waves(tmp_path):
+    """Waves of few levels hold few loads: on up to 4 and 8 levels (2 and 4 items a lane) they leave
+    registers for 5 and 4 waves a SIMD, where the 16 items of many levels leave 2."""
+    u = _usage("mesh_kernels.hip", tmp_path)
+    for items, waves in ((2, 5), (4, 4), (8, 3), (16, 2)):
+        k = u[f"gsh::k_momentum<{items}>"]
+        assert k["Occupancy"] >= waves and k["ScratchSize"] == 0
