@@ -262,6 +262,29 @@ struct gsh_solver {
   int tiles_for(int rows) const { return (rows + kTpb * rpt - 1) / (kTpb * rpt); }
 };
 
+// The longest row of a CSR pattern and its largest |column - row| (pcg_run_fits). Where every row's
+// columns ascend, which one vectorised pass shows (no entry below its predecessor but at a row's
+// start), the rows' ends have the extremes.
+static void pattern_extent(const std::vector<int32_t>& indptr, const std::vector<int32_t>& indices, int32_t& max_row,
+                           int32_t& band) {
+  const int32_t n = (int32_t)indptr.size() - 1, nnz = indptr[n];
+  const int32_t* col = indices.data();
+  int32_t descents = 0, longest = 0, reach = 0;
+  for (int32_t k = 1; k < nnz; ++k) descents += col[k] < col[k - 1];
+  for (int32_t i = 0; i < n; ++i) {
+    const int32_t a = indptr[i], b = indptr[i + 1];
+    longest = std::max(longest, b - a);
+    if (b == a) continue;
+    if (a > 0) descents -= col[a] < col[a - 1];
+    reach = std::max(reach, std::max(std::abs(i - col[a]), std::abs(col[b - 1] - i)));
+  }
+  if (descents != 0)
+    for (int32_t i = 0; i < n; ++i)
+      for (int32_t k = indptr[i]; k < indptr[i + 1]; ++k) reach = std::max(reach, std::abs(col[k] - i));
+  max_row = longest;
+  band = reach;
+}
+
 static void solver_alloc(gsh_solver* s, int32_t n, int64_t nnz, const std::vector<int32_t>& indptr,
                          const std::vector<int32_t>& indices, const std::vector<int32_t>& diag_abs) {
   s->n = n;
@@ -272,21 +295,25 @@ static void solver_alloc(gsh_solver* s, int32_t n, int64_t nnz, const std::vecto
   s->rowptr = P.upload(indptr);
   s->col = P.upload(indices);
   s->diag = P.upload(diag_abs);
-  // int16 column offsets from the first row of each 64-row chunk, when the bandwidth allows
+  // int16 column offsets from the first row of each 64-row chunk, when the bandwidth allows (a chunk's
+  // entries in one loop without exits, which the compiler vectorises)
   {
     std::vector<int16_t> cdel(nnz);
+    const int32_t* col = indices.data();
+    int16_t* out = cdel.data();
     bool ok = true;
-    for (int32_t i = 0; i < n && ok; ++i)
-      for (int32_t k = indptr[i]; k < indptr[i + 1]; ++k) {
-        const int32_t d = indices[k] - (i & ~63);
-        if (d < -32768 || d > 32767) {
-          ok = false;
-          break;
-        }
-        cdel[k] = (int16_t)d;
+    for (int32_t r = 0; r < n; r += 64) {
+      int32_t lo = r, hi = r;
+      for (int32_t k = indptr[r], end = indptr[std::min(r + 64, n)]; k < end; ++k) {
+        lo = std::min(lo, col[k]);
+        hi = std::max(hi, col[k]);
+        out[k] = (int16_t)(col[k] - r);
       }
+      ok = ok && lo - r >= -32768 && hi - r <= 32767;
+    }
     s->cdel = ok ? P.upload(cdel) : nullptr;
   }
+  if (n <= kRunRows) pattern_extent(indptr, indices, s->max_row, s->band);
   s->val = P.alloc<double>(nnz);
   s->b = P.alloc<double>(n);
   s->x = P.alloc<double>(n);
@@ -316,10 +343,6 @@ static void solver_alloc(gsh_solver* s, int32_t n, int64_t nnz, const std::vecto
   s->dtiles = P.alloc<TileRef>(nt);
   s->red2 = P.alloc<double>(2);
   s->run_words = P.alloc<uint64_t>(kRunWords);
-  for (int32_t i = 0; i < n; ++i) {
-    s->max_row = std::max(s->max_row, indptr[i + 1] - indptr[i]);
-    for (int32_t k = indptr[i]; k < indptr[i + 1]; ++k) s->band = std::max(s->band, std::abs(indices[k] - i));
-  }
   if (s->precision == GSH_PREC_MIXED) {
     s->val32 = P.alloc<float>(nnz);
     s->r64 = P.alloc<double>(n);
@@ -1471,11 +1494,6 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.etype = P.upload(std::vector<int8_t>(n, -1));
     d.elem = P.upload(erec);
     d.area = P.upload(m->geo.area);
-    {
-      std::vector<double2> ai(ne);
-      for (int32_t e = 0; e < ne; ++e) ai[e] = make_double2(m->geo.area[e], 1.0 / m->geo.area[e]);
-      d.area_inv = P.upload(ai);
-    }
     d.gradphi = P.upload(m->geo.gradphi);
     d.elem_wet = P.alloc<int8_t>(ne);
     d.elem_kb = P.alloc<int32_t>(ne);
@@ -1488,12 +1506,6 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.side_cx = P.upload(m->geo.side_cx);
     d.side_cy = P.upload(m->geo.side_cy);
     d.side_len = P.upload(m->geo.side_len);
-    {
-      std::vector<double4> sg(ns);
-      for (int32_t s = 0; s < ns; ++s)
-        sg[s] = make_double4(m->geo.side_nx[s], m->geo.side_ny[s], m->geo.side_len[s], (double)srec[s].z);
-      d.side_geo = P.upload(sg);
-    }
     d.side_kb = P.alloc<int32_t>(ns);
     d.side_wet = P.alloc<int8_t>(ns);
     d.zc = P.alloc<double>((int64_t)ns * nv);
@@ -1507,15 +1519,6 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.chi = P.alloc<double>(ns);
     d.ball_ptr = P.upload(t.ball_ptr);
     d.ball_elem = P.upload(t.ball_elem);
-    {
-      std::vector<int4> br(t.ball_elem.size());
-      for (size_t j = 0; j < br.size(); ++j) {
-        const int32_t e = t.ball_elem[j], l = t.ball_loc[j];
-        const int32_t* es = &t.elside[3 * (size_t)e];  // side c lies opposite corner c
-        br[j] = make_int4(e, es[l], es[(l + 1) % 3], es[(l + 2) % 3]);
-      }
-      d.ball_rec = P.upload(br);
-    }
     d.ball_loc = P.upload(t.ball_loc);
     d.ball_slot = P.upload(ball_slot);
     d.nbr_ptr = P.upload(t.nbr_ptr);
@@ -1523,6 +1526,16 @@ int gsh_mesh_create(gsh_ctx* ctx, const gsh_mesh_desc* desc, gsh_mesh** out, int
     d.csr_slot = P.upload(t.csr_slot);
     d.indptr = P.upload(t.indptr);
     d.diag_off = P.upload(t.diag_off);
+    // records packed from the arrays above, on the device: built here and copied they took 2 to 5 % of
+    // a mesh's creation
+    const int32_t nball = (int32_t)t.ball_elem.size();
+    double2* area_inv = P.alloc<double2>(ne);
+    double4* side_geo = P.alloc<double4>(ns);
+    int4* ball_rec = P.alloc<int4>(nball);
+    launch_pack_geometry(d, area_inv, side_geo, ball_rec, nball, ctx->stream);
+    d.area_inv = area_inv;
+    d.side_geo = side_geo;
+    d.ball_rec = ball_rec;
     // initial levels with eta2 = 0
     gsh_step_params p;
     gsh_step_params_default(&p);
@@ -1922,7 +1935,9 @@ int gsh_solver_create_csr(gsh_ctx* ctx, int32_t n, int64_t nnz, const int32_t* i
     GSH_REQUIRE(nnz < (int64_t)1 << 31, GSH_E_ARG, "nnz exceeds int32 indexing");
     GSH_REQUIRE(indptr[0] == 0 && indptr[n] == nnz, GSH_E_ARG, "indptr must start at 0 and end at nnz");
     for (int32_t i = 0; i < n; ++i) GSH_REQUIRE(indptr[i + 1] >= indptr[i], GSH_E_ARG, "indptr must be non-decreasing");
-    for (int64_t k = 0; k < nnz; ++k) GSH_REQUIRE(indices[k] >= 0 && indices[k] < n, GSH_E_ARG, "column out of range");
+    bool in_range = true;
+    for (int64_t k = 0; k < nnz; ++k) in_range &= (uint32_t)indices[k] < (uint32_t)n;
+    GSH_REQUIRE(in_range, GSH_E_ARG, "column out of range");
     ctx->set();
     auto s = std::make_unique<gsh_solver>();
     s->ctx = ctx;

@@ -217,6 +217,7 @@ struct BlkSys {
 };
 
 // ---------------------------------------------------------------- launch wrappers
+void launch_pack_geometry(const DMesh& m, double2* area_inv, double4* side_geo, int4* ball_rec, int nball, hipStream_t s);
 void launch_levels(const DMesh& m, const StepArgs& a, hipStream_t s);
 void launch_backtrack(const DMesh& m, const StepArgs& a, const int32_t* list_side, const int32_t* list_lev,
                       int32_t count, hipStream_t s);
@@ -242,7 +243,9 @@ void launch_pcg_phase(int which, const PcgSys<VT>* sys, const TileRef* tiles, in
 // Up to `iters` iterations of one system in one launch, for systems that pcg_run_fits accepts: max_row,
 // the longest row; band, the largest |column - row|. words: kRunWords exchange words, zero at first;
 // epoch: above iters plus that of every earlier launch on these words, so at least 1.
-constexpr int kRunWords = 6 * 128;
+constexpr int kRunTiles = 128;                   // tiles at most
+constexpr int kRunRows = 4 * kTpb * kRunTiles;   // rows at most
+constexpr int kRunWords = 6 * kRunTiles;
 bool pcg_run_fits(int ntiles, int rpt, int max_row, int band);
 template <class VT>
 void launch_pcg_run(const PcgSys<VT>* sys, int ntiles, int rpt, uint64_t* words, uint32_t epoch, int band, int iters,

@@ -49,6 +49,36 @@ __device__ __forceinline__ double zcoord(const DMesh& m, double h0, int node, in
   return z_wet(m, node, eta, h, m.kb[node], k);
 }
 
+// ---------------------------------------------------------------- packed geometry (mesh creation)
+// DMesh::area_inv, side_geo (the side's unit normal as populateSides forms it, meshdata.cu:2283-2287)
+// and ball_rec (side c of an element lies opposite its corner c).
+__global__ void k_pack_geometry(DMesh m, double2* __restrict__ area_inv, double4* __restrict__ side_geo,
+                                int4* __restrict__ ball_rec, int nball) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < m.ne) {
+    const double a = m.area[i];
+    area_inv[i] = make_double2(a, 1.0 / a);
+  }
+  if (i < m.ns) {
+    const int4 sr = m.side[i];
+    const double vx = -(m.y[sr.x] - m.y[sr.y]), vy = m.x[sr.x] - m.x[sr.y];
+    const double l = sqrt(vx * vx + vy * vy);
+    side_geo[i] = make_double4(vx / l, vy / l, m.side_len[i], (double)sr.z);
+  }
+  if (i < nball) {
+    const int e = m.ball_elem[i], l = m.ball_loc[i];
+    const int* es = reinterpret_cast<const int*>(m.elem + 2 * (int64_t)e) + 3;
+    ball_rec[i] = make_int4(e, es[l], es[l == 2 ? 0 : l + 1], es[l == 0 ? 2 : l - 1]);
+  }
+}
+
+void launch_pack_geometry(const DMesh& m, double2* area_inv, double4* side_geo, int4* ball_rec, int nball,
+                          hipStream_t st) {
+  const int count = max(nball, max(m.ne, m.ns));
+  hipLaunchKernelGGL(k_pack_geometry, dim3((count + 255) / 256), dim3(256), 0, st, m, area_inv, side_geo, ball_rec,
+                     nball);
+}
+
 // ---------------------------------------------------------------- a3: levels and wet/dry
 // ul0ComputeDryElements (meshdata.cu:5550-5580)
 __global__ void k_elem_levels(DMesh m, double h0) {

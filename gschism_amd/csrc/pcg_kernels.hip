@@ -501,7 +501,6 @@ __global__ void __launch_bounds__(W ? kTpb * R : kTpb) k_pcg_phase_b(const PcgSy
 // per CU two such launches are resident together (the host admits no more, RunSlots). A launch whose
 // workgroups do not become resident together all the same (another process's solve) gives up after
 // kRunSpin polls and leaves the solve to the phases.
-constexpr int kRunTiles = 128;
 constexpr int kRunRow = 12;     // entries of a row held in registers
 constexpr int kRunWin = 6144;   // p of the tile and its halo, words of LDS
 

@@ -715,6 +715,28 @@ def test_small_systems_in_one_launch(ctx, rpt, n, maxiter):
     s.close()
 
 
+@pytest.mark.parametrize("order", [(2, 0, 4, 1, 3), (3, 4, 0, 2, 1), (4, 3, 2, 1, 0)])
+def test_one_launch_with_columns_in_any_order(ctx, order):
+    """A CSR pattern whose rows do not ascend, their first and last entries near the diagonal or far
+    from it: the window of p that a workgroup keeps covers the farthest column all the same."""
+    n = 5 * 1024 + 77
+    rows = np.repeat(np.arange(n), 5)
+    cols = rows + np.tile(np.array([-700, -1, 0, 1, 450])[list(order)], n)
+    on = (cols >= 0) & (cols < n)
+    rows, cols = rows[on], cols[on].astype(np.int32)
+    ip = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    val = np.where(rows == cols, 4.5, -1.0)
+    b = cases.normal(71, n)
+    s = core.Solver(None, ctx=ctx, indptr=ip, indices=cols)
+    s.set_values(val)
+    print(f"[gpu] one-launch solve, columns in the order {order}", flush=True)
+    x, it, _ = s.solve(b, rtol=1e-300, maxiter=30, check_every=10)
+    xo, ito, _, _ = O.pcg(ip, cols, val, b, rtol=1e-300, maxiter=30, check_every=10, rows_per_thread=4)
+    assert it == ito
+    assert_bitwise(x, xo, f"solution, columns in the order {order}")
+    s.close()
+
+
 def test_concurrent_one_launch_solves(ctx):
     """Four contexts solving at once, together more workgroups than may wait for each other on the
     device: some take the phases, all return the same bits, three times in a row."""
