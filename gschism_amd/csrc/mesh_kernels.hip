@@ -228,15 +228,15 @@ __device__ __forceinline__ double third(double a) {
   return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-3.0, q, a), y, q), 3.0, a);
 }
 
-// LDS-staged element patch (k_backtrack with ST = true): every element the walk and the
-// interpolation read, for the elements on both sides of each of the workgroup's sides and their
-// neighbours, in one record, in an LDS table keyed by element id (open addressing, linear
-// probing). An element outside the patch is read from global memory as before, so the values
+// LDS-staged element patch (k_backtrack with ST = true): what the walk reads of an element and the
+// vertical search of its nodes, for the elements on both sides of each of the workgroup's sides and
+// their neighbours, in one record, in an LDS table keyed by element id (open addressing, linear
+// probing). The interpolation's area and reciprocal come from DMesh::area_inv, once per element
+// entered (BtCell). An element outside the patch is read from global memory as before, so the values
 // and results are those of the unstaged kernel.
 struct StElem {
   double x[3], y[3];    // corners in node order n0, n1, n2
-  double eta[3], h[3];  // eta2 and depth of the corners
-  double area;
+  double eta[3], h[3];  // eta2 and depth of the corners (VM = 0)
   int n[3], s[3];       // node ids; sides opposite the corners
   int ekb, kb[3];       // element bottom level; the corners' kb
 };
@@ -310,7 +310,6 @@ __device__ void st_build(const DMesh& m, int* key, StElem* rec, int s_first, int
     R.s[0] = r0.w;
     R.s[1] = r1.x;
     R.s[2] = r1.y;
-    R.area = m.area[e];
     R.ekb = m.elem_kb[e];
   }
   __syncthreads();
