@@ -517,19 +517,29 @@ static void solver_roll(gsh_solver* s) {
 // ---------------------------------------------------------------------- PCG driver
 // Whole-solve launches wait for their own workgroups, so those of all streams together must fit the
 // device: the solves of this process hold slots of it while they run, and a solve that gets none
-// takes the launches per phase. (Other processes are not counted; see the launches' bounded wait.)
+// takes the launches per phase. A workgroup (up to 1,024 threads, 66 KB of LDS) fits an empty CU, so
+// with as many slots as the device has CUs (a partition fewer than a whole chip) there is always a
+// CU for the next one. (Other processes are not counted; see the launches' bounded wait.)
 struct RunSlots {
-  static constexpr int kSlots = 256;  // workgroups of up to 1,024 threads resident on any device here
   static std::atomic<int>& used(int device) {
     static std::atomic<int> u[64];
     return u[device & 63];
+  }
+  static int slots(int device) {
+    static std::atomic<int> cus[64];
+    int c = cus[device & 63];
+    if (c == 0) {
+      if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
+      cus[device & 63] = c;
+    }
+    return c;
   }
   std::atomic<int>* u = nullptr;
   int n = 0;
   RunSlots(int device, int wgs) {
     if (wgs <= 0) return;
     std::atomic<int>& a = used(device);
-    if (a.fetch_add(wgs) + wgs > kSlots) {
+    if (a.fetch_add(wgs) + wgs > slots(device)) {
       a.fetch_sub(wgs);
       return;
     }
