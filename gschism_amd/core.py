@@ -369,6 +369,17 @@ class Solver:
     def set_graphs(self, on: bool) -> None:
         check(L.lib().gsh_solver_set_graphs(self.h, 1 if on else 0))
 
+    def set_one_launch(self, polls: int = -1, epoch: int = 0) -> None:
+        """The bound on the waits of one-launch solves (-1: default, 0: every wait gives up at once) and,
+        where > 0, their exchange counter; ends a stay on the phases after a launch that gave up."""
+        check(L.lib().gsh_solver_set_one_launch(self.h, polls, epoch))
+
+    def one_launch_info(self) -> tuple[int, int]:
+        """(solves that ran whole in a launch, solves that a launch gave up and the phases solved)"""
+        whole, gave_up = C.c_int32(), C.c_int32()
+        check(L.lib().gsh_solver_one_launch_info(self.h, C.byref(whole), C.byref(gave_up)))
+        return whole.value, gave_up.value
+
     def set_omega(self, omega: float) -> None:
         check(L.lib().gsh_solver_set_omega(self.h, omega))
 

@@ -245,6 +245,9 @@ struct gsh_solver {
   uint64_t* run_words = nullptr;
   uint32_t run_epoch = 1;
   int32_t max_row = 0, band = 0;
+  // their bounded wait; solves still kept on the phases after a launch that gave up, and how many the
+  // last one meant; solves that ran whole, and that gave up and took the phases
+  int32_t run_polls = kRunPolls, run_skip = 0, run_backoff = 0, run_whole = 0, run_gave_up = 0;
   // mixed precision
   float* val32 = nullptr;
   double* r64 = nullptr;
@@ -622,6 +625,13 @@ struct PhaseTimes {
 // single system whose pattern was counted on the host (its small systems run whole in a launch).
 constexpr int kRunIters = 512;  // iterations of a launch at most (milliseconds, so time limits hold)
 constexpr uint32_t kRunEpochs = 0xffff0000u;  // last first epoch of a launch before the words are cleared
+constexpr int kRunBackoff = 16, kRunBackoffMax = 1024;  // solves on the phases after the first and further give-ups
+
+static void clear_run_words(gsh_solver* s, uint32_t epoch) {
+  hipLaunchKernelGGL(k_fill_words, dim3((kRunWords + 255) / 256), dim3(256), 0, s->ctx->stream, s->run_words, kRunWords);
+  s->run_epoch = epoch;
+}
+
 template <class VT>
 static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const TileRef* dtiles, int ntiles, int rpt,
                          double rtol, int maxiter, int check_every, double timeout_s, PcgState* dgather,
@@ -638,18 +648,18 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
   else
     launch_pcg_init<VT>(dsys, dtiles, ntiles, rpt, st);
   HIPCHK(hipGetLastError());
-  const bool fits = solo && !prof && !(graph && graph->enabled) && pcg_run_fits(ntiles, rpt, solo->max_row, solo->band);
+  bool fits = solo && !prof && !(graph && graph->enabled) && pcg_run_fits(ntiles, rpt, solo->max_row, solo->band);
+  if (fits && solo->run_skip > 0) {
+    --solo->run_skip;
+    fits = false;
+  }
   if (const RunSlots held(ctx->device, fits ? ntiles : 0); held) {
     // a small system: hundreds of iterations per launch, which stops itself at the passing test
     const auto t0 = Clock::now();
     for (int issued = 0;;) {
       const int w = std::min(kRunIters, maxiter - issued);
-      if (solo->run_epoch > kRunEpochs) {  // the words start again at epoch 0, as when they were allocated
-        hipLaunchKernelGGL(k_fill_words, dim3((kRunWords + 255) / 256), dim3(256), 0, st, solo->run_words,
-                           kRunWords);
-        solo->run_epoch = 1;
-      }
-      launch_pcg_run<VT>(dsys, ntiles, rpt, solo->run_words, solo->run_epoch, solo->band, w, st);
+      if (solo->run_epoch > kRunEpochs) clear_run_words(solo, 1);  // as when they were allocated
+      launch_pcg_run<VT>(dsys, ntiles, rpt, solo->run_words, solo->run_epoch, solo->band, w, solo->run_polls, st);
       solo->run_epoch += (uint32_t)w + 1;
       issued += w;
       launch_pcg_finish<VT>(dsys, dtiles, ntiles, rpt, st);
@@ -658,11 +668,20 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
       HIPCHK(hipEventRecord(ctx->ev[0], st));
       HIPCHK(hipGetLastError());
       wait_event(ctx->ev[0], timeout_s, "PCG launch");
-      if (slots[0].pad0) break;  // its workgroups did not meet: the phases solve it, from the start
-      if (slots[0].done >= 0 || issued >= maxiter) return;
+      if (slots[0].gave_up) break;  // its workgroups did not meet: the phases solve it, from the start
+      if (slots[0].done >= 0 || issued >= maxiter) {
+        solo->run_backoff = 0;
+        ++solo->run_whole;
+        return;
+      }
       if (std::chrono::duration<double>(Clock::now() - t0).count() > timeout_s)
         throw Error(GSH_E_TIMEOUT, "PCG: time limit exceeded while issuing iterations");
     }
+    // whatever kept them apart may last: each give-up costs its waits, so the next solves go straight
+    // to the phases, twice as many after every further one
+    ++solo->run_gave_up;
+    solo->run_backoff = std::min(kRunBackoffMax, std::max(kRunBackoff, 2 * solo->run_backoff));
+    solo->run_skip = solo->run_backoff;
     launch_pcg_reset<VT>(dsys, nsys, rtol, maxiter, check_every, st, rtols_dev);
     launch_pcg_init<VT>(dsys, dtiles, ntiles, rpt, st);
   }
@@ -2105,6 +2124,27 @@ int gsh_solver_set_graphs(gsh_solver* s, int on) {
       g->failed = false;
       g->enabled = on != 0;
     }
+  })
+}
+
+int gsh_solver_set_one_launch(gsh_solver* s, int polls, uint32_t epoch) {
+  GSH_API_BODY({
+    GSH_REQUIRE(s, GSH_E_ARG, "solver is NULL");
+    s->ctx->set();
+    s->run_polls = polls < 0 ? kRunPolls : polls;
+    s->run_skip = s->run_backoff = 0;
+    if (epoch > 0) {
+      clear_run_words(s, std::min(epoch, kRunEpochs));
+      HIPCHK(hipGetLastError());
+    }
+  })
+}
+
+int gsh_solver_one_launch_info(gsh_solver* s, int32_t* whole, int32_t* gave_up) {
+  GSH_API_BODY({
+    GSH_REQUIRE(s && whole && gave_up, GSH_E_ARG, "NULL argument");
+    *whole = s->run_whole;
+    *gave_up = s->run_gave_up;
   })
 }
 

@@ -106,7 +106,7 @@ struct StepArgs {
 struct PcgState {
   int32_t k, kk, done, zero;
   int32_t maxiter, check_every;
-  int32_t pad0;     // set when a whole-solve launch gave up waiting for its other workgroups
+  int32_t gave_up;  // set when a whole-solve launch gave up waiting for its other workgroups
   int32_t pad1;
   double rtol, atol2, rr_last, bb;
   double rho[2];    // r.z used by iteration k (slot k & 1)
@@ -242,14 +242,16 @@ void launch_pcg_phase(int which, const PcgSys<VT>* sys, const TileRef* tiles, in
                       hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // Up to `iters` iterations of one system in one launch, for systems that pcg_run_fits accepts: max_row,
 // the longest row; band, the largest |column - row|. words: kRunWords exchange words, zero at first;
-// epoch: above iters plus that of every earlier launch on these words, so at least 1.
+// epoch: above iters plus that of every earlier launch on these words, so at least 1. polls: the bound
+// of a workgroup's wait for the others (kRunPolls; 0: every workgroup gives up at its first wait).
 constexpr int kRunTiles = 128;                   // tiles at most
 constexpr int kRunRows = 4 * kTpb * kRunTiles;   // rows at most
 constexpr int kRunWords = 6 * kRunTiles;
+constexpr int kRunPolls = 1 << 16;               // tens of milliseconds
 bool pcg_run_fits(int ntiles, int rpt, int max_row, int band);
 template <class VT>
 void launch_pcg_run(const PcgSys<VT>* sys, int ntiles, int rpt, uint64_t* words, uint32_t epoch, int band, int iters,
-                    hipStream_t s);
+                    int polls, hipStream_t s);
 template <class VT>
 void launch_pcg_check(const PcgSys<VT>* sys, int nsys, hipStream_t s);
 template <class VT>

@@ -95,7 +95,7 @@ __global__ void k_pcg_reset(const PcgSys<VT>* sys, int nsys, double rtol, int ma
   st->bb = 0.0;
   st->rho[0] = 0.0;
   st->rho[1] = 0.0;
-  st->pad0 = 0;
+  st->gave_up = 0;
 }
 
 // ------------------------------------------------------------------ CSR row sums (block staged)
@@ -498,9 +498,9 @@ __global__ void __launch_bounds__(W ? kTpb * R : kTpb) k_pcg_phase_b(const PcgSy
 // 384 rows (one workgroup, no exchange) 4.2 against 12.4 with the solve's set-up, 16,000 rows 6.1
 // against 15.1, 66,887 rows 6.6 against 14.8, 128,000 rows 7.0 against 17. Up to kRunTiles
 // workgroups: an exchange takes 1.2 us among 32, 2.3 among 128, and at one workgroup of 1,024 threads
-// per CU two such launches are resident together (the host admits no more, RunSlots). A launch whose
-// workgroups do not become resident together all the same (another process's solve) gives up after
-// kRunSpin polls and leaves the solve to the phases.
+// per CU two such launches are resident together on 256 CUs (the host admits no more than a workgroup
+// a CU, RunSlots). A launch whose workgroups do not become resident together all the same (another
+// process's solve) gives up after `polls` polls and leaves the solve to the phases.
 constexpr int kRunRow = 12;     // entries of a row held in registers
 constexpr int kRunWin = 6144;   // p of the tile and its halo, words of LDS
 
@@ -548,7 +548,8 @@ __device__ __forceinline__ void run_totals(double (&v)[N], double* red) {
 // Publishes this tile's N partials (v, the same in every thread) and returns in v of thread t < T
 // tile t's, 0 in the others. False in a thread that gave up.
 template <int N>
-__device__ __forceinline__ bool run_exchange(double (&v)[N], gptr<uint64_t> words, int tile, int T, uint32_t epoch) {
+__device__ __forceinline__ bool run_exchange(double (&v)[N], gptr<uint64_t> words, int tile, int T, uint32_t epoch,
+                                             int polls) {
   const int tid = threadIdx.x;
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   if (tid < 2 * N) {
@@ -560,18 +561,18 @@ __device__ __forceinline__ bool run_exchange(double (&v)[N], gptr<uint64_t> word
   }
   bool ok = true;
   if (tid < T) {
-    uint64_t u[2 * N];
-    for (int spin = 0;;) {
+    uint64_t u[2 * N] = {};
+    for (int spin = 0;; ++spin) {
+      if (spin == polls) {
+        ok = false;
+        break;
+      }
 #pragma unroll
       for (int a = 0; a < 2 * N; ++a) u[a] = ld_agent((gptr<const uint64_t>)words + (int64_t)tid * 2 * N + a);
       bool all = true;
 #pragma unroll
       for (int a = 0; a < 2 * N; ++a) all = all && (uint32_t)(u[a] >> 32) == epoch;
       if (all) break;
-      if (++spin == kRunSpin) {
-        ok = false;
-        break;
-      }
     }
 #pragma unroll
     for (int a = 0; a < N; ++a) v[a] = run_value(u[2 * a], u[2 * a + 1]);
@@ -584,10 +585,10 @@ __device__ __forceinline__ bool run_exchange(double (&v)[N], gptr<uint64_t> word
 }
 
 // words: 6 x 128 exchange words of the solver; epoch0: the launch's first epoch, above every earlier
-// launch's; band: the largest |column - row|; iters: iterations at most.
+// launch's; band: the largest |column - row|; iters: iterations at most; polls: run_exchange's bound.
 template <class VT, int R, bool SOLO>
 __global__ void __launch_bounds__(kTpb * R) k_pcg_run(const PcgSys<VT>* __restrict__ sys, uint64_t* __restrict__ words_,
-                                                      uint32_t epoch0, int band, int iters) {
+                                                      uint32_t epoch0, int band, int iters, int polls) {
   constexpr int kRows = kTpb * R;
   __shared__ double red[8], redt[8], rows[2 * kRows];
   __shared__ int stuck;
@@ -696,7 +697,7 @@ __global__ void __launch_bounds__(kTpb * R) k_pcg_run(const PcgSys<VT>* __restri
     double t1[1] = {in ? (double)p * (double)q : 0.0};
     run_tile_sums<R>(t1, rows, red, false);
     if (!SOLO) {
-      if (!run_exchange(t1, wpq, tile, T, epoch)) stuck = 1;
+      if (!run_exchange(t1, wpq, tile, T, epoch, polls)) stuck = 1;
     } else if (tid != 0) {
       t1[0] = 0.0;
     }
@@ -716,7 +717,7 @@ __global__ void __launch_bounds__(kTpb * R) k_pcg_run(const PcgSys<VT>* __restri
     run_tile_sums<R>(t2, rows, red, !SOLO);
     double s2[2] = {t2[0], t2[1]};
     if (!SOLO) {
-      if (!run_exchange(s2, wrr, tile, T, epoch)) stuck = 1;
+      if (!run_exchange(s2, wrr, tile, T, epoch, polls)) stuck = 1;
     } else if (tid != 0) {
       s2[0] = s2[1] = 0.0;
     }
@@ -735,7 +736,7 @@ __global__ void __launch_bounds__(kTpb * R) k_pcg_run(const PcgSys<VT>* __restri
     }
   }
   if (!SOLO && stuck) {
-    if (tid == 0) st->pad0 = 1;
+    if (tid == 0) st->gave_up = 1;
     return;
   }
   if (in) {
@@ -1008,14 +1009,15 @@ bool pcg_run_fits(int ntiles, int rpt, int max_row, int band) {
 
 template <class VT>
 void launch_pcg_run(const PcgSys<VT>* sys, int ntiles, int rpt, uint64_t* words, uint32_t epoch, int band, int iters,
-                    hipStream_t s) {
+                    int polls, hipStream_t s) {
   with_rpt(rpt, [&](auto r) {
     constexpr int R = decltype(r)::value;
     if constexpr (R <= 4) {
       if (ntiles == 1)
-        launch_stamped(k_pcg_run<VT, R, true>, 1, kTpb * R, s, nullptr, nullptr, sys, words, epoch, band, iters);
+        launch_stamped(k_pcg_run<VT, R, true>, 1, kTpb * R, s, nullptr, nullptr, sys, words, epoch, band, iters, polls);
       else
-        launch_stamped(k_pcg_run<VT, R, false>, ntiles, kTpb * R, s, nullptr, nullptr, sys, words, epoch, band, iters);
+        launch_stamped(k_pcg_run<VT, R, false>, ntiles, kTpb * R, s, nullptr, nullptr, sys, words, epoch, band, iters,
+                       polls);
     }
   });
 }
@@ -1042,8 +1044,8 @@ template void launch_pcg_phase<double>(int, const PcgSys<double>*, const TileRef
                                        hipEvent_t);
 template void launch_pcg_phase<float>(int, const PcgSys<float>*, const TileRef*, int, int, hipStream_t, hipEvent_t,
                                        hipEvent_t);
-template void launch_pcg_run<double>(const PcgSys<double>*, int, int, uint64_t*, uint32_t, int, int, hipStream_t);
-template void launch_pcg_run<float>(const PcgSys<float>*, int, int, uint64_t*, uint32_t, int, int, hipStream_t);
+template void launch_pcg_run<double>(const PcgSys<double>*, int, int, uint64_t*, uint32_t, int, int, int, hipStream_t);
+template void launch_pcg_run<float>(const PcgSys<float>*, int, int, uint64_t*, uint32_t, int, int, int, hipStream_t);
 template void launch_pcg_check<double>(const PcgSys<double>*, int, hipStream_t);
 template void launch_pcg_check<float>(const PcgSys<float>*, int, hipStream_t);
 template void launch_pcg_finish<double>(const PcgSys<double>*, const TileRef*, int, int, hipStream_t);

@@ -109,7 +109,6 @@ __device__ __forceinline__ void wait_stores() {
   __builtin_amdgcn_s_waitcnt(0);
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
-constexpr int kRunSpin = 1 << 16;  // polls before a workgroup gives up on the others (tens of milliseconds)
 
 // A double as two 64-bit words of (epoch, 32 bits): each word is whole in itself, so a reader knows
 // from the epochs when it has the value.

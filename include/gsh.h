@@ -356,6 +356,16 @@ int gsh_solver_autotune(gsh_solver* s, int iters, int* best_rpt, double* us_per_
 /* No counterpart in the reference: on != 0 captures each solve window (check_every iterations
  * and the window-end test) of this solver into a HIP graph once and replays it; default off. */
 int gsh_solver_set_graphs(gsh_solver* s, int on);
+/* No counterpart in the reference: small Jacobi systems are solved whole in one launch, whose
+ * workgroups wait for each other up to `polls` polls each and otherwise leave the solve to the launches
+ * per phase, which give the same bits. polls < 0 sets the default bound; with 0 every launch that waits
+ * gives up at once. A launch that gave up keeps the solver's next solves (16, doubling up to 1024) on
+ * the phases; this call ends that. epoch > 0 also restarts the exchange's counter there (at most
+ * 0xffff0000, from where it starts again at 1). */
+int gsh_solver_set_one_launch(gsh_solver* s, int polls, uint32_t epoch);
+/* Solves (inner solves of MIXED) of this solver that ran whole in a launch, and those of which a launch
+ * gave up and that the phases solved. */
+int gsh_solver_one_launch_info(gsh_solver* s, int32_t* whole, int32_t* gave_up);
 /* SSOR relaxation factor omega in (0, 2), default 1 (symmetric Gauss-Seidel). */
 int gsh_solver_set_omega(gsh_solver* s, double omega);
 /* SSOR layout: number of colours, rows after padding every colour block to whole reduction

@@ -664,6 +664,20 @@ def test_step_call_argument_errors(ctx):
     mesh.close()
 
 
+def _banded(ctx, n, offsets, rpt, precision=L.PREC_FP64):
+    """A solver on a diagonally dominant matrix with the given diagonals, and (indptr, columns, values)."""
+    rows = np.repeat(np.arange(n), len(offsets))
+    cols = rows + np.tile(offsets, n)
+    on = (cols >= 0) & (cols < n)
+    rows, cols = rows[on], cols[on].astype(np.int32)
+    ip = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    val = np.where(rows == cols, len(offsets) - 0.5, -1.0)
+    s = core.Solver(None, precision, ctx=ctx, indptr=ip, indices=cols)
+    s.set_tuning(rpt)
+    s.set_values(val)
+    return s, (ip, cols, val)
+
+
 @pytest.mark.parametrize("rpt", [2, 4])
 @pytest.mark.parametrize("half", [4, 5])
 def test_wide_phases_and_long_chunks(ctx, rpt, half):
@@ -680,10 +694,26 @@ def test_wide_phases_and_long_chunks(ctx, rpt, half):
     s = core.Solver(None, ctx=ctx, indptr=ip, indices=cols)
     s.set_tuning(rpt)
     s.set_values(val)
+    s.set_one_launch(polls=0)  # so few tiles would run whole in a launch: its waits give up, the phases solve
     x, it, st = s.solve(b, rtol=1e-12, maxiter=500, check_every=10)
+    assert s.one_launch_info() == (0, 1)
     xo, ito, _, _ = O.pcg(ip, cols, val, b, rtol=1e-12, maxiter=500, check_every=10, rows_per_thread=rpt)
     assert st == 0 and it == ito
     assert_bitwise(x, xo, f"banded solve, half width {half}, {rpt} rows per thread")
+    s.close()
+
+
+@pytest.mark.parametrize("rpt,n", [(4, 129 * 1024 + 5), (2, 300 * 512 + 131), (4, 512 * 1024 - 1), (4, 512 * 1024 + 1)])
+def test_wide_phases_above_one_launch(ctx, rpt, n):
+    """129 to 512 tiles, which run the wide phases, and one tile more, which runs the narrow ones."""
+    s, sys = _banded(ctx, n, [-300, -1, 0, 1, 300], rpt)
+    b = cases.normal(43, n)
+    print(f"[gpu] phases, n={n}, {rpt} rows per thread", flush=True)
+    x, it, _ = s.solve(b, rtol=1e-300, maxiter=30, check_every=10)
+    assert s.one_launch_info() == (0, 0)
+    xo, ito, _, _ = O.pcg(*sys, b, rtol=1e-300, maxiter=30, check_every=10, rows_per_thread=rpt, nthreads=8)
+    assert it == ito
+    assert_bitwise(x, xo, f"{n} rows, {rpt} rows per thread")
     s.close()
 
 
@@ -712,6 +742,93 @@ def test_small_systems_in_one_launch(ctx, rpt, n, maxiter):
         assert it == ito
         assert_bitwise(x, xo, f"solution {rep}")
         hist = [xo] + hist[:2]
+    assert s.one_launch_info() == (2 if n <= 131072 else 0, 0)
+    s.close()
+
+
+@pytest.mark.parametrize("rpt,n,offsets,whole", [
+    (4, 9 * 1024 + 3, [-2560, -1, 0, 1, 2560], True),    # the widest window of p: 1024 + 2 * 2560 = 6144
+    (4, 9 * 1024 + 3, [-2561, -1, 0, 1, 2561], False),
+    (1, 33 * 256 - 7, [-700, -1, 0, 1, 700], True),      # a halo of more rows than four strides of the threads
+    (2, 12 * 512 + 1, list(range(-5, 7)), True),         # 12 entries a row, the most kept in registers
+    (2, 12 * 512 + 1, list(range(-6, 7)), False)])
+def test_one_launch_limits(ctx, rpt, n, offsets, whole):
+    """The widest window, the longest halo and rows that run whole in a launch, and one past them."""
+    s, sys = _banded(ctx, n, offsets, rpt)
+    b = cases.normal(44, n)
+    print(f"[gpu] one-launch limits, n={n}, {rpt} rows per thread, {len(offsets)} diagonals", flush=True)
+    x, it, _ = s.solve(b, rtol=1e-300, maxiter=30, check_every=10)
+    assert s.one_launch_info() == (int(whole), 0)
+    xo, ito, _, _ = O.pcg(*sys, b, rtol=1e-300, maxiter=30, check_every=10, rows_per_thread=rpt)
+    assert it == ito
+    assert_bitwise(x, xo, f"{n} rows, diagonals {offsets[0]} to {offsets[-1]}")
+    s.close()
+
+
+@pytest.mark.parametrize("polls", [0, 1, 3, 20])
+def test_one_launch_gives_up(ctx, polls):
+    """Waits so short that workgroups give up, all at once or some of them in the middle of a solve,
+    while others go on with sums that are none: the phases solve from the start, with the history, bit
+    for bit; the next solves stay on them, and the same exchange words serve the launches after that."""
+    n = 20 * 1024 + 11
+    s, sys = _banded(ctx, n, [-37, -1, 0, 1, 37], 4)
+    s.set_one_launch(polls=polls)
+    hist = [np.zeros(n)] * 3
+    print(f"[gpu] one-launch solve with waits of {polls} polls", flush=True)
+    for rep in range(5):
+        if rep == 3:
+            s.set_one_launch()
+        before = s.one_launch_info()
+        b = cases.normal(80 + rep, n)
+        x, it, _ = s.solve(b, rtol=1e-12, maxiter=400, check_every=10)
+        whole, gave_up = s.one_launch_info()
+        xo, ito, _, _ = O.pcg(*sys, b, hist=hist, rtol=1e-12, maxiter=400, check_every=10, rows_per_thread=4, nthreads=8)
+        assert it == ito
+        assert_bitwise(x, xo, f"solution {rep} with waits of {polls} polls")
+        hist = [xo] + hist[:2]
+        if rep >= 3:
+            assert (whole, gave_up) == (before[0] + 1, before[1])
+        elif before[1] > 0:
+            assert (whole, gave_up) == before  # kept on the phases
+        elif polls == 0:
+            assert (whole, gave_up) == (0, 1)
+    s.close()
+
+
+@pytest.mark.parametrize("rpt", [1, 2, 4])
+def test_one_launch_mixed_equals_the_phases(ctx, rpt):
+    """Mixed precision: inner FP32 solves whole in a launch against the same solver whose first launch
+    gives up, so that the phases solve this one and the ones after it. Bit for bit, twice."""
+    n = 11 * 1024 + 100
+    out = []
+    for polls in (-1, 0):
+        s, _ = _banded(ctx, n, [-90, -1, 0, 1, 90], rpt, L.PREC_MIXED)
+        s.set_one_launch(polls=polls)
+        print(f"[gpu] mixed solve, {rpt} rows per thread, polls {polls}", flush=True)
+        out.append([s.solve(cases.normal(90 + rep, n), rtol=1e-11, maxiter=400, check_every=10) for rep in range(2)])
+        whole, gave_up = s.one_launch_info()
+        assert (whole > 1, gave_up) == ((True, 0) if polls else (False, 1))
+        s.close()
+    for (x, it, st), (xp, itp, stp) in zip(*out):
+        assert (it, st) == (itp, stp)
+        assert_bitwise(x, xp, "mixed solution")
+
+
+@pytest.mark.parametrize("epoch", [0xFFFEFFFF, 0xFFFF0000])
+def test_one_launch_counter_starts_again(ctx, epoch):
+    """Solves around the end of the exchange's 32-bit counter, where its words are cleared."""
+    n = 6 * 1024 + 1
+    s, sys = _banded(ctx, n, [-37, -1, 0, 1, 37], 4)
+    s.set_one_launch(epoch=epoch)
+    print(f"[gpu] one-launch solves from counter {epoch:#x}", flush=True)
+    for rep in range(4):
+        b = cases.normal(95 + rep, n)
+        s.reset_history()
+        x, it, _ = s.solve(b, rtol=1e-300, maxiter=60, check_every=10)
+        xo, ito, _, _ = O.pcg(*sys, b, rtol=1e-300, maxiter=60, check_every=10, rows_per_thread=4)
+        assert it == ito
+        assert_bitwise(x, xo, f"solution {rep}")
+    assert s.one_launch_info() == (4, 0)
     s.close()
 
 
