@@ -613,7 +613,8 @@ struct WindowPacer {
 
 // Runs the PCG iteration for nsys systems described by dsys (device) over the tile table
 // dtiles. Each system stops at its own first check with r.r <= atol^2 (pcg_loop.cpp:405-412).
-// Per-phase launch timing collected with HIP events on the solver stream.
+// Per-phase launch timing collected with HIP events on the solver stream; launches counts iterations,
+// and a one-launch solve's time goes to ms_a.
 struct PhaseTimes {
   double ms_a = 0.0, ms_b = 0.0;
   int64_t launches = 0;
@@ -626,6 +627,27 @@ struct PhaseTimes {
 constexpr int kRunIters = 512;  // iterations of a launch at most (milliseconds, so time limits hold)
 constexpr uint32_t kRunEpochs = 0xffff0000u;  // last first epoch of a launch before the words are cleared
 constexpr int kRunBackoff = 16, kRunBackoffMax = 1024;  // solves on the phases after the first and further give-ups
+
+// A kernel's start and end events for the launchers that stamp them; none (NULL) when off.
+struct Stamps {
+  hipEvent_t e[2] = {nullptr, nullptr};
+  explicit Stamps(bool on) {
+    if (!on) return;
+    for (auto& x : e) HIPCHK(hipEventCreate(&x));
+  }
+  double ms() const {
+    float t = 0.f;
+    HIPCHK(hipEventSynchronize(e[1]));
+    HIPCHK(hipEventElapsedTime(&t, e[0], e[1]));
+    return t;
+  }
+  ~Stamps() {
+    for (auto& x : e)
+      if (x) (void)hipEventDestroy(x);
+  }
+  Stamps(const Stamps&) = delete;
+  Stamps& operator=(const Stamps&) = delete;
+};
 
 static void clear_run_words(gsh_solver* s, uint32_t epoch) {
   hipLaunchKernelGGL(k_fill_words, dim3((kRunWords + 255) / 256), dim3(256), 0, s->ctx->stream, s->run_words, kRunWords);
@@ -648,7 +670,7 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
   else
     launch_pcg_init<VT>(dsys, dtiles, ntiles, rpt, st);
   HIPCHK(hipGetLastError());
-  bool fits = solo && !prof && !(graph && graph->enabled) && pcg_run_fits(ntiles, rpt, solo->max_row, solo->band);
+  bool fits = solo && !(graph && graph->enabled) && pcg_run_fits(ntiles, rpt, solo->max_row, solo->band);
   if (fits && solo->run_skip > 0) {
     --solo->run_skip;
     fits = false;
@@ -659,7 +681,9 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
     for (int issued = 0;;) {
       const int w = std::min(kRunIters, maxiter - issued);
       if (solo->run_epoch > kRunEpochs) clear_run_words(solo, 1);  // as when they were allocated
-      launch_pcg_run<VT>(dsys, ntiles, rpt, solo->run_words, solo->run_epoch, solo->band, w, solo->run_polls, st);
+      Stamps stamps(prof != nullptr);
+      launch_pcg_run<VT>(dsys, ntiles, rpt, solo->run_words, solo->run_epoch, solo->band, w, solo->run_polls, st,
+                         stamps.e[0], stamps.e[1]);
       solo->run_epoch += (uint32_t)w + 1;
       issued += w;
       launch_pcg_finish<VT>(dsys, dtiles, ntiles, rpt, st);
@@ -669,6 +693,10 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
       HIPCHK(hipGetLastError());
       wait_event(ctx->ev[0], timeout_s, "PCG launch");
       if (slots[0].gave_up) break;  // its workgroups did not meet: the phases solve it, from the start
+      if (prof) {
+        prof->ms_a += stamps.ms();
+        prof->launches += w;
+      }
       if (slots[0].done >= 0 || issued >= maxiter) {
         solo->run_backoff = 0;
         ++solo->run_whole;
@@ -2092,10 +2120,20 @@ int gsh_solver_autotune(gsh_solver* s, int iters, int* best_rpt, double* us_per_
         }
         us = tt.iters ? 1e3 * (tt.ms_bwd + tt.ms_fwd + tt.ms_upd) / tt.iters : 1e300;
       } else {
+        // the launches that a solve of this tile size takes: whole in one where it fits, in the precision
+        // of the solver's iterations
         solver_sync_desc(s);
         PcgOutcome o;
         PhaseTimes pt;
-        run_pcg<double>(s->ctx, s->ds, 1, s->dtiles, s->ntiles, r, 1e-300, iters, iters, 60.0, o, nullptr, -1, &pt);
+        if (s->precision == GSH_PREC_MIXED) {
+          launch_cast_values(s->val, s->val32, s->nnz, st);
+          launch_copy_f64(s->r64, s->b, s->n, st);
+          run_pcg<float>(s->ctx, s->ds32, 1, s->dtiles, s->ntiles, r, 1e-300, iters, iters, 60.0, o, nullptr, -1, &pt,
+                         nullptr, nullptr, s);
+        } else {
+          run_pcg<double>(s->ctx, s->ds, 1, s->dtiles, s->ntiles, r, 1e-300, iters, iters, 60.0, o, nullptr, -1, &pt,
+                          nullptr, &s->wg_jacobi, s);
+        }
         us = pt.launches ? 1e3 * (pt.ms_a + pt.ms_b) / pt.launches : 1e300;
       }
       if (us_per_iter) us_per_iter[c] = us;

@@ -251,7 +251,7 @@ constexpr int kRunPolls = 1 << 16;               // tens of milliseconds
 bool pcg_run_fits(int ntiles, int rpt, int max_row, int band);
 template <class VT>
 void launch_pcg_run(const PcgSys<VT>* sys, int ntiles, int rpt, uint64_t* words, uint32_t epoch, int band, int iters,
-                    int polls, hipStream_t s);
+                    int polls, hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 template <class VT>
 void launch_pcg_check(const PcgSys<VT>* sys, int nsys, hipStream_t s);
 template <class VT>

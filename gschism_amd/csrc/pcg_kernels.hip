@@ -1009,15 +1009,14 @@ bool pcg_run_fits(int ntiles, int rpt, int max_row, int band) {
 
 template <class VT>
 void launch_pcg_run(const PcgSys<VT>* sys, int ntiles, int rpt, uint64_t* words, uint32_t epoch, int band, int iters,
-                    int polls, hipStream_t s) {
+                    int polls, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
   with_rpt(rpt, [&](auto r) {
     constexpr int R = decltype(r)::value;
     if constexpr (R <= 4) {
       if (ntiles == 1)
-        launch_stamped(k_pcg_run<VT, R, true>, 1, kTpb * R, s, nullptr, nullptr, sys, words, epoch, band, iters, polls);
+        launch_stamped(k_pcg_run<VT, R, true>, 1, kTpb * R, s, e0, e1, sys, words, epoch, band, iters, polls);
       else
-        launch_stamped(k_pcg_run<VT, R, false>, ntiles, kTpb * R, s, nullptr, nullptr, sys, words, epoch, band, iters,
-                       polls);
+        launch_stamped(k_pcg_run<VT, R, false>, ntiles, kTpb * R, s, e0, e1, sys, words, epoch, band, iters, polls);
     }
   });
 }
@@ -1044,8 +1043,10 @@ template void launch_pcg_phase<double>(int, const PcgSys<double>*, const TileRef
                                        hipEvent_t);
 template void launch_pcg_phase<float>(int, const PcgSys<float>*, const TileRef*, int, int, hipStream_t, hipEvent_t,
                                        hipEvent_t);
-template void launch_pcg_run<double>(const PcgSys<double>*, int, int, uint64_t*, uint32_t, int, int, int, hipStream_t);
-template void launch_pcg_run<float>(const PcgSys<float>*, int, int, uint64_t*, uint32_t, int, int, int, hipStream_t);
+template void launch_pcg_run<double>(const PcgSys<double>*, int, int, uint64_t*, uint32_t, int, int, int, hipStream_t, hipEvent_t,
+                                     hipEvent_t);
+template void launch_pcg_run<float>(const PcgSys<float>*, int, int, uint64_t*, uint32_t, int, int, int, hipStream_t, hipEvent_t,
+                                    hipEvent_t);
 template void launch_pcg_check<double>(const PcgSys<double>*, int, hipStream_t);
 template void launch_pcg_check<float>(const PcgSys<float>*, int, hipStream_t);
 template void launch_pcg_finish<double>(const PcgSys<double>*, const TileRef*, int, int, hipStream_t);

@@ -348,8 +348,9 @@ int gsh_solver_last_stats(gsh_solver* s, gsh_solve_stats* out);
 /* Tuning knobs: rows per thread of the PCG tiles (1, 2, 4, 8) and the inner tolerance of the
  * mixed-precision refinement. */
 int gsh_solver_set_tuning(gsh_solver* s, int rows_per_thread, double inner_rtol);
-/* Autotuner (no counterpart in the reference): times `iters` FP64 iterations on the solver's
- * current system for rows_per_thread 1, 2, 4 and 8 (kernel-stamped events) and keeps the fastest;
+/* Autotuner (no counterpart in the reference): times `iters` iterations on the solver's current
+ * system, as its solves run them (FP32 for MIXED, whole in one launch where the system fits one), for
+ * rows_per_thread 1, 2, 4 and 8 (kernel-stamped events) and keeps the fastest;
  * us_per_iter[4] (may be NULL) receives the measured microseconds per iteration. The solution
  * buffer is overwritten, the history of previous solutions is kept. */
 int gsh_solver_autotune(gsh_solver* s, int iters, int* best_rpt, double* us_per_iter);

@@ -814,6 +814,23 @@ def test_one_launch_mixed_equals_the_phases(ctx, rpt):
         assert_bitwise(x, xp, "mixed solution")
 
 
+@pytest.mark.parametrize("precision", [L.PREC_FP64, L.PREC_MIXED])
+@pytest.mark.parametrize("n", [40000, 69000, 120000])
+def test_autotune_keeps_one_launch(ctx, precision, n):
+    """Systems that run whole in a launch at some tile sizes only (of 40,000 rows 512 or more, of 69,000
+    and 120,000 rows 1024): the autotuner times that path, several times faster than the phases, so the
+    solves that follow take it."""
+    s, _ = _banded(ctx, n, [-200, -1, 0, 1, 200], 4, precision)
+    s.set_rhs(cases.normal(47, n))
+    best, us = s.autotune(30)
+    print(f"[gpu] autotune n={n}, precision {precision}: {best} rows per thread, us/iter {us}", flush=True)
+    assert best == 4 or (n == 40000 and best == 2)
+    before = s.one_launch_info()[0]
+    _, _, st = s.solve(None, rtol=1e-10, maxiter=400, check_every=10)
+    assert st == 0 and s.one_launch_info()[0] > before
+    s.close()
+
+
 @pytest.mark.parametrize("epoch", [0xFFFEFFFF, 0xFFFF0000])
 def test_one_launch_counter_starts_again(ctx, epoch):
     """Solves around the end of the exchange's 32-bit counter, where its words are cleared."""
