@@ -62,13 +62,14 @@ def backtrack_bound():
     """Per-launch FP64 operations, HBM bytes, VALU busy fraction and occupancy of k_backtrack on
     this workload, from the committed rocprofv3 counter summary (profiles/), or None. The summary
     holds one line 'bound k_backtrack fp64_ops_per_launch=<F> hbm_bytes_per_launch=<B>
-    valu_busy=<V> waves_per_simd=<W>'."""
+    valu_busy=<V> waves_per_simd=<W> vgprs=<R>'; the registers name the build that was counted
+    (tests/test_cpu_kernel_resources.py holds them against the sources)."""
     path = os.path.join(ROOT, "profiles", "backtrack_counters_channel-1024x1024.md")
     try:
         with open(path) as f:
             for line in f:
                 w = line.strip().strip("`").split()
-                if len(w) == 6 and w[0] == "bound" and w[1] == "k_backtrack":
+                if len(w) == 7 and w[0] == "bound" and w[1] == "k_backtrack":
                     return {k: float(v) for k, v in (x.split("=", 1) for x in w[2:])}
     except OSError:
         pass

@@ -1,5 +1,6 @@
 """What the compiler gives the kernels whose speed hangs on their occupancy, from its own
 kernel-resource-usage remarks on this library's sources (no GPU)."""
+import importlib.util
 import re
 import shutil
 import subprocess
@@ -21,7 +22,7 @@ def _usage(source, tmp_path):
         m = re.search(r"remark: +Function Name: (?:void )?(.*?)\(", line)
         if m:
             cur = out.setdefault(m.group(1), {})
-        m = re.search(r"remark: +(VGPRs|Occupancy|ScratchSize)[^:]*: (\d+)", line)
+        m = re.search(r"remark: +(VGPRs|Occupancy|ScratchSize)(?: \[[^\]]*\])?: (\d+)", line)
         if m and cur is not None:
             cur[m.group(1)] = int(m.group(2))
     return out
@@ -51,3 +52,15 @@ def test_momentum_of_few_levels_keeps_its_waves(tmp_path):
     for items, waves in ((2, 5), (4, 4), (8, 3), (16, 2)):
         k = u[f"gsh::k_momentum<{items}>"]
         assert k["Occupancy"] >= waves and k["ScratchSize"] == 0
+
+
+@needs_compiler
+def test_backtracking_counters_are_of_this_kernel(tmp_path):
+    """bench.py divides the committed counters of k_backtrack by its own time: they are of the kernel
+    that these sources build, at least as far as its registers tell."""
+    spec = importlib.util.spec_from_file_location("bench", build.CSRC.parents[1] / "bench.py")
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    bound = bench.backtrack_bound()
+    k = _usage("mesh_kernels.hip", tmp_path)["gsh::k_backtrack<0, false, true>"]
+    assert bound["vgprs"] == k["VGPRs"] and bound["waves_per_simd"] <= k["Occupancy"]
