@@ -431,36 +431,51 @@ __device__ __forceinline__ void z_bracket(const Z& z, double s0, double s1, doub
   }
 }
 
-// What the last interpolation of a start point read: the element, its area and reciprocal, and the
-// z and velocities of its nodes at the two levels of the vertical bracket. Most substeps stay in
-// their prism, and then read nothing: every operand is here, in the operations of the full search.
-// It takes 58 registers: three waves a SIMD instead of four (four spill: 16.8 ms against 7.5, two 9.8),
-// and 64 % of the time is VALU issue. 1,048,576 nodes x 31 levels 8.58 -> 7.48 ms (8.36 with only the
-// last interpolation spared), per-node sigma 417x263 841 -> 685 us.
+// What the last interpolation of a start point read: the element, the z of its nodes at the two levels
+// of the vertical bracket and the velocities there. A substep that stays in its prism reads nothing but
+// the element's area: every operand is here, in the operations of the full search.
+// LV: the velocities (36 registers' worth) lie in LDS and the area is read again, which leaves four waves
+// a SIMD; otherwise all of it is in registers, for three. With three waves the full search, which every
+// substep pays that enters a new element, was slower than without anything kept: 700x500 nodes x 31
+// levels, 15 s substeps of flows up to 1 m/s, ms without / kept in registers / kept with LV:
+//   one sigma, dx 1000 m 4.32 / 3.45 / 3.20, 50 m 5.82 / 6.80 / 5.98, 10 m 8.86 / 10.87 / 9.36
+//   per-node sigma       5.33 / 4.09 / 3.90        7.16 / 8.55 / 8.01       12.5 / 15.4 / 14.1
+// (before brackets were kept either: one sigma 5.17, 6.57, 9.60, per-node 9.52, 11.1, 14.7). 1,048,576
+// nodes x 31 levels 8.58 ms with nothing kept, 7.48 in registers (16.8 at four waves, which spill), 6.94 LV.
+constexpr int kCellVel = 18;  // (u, v, w) of nodes 0-2 at the lower level, then at the upper one
+template <bool LV>
 struct BtCell {
-  int e = -1;  // -1: none
-  int L = 0, R = 0;
-  bool kept = false;  // the bracket's values hold, and the column's levels do not decrease
-  double2 area;
-  double3 zL, zR;                      // per node
-  double3 u0, u1, u2, v0, v1, v2;      // (u, v, w) of nodes 0-2 at L, and at R
+  int e = -1;         // -1: none
+  int br = -1;        // the bracket's levels, (L + 1) << 10 | R (nvrt <= 1024); -1: not kept
+  double2 area;       // (LV: read each time)
+  double3 zL, zR;     // per node, where the column's levels do not decrease
+  double v[LV ? 1 : kCellVel];
+  double* lv;         // LV: the thread's column of LDS, kCellVel values 256 apart
+  __device__ __forceinline__ double get(int i) const { return LV ? lv[256 * i] : v[LV ? 0 : i]; }
+  __device__ __forceinline__ void put(int i, double x) {
+    if (LV)
+      lv[256 * i] = x;
+    else
+      v[LV ? 0 : i] = x;
+  }
 };
 
 // Element::interpolateVelocities for triangles, ics=1 (meshdata.cu:1209-1291) with
 // computeShapeCoords(fiAnywhere) (meshdata.cu:990-1043); g is element e's geometry.
 // hint: the lower level of the previous vertical bracket (updated here).
 // rc: element e's staged record (ST), else NULL.
-template <int VM, bool ST, bool F>
+template <int VM, bool ST, bool F, bool LV>
 __device__ void interp_velocity(const DMesh& m, const double* sig, double h0, int e, const ElemGeom& g,
-                                const StElem* rc, BtCell& c, double px, double py, double pz, double& uo, double& vo,
+                                const StElem* rc, BtCell<LV>& c, double px, double py, double pz, double& uo, double& vo,
                                 double& wo, int& hint) {
   const int n0 = g.n0, n1 = g.n1, n2 = g.n2;
   const double x0 = g.x0, y0 = g.y0, x1 = g.x1, y1 = g.y1, x2 = g.x2, y2 = g.y2;
-  if (c.e != e) {
+  const bool entered = c.e != e;
+  if (entered) {
     c.e = e;
-    c.kept = false;
-    c.area = m.area_inv[ux(e)];
+    c.br = -1;
   }
+  if (LV || entered) c.area = m.area_inv[ux(e)];
   const double a0 = signed_area(px, py, x1, y1, x2, y2), a1 = signed_area(x0, y0, px, py, x2, y2);
   double s0 = div_by(a0, c.area.x, c.area.y);
   double s1 = div_by(a1, c.area.x, c.area.y);
@@ -479,11 +494,11 @@ __device__ void interp_velocity(const DMesh& m, const double* sig, double h0, in
   const int R0 = nv - 1;
   double w1 = 1.0, w2 = 0.0;
   bool hit = false;
-  if (c.kept) {
+  if (c.br >= 0) {
     // the kept bracket: strictly inside two neighbouring levels, or the whole column (L0, R0) with the
     // point at or beyond an end: then z_bracket ends in it, with the same weights
     const double zL = s0 * c.zL.x + s1 * c.zL.y + s2 * c.zL.z + 0.0, zR = s0 * c.zR.x + s1 * c.zR.y + s2 * c.zR.z + 0.0;
-    const bool whole = c.R - c.L > 1;
+    const bool whole = (c.br & 1023) > (c.br >> 10);  // R - L > 1
     if (!whole) {
       hit = zL < pz && pz < zR;
       if (hit) {
@@ -500,13 +515,13 @@ __device__ void interp_velocity(const DMesh& m, const double* sig, double h0, in
   }
   if (!hit) {
     int L, R, kb0, kb1, kb2;
+    bool mono = true;
     const int L0 = F ? 0 : (st ? rc->ekb : m.elem_kb[ux(e)]) - 1;
     if constexpr (VM == 0) {
       const ZSigma<F> z{st ? st_node_z(*rc, 0) : node_z<F>(m, n0), st ? st_node_z(*rc, 1) : node_z<F>(m, n1),
                         st ? st_node_z(*rc, 2) : node_z<F>(m, n2), sig, nv};
       kb0 = z.q0.kb, kb1 = z.q1.kb, kb2 = z.q2.kb;
       z_bracket(z, s0, s1, s2, pz, L0, min(kb0, min(kb1, kb2)), R0, true, hint, L, R, w1, w2);
-      c.kept = true;
       c.zL = z.nodes(L);
       c.zR = z.nodes(R);
     } else {
@@ -515,26 +530,27 @@ __device__ void interp_velocity(const DMesh& m, const double* sig, double h0, in
                 f2 = m.zn ? m.nkz[ux(n2)] : m.kb[ux(n2)];
       kb0 = f0 & kKbMask, kb1 = f1 & kKbMask, kb2 = f2 & kKbMask;
       const ZColumns z{m, h0, n0, n1, n2};
-      const bool mono = m.zn && !((f0 | f1 | f2) & ~kKbMask);
+      mono = m.zn && !((f0 | f1 | f2) & ~kKbMask);
       z_bracket(z, s0, s1, s2, pz, L0, min(kb0, min(kb1, kb2)), R0, mono, hint, L, R, w1, w2);
-      c.kept = mono;
       c.zL = z.nodes(L);
       c.zR = z.nodes(R);
     }
-    c.L = L;
-    c.R = R;
+    c.br = mono ? (L + 1) << 10 | R : -1;
     // the three nodes' level rows (64-bit row offsets), then two levels of each
     const double4* U = reinterpret_cast<const double4*>(m.uvw);
     auto at = [&](int node, int level, int kb) {
-      const double4 q = U[(uint64_t)ux(node) * ux(nv) + ux(F ? level : max(level, kb))];
-      return double3{q.x, q.y, q.z};
+      return U[(uint64_t)ux(node) * ux(nv) + ux(F ? level : max(level, kb))];
     };
-    c.u0 = at(n0, L, kb0), c.u1 = at(n1, L, kb1), c.u2 = at(n2, L, kb2);
-    c.v0 = at(n0, R, kb0), c.v1 = at(n1, R, kb1), c.v2 = at(n2, R, kb2);
+    const double4 q[6] = {at(n0, L, kb0), at(n1, L, kb1), at(n2, L, kb2), at(n0, R, kb0), at(n1, R, kb1), at(n2, R, kb2)};
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      c.put(3 * i, q[i].x);
+      c.put(3 * i + 1, q[i].y);
+      c.put(3 * i + 2, q[i].z);
+    }
   }
-  const double uL = s0 * c.u0.x + s1 * c.u1.x + s2 * c.u2.x + 0.0, vL = s0 * c.u0.y + s1 * c.u1.y + s2 * c.u2.y + 0.0;
-  const double uR = s0 * c.v0.x + s1 * c.v1.x + s2 * c.v2.x + 0.0, vR = s0 * c.v0.y + s1 * c.v1.y + s2 * c.v2.y + 0.0;
-  const double wL = s0 * c.u0.z + s1 * c.u1.z + s2 * c.u2.z + 0.0, wR = s0 * c.v0.z + s1 * c.v1.z + s2 * c.v2.z + 0.0;
+  auto mean = [&](int i) { return s0 * c.get(i) + s1 * c.get(i + 3) + s2 * c.get(i + 6) + 0.0; };
+  const double uL = mean(0), vL = mean(1), uR = mean(9), vR = mean(10), wL = mean(2), wR = mean(11);
   uo = w1 * uL + w2 * uR;
   vo = w1 * vL + w2 * vR;
   wo = w1 * wL + w2 * wR;
@@ -616,12 +632,13 @@ __device__ bool celestial_walk(const DMesh& m, const int* key, const StElem* rec
 }
 
 // Side::btrack (meshdata.cu:1449-1629). Returns the final velocity and the foot element.
-template <int VM, bool ST, bool F>
-__device__ void btrack(const DMesh& m, const double* sig, const int* key, const StElem* rec, const StepArgs& a, int s,
+template <int VM, bool ST, bool F, bool LV>
+__device__ void btrack(const DMesh& m, const double* sig, double* lv, const int* key, const StElem* rec, const StepArgs& a, int s,
                        int k, double dtbk, int cur, double& ux, double& uy, int& foot, int& status) {
   const double h0 = a.h0;
   double x0x = m.side_cx[s], x0y = m.side_cy[s], x0z = m.zc[(int64_t)s * m.nvrt + k];
-  double time_rm = a.dt, t1 = 1e10, t2 = 2e10, t3 = 3e10;
+  double time_rm = a.dt;
+  int still = 0;  // iterations on end, not counting the first, that left time_rm as it was
   const int4 sr = m.side[s];
   const double4* U = reinterpret_cast<const double4*>(m.uvw);
   double uix = m.su2[2 * ((int64_t)s * m.nvrt + k)], uiy = m.su2[2 * ((int64_t)s * m.nvrt + k) + 1];
@@ -632,9 +649,9 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
   ElemGeom geo;  // set by every walk before its first use
   int slot = -1;  // geo's staged slot (ST)
   bool geo_valid = false;
-  BtCell cell;
-  double fu = 0.0, fv = 0.0;  // the interpolated velocity at the last point, where there is one
-  bool interpolated = false;
+  BtCell<LV> cell;
+  cell.lv = lv;
+  bool interpolated = false;  // (uix, uiy) is the interpolated velocity at the last point
   while (true) {
     interpolated = false;
     const double dtb = fmin(dtbk, time_rm);
@@ -645,7 +662,9 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
     const bool found = celestial_walk<ST>(m, key, rec, cur, x0x, x0y, xtx, xty, last, status, geo, slot, geo_valid);
     geo_valid = true;
     const StElem* rc = (ST && slot >= 0) ? rec + slot : nullptr;
-    if (t3 <= time_rm) {
+    // the reference compares time_rm with that of three iterations before (1e10 s before the first); it
+    // never grows, so it is not less after two iterations on end that left it as it was
+    if (still == 2) {
       xtx = x0x;
       xty = x0y;
       xtz = x0z;
@@ -674,7 +693,9 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
                   1.0);
         if (sp < 0.0000000001) sp = 0.0;
       }
+      const double before = time_rm;
       time_rm -= sp * dtb;
+      still = (iter > 0 && time_rm == before) ? still + 1 : 0;
       const double nz = x0z + sp * (xtz - x0z);
       xtx = p1x + t * v2x;
       xty = p1y + t * v2y;
@@ -686,21 +707,19 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
       const double len = sqrt(v2x * v2x + v2y * v2y);
       const double tx = v2x / len, ty = v2y / len;
       double iu, iv, iw;
-      interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, rc, cell, xtx, xty, xtz, iu, iv, iw, hint);
-      fu = iu;
-      fv = iv;
+      interp_velocity<VM, ST, F, LV>(m, sig, h0, cur, geo, rc, cell, xtx, xty, xtz, iu, iv, iw, hint);
       const double d = iu * tx + iv * ty;
       uix = tx * d;
       uiy = ty * d;
       uiz = iw;
       status |= GSH_BT_SLIDE;
     } else {
+      const double before = time_rm;
       time_rm -= dtb;
-      interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, rc, cell, xtx, xty, xtz, uix, uiy, uiz, hint);
-      fu = uix;
-      fv = uiy;
+      still = (iter > 0 && time_rm == before) ? still + 1 : 0;
+      interp_velocity<VM, ST, F, LV>(m, sig, h0, cur, geo, rc, cell, xtx, xty, xtz, uix, uiy, uiz, hint);
+      interpolated = true;
     }
-    interpolated = true;
     if (time_rm <= 0.0) break;
     if (uix * uix + uiy * uiy <= a.velmin2) {
       ux = uix;
@@ -719,16 +738,14 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
       foot = cur;
       return;
     }
-    t3 = t2;
-    t2 = t1;
-    t1 = time_rm;
   }
-  // the velocity at the last point: already interpolated unless the walk stuck or left the mesh there
-  ux = fu;
-  uy = fv;
+  // the velocity at the last point: already interpolated unless the walk slid, stuck or left the mesh
+  // there
+  ux = uix;
+  uy = uiy;
   if (!interpolated) {
     double iw;
-    interp_velocity<VM, ST, F>(m, sig, h0, cur, geo, (ST && slot >= 0) ? rec + slot : nullptr, cell, xtx, xty, xtz, ux,
+    interp_velocity<VM, ST, F, LV>(m, sig, h0, cur, geo, (ST && slot >= 0) ? rec + slot : nullptr, cell, xtx, xty, xtz, ux,
                                uy, iw, hint);
   }
   foot = cur;
@@ -737,14 +754,15 @@ __device__ void btrack(const DMesh& m, const double* sig, const int* key, const 
 // backtrackAllNodes (meshdata.cu:3547-3660), one thread per (side, level): consecutive
 // lanes are consecutive levels of one side, so the nodal [node][level] gathers of a wave
 // fall on a few contiguous cache lines.
-// VM: 0, one sigma per level (kept in LDS) and levels that do not decrease in any wet column; 1, each
+// LV: BtCell's velocities in LDS. VM: 0, one sigma per level (kept in LDS) and levels that do not decrease in any wet column; 1, each
 // node's own levels (DMesh::vmode 1 and 2, and 0 where levels may decrease).
 // ST: the workgroup first stages its element patch in LDS (all sides and levels, no list).
 // F: a mesh with kb = 0 at every node whose last sigma is 0 (VM = 0).
-template <int VM, bool ST, bool F>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 8)))
+template <int VM, bool ST, bool F, bool LV>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LV ? 4 : 3, 8)))
 k_backtrack(DMesh m, StepArgs a, const int32_t* list_side, const int32_t* list_lev, int32_t count) {
-  __shared__ double sig[VM == 0 ? 1024 : 1];
+  extern __shared__ double bt_lds[];  // LV: kCellVel x 256; VM = 0: the sigma levels
+  double* sig = bt_lds + (LV ? kCellVel * 256 : 0);
   __shared__ int st_key[ST ? kStSlots : 1];
   __shared__ StElem st_rec[ST ? kStSlots : 1];
   if (VM == 0) {
@@ -795,7 +813,7 @@ k_backtrack(DMesh m, StepArgs a, const int32_t* list_side, const int32_t* list_l
     const int ndelt = max(a.ndelt_min, min(nd, a.ndelt_max));
     const double dtbk = a.dt / ndelt;
     const int start = m.elem_wet[sr.z] ? sr.z : sr.w;
-    btrack<VM, ST, F>(m, sig, st_key, st_rec, a, s, k, dtbk, start, bx, by, foot, status);
+    btrack<VM, ST, F, LV>(m, sig, bt_lds + threadIdx.x, st_key, st_rec, a, s, k, dtbk, start, bx, by, foot, status);
   }
   m.btu[2 * idx] = bx;
   m.btu[2 * idx + 1] = by;
@@ -836,6 +854,13 @@ __global__ void k_pack_levels(DMesh m, double h0) {
   if (k > 0 && !(level(k - 1) <= z)) atomicOr(&m.nkz[i], kKbMask + 1);
 }
 
+// Workgroups from which the fourth wave a SIMD of the LV form pays for its LDS trips: three waves hold 768
+// on the chip. Register form / LV, flows that stay in their elements and that leave one each substep:
+// one sigma, 60x40x11 (303 workgroups) 45 / 49 and 119 / 126 us, 110x80x12 (1,220) 71 / 71 and 193 /
+// 190, 120x90x14 (1,750) 87 / 87 and 240 / 224; per-node sigma, whose search spills at four waves,
+// 120x80x21 (2,350) 116 / 119 and 368 / 385, 301x173x31 (18,900) 679 / 670 and 1,956 / 1,791.
+constexpr unsigned kBtFill = 1536, kBtFillColumns = 6144;
+
 void launch_backtrack(const DMesh& mesh, const StepArgs& a, const int32_t* ls, const int32_t* ll, int32_t count,
                       hipStream_t st) {
   DMesh m = mesh;
@@ -851,20 +876,31 @@ void launch_backtrack(const DMesh& mesh, const StepArgs& a, const int32_t* ls, c
   }
   const dim3 grid((unsigned)((total + 255) / 256));
   const bool stage = m.bt_stage != 0 && !ls;
-  auto go = [&](auto ker) { hipLaunchKernelGGL(ker, grid, dim3(256), 0, st, m, a, ls, ll, count); };
   // One sigma per level: a wet node's levels do not decrease where 0 <= h0 < H and every sigma between
   // bed and surface lies in [-1, 0], which VM = 0 relies on. Outside that, VM = 1 searches in full.
   const bool sigma = m.vmode == 0 && m.sig_mono && a.h0 >= 0.0;
-  if (sigma && stage)
-    go(k_backtrack<0, true, false>);
-  else if (sigma && m.flat)
-    go(k_backtrack<0, false, true>);
+  const size_t lds_sig = sigma ? 8 * (size_t)m.nvrt : 0;
+  auto go = [&](auto ker, size_t lds) { hipLaunchKernelGGL(ker, grid, dim3(256), lds, st, m, a, ls, ll, count); };
+  if (stage) {
+    if (sigma)
+      go(k_backtrack<0, true, false, false>, lds_sig);
+    else
+      go(k_backtrack<1, true, false, false>, 0);
+    return;
+  }
+  const bool lv = grid.x > (sigma ? kBtFill : kBtFillColumns);
+  auto pick = [&](auto ldsv, auto regv) {
+    if (lv)
+      go(ldsv, lds_sig + 8 * kCellVel * 256);
+    else
+      go(regv, lds_sig);
+  };
+  if (sigma && m.flat)
+    pick(k_backtrack<0, false, true, true>, k_backtrack<0, false, true, false>);
   else if (sigma)
-    go(k_backtrack<0, false, false>);
-  else if (stage)
-    go(k_backtrack<1, true, false>);
+    pick(k_backtrack<0, false, false, true>, k_backtrack<0, false, false, false>);
   else
-    go(k_backtrack<1, false, false>);
+    pick(k_backtrack<1, false, false, true>, k_backtrack<1, false, false, false>);
 }
 
 // ---------------------------------------------------------------- nodal velocities

@@ -56,11 +56,24 @@ def test_momentum_of_few_levels_keeps_its_waves(tmp_path):
 
 @needs_compiler
 def test_backtracking_counters_are_of_this_kernel(tmp_path):
-    """bench.py divides the committed counters of k_backtrack by its own time: they are of the kernel
-    that these sources build, at least as far as its registers tell."""
+    """bench.py divides the committed counters of k_backtrack by its own time: the profile names a
+    kernel that these sources build, with its registers and waves."""
     spec = importlib.util.spec_from_file_location("bench", build.CSRC.parents[1] / "bench.py")
     bench = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(bench)
     bound = bench.backtrack_bound()
-    k = _usage("mesh_kernels.hip", tmp_path)["gsh::k_backtrack<0, false, true>"]
+    text = (build.CSRC.parents[1] / "profiles" / "backtrack_counters_channel-1024x1024.md").read_text()
+    k = _usage("mesh_kernels.hip", tmp_path)["gsh::" + re.search(r"`(k_backtrack<[^`]*>)`", text).group(1)]
     assert bound["vgprs"] == k["VGPRs"] and bound["waves_per_simd"] <= k["Occupancy"]
+
+
+@needs_compiler
+def test_backtracking_forms_keep_their_waves(tmp_path):
+    """With the kept velocities in LDS four waves a SIMD, which flows that change element in each substep
+    need; in registers, for grids that do not fill the chip, three. No scratch on one sigma and flat beds."""
+    u = _usage("mesh_kernels.hip", tmp_path)
+    for variant in ("0, false, true", "0, false, false", "1, false, false"):
+        assert u[f"gsh::k_backtrack<{variant}, true>"]["Occupancy"] >= 4
+        assert u[f"gsh::k_backtrack<{variant}, false>"]["Occupancy"] >= 3
+    for lv in ("true", "false"):
+        assert u[f"gsh::k_backtrack<0, false, true, {lv}>"]["ScratchSize"] == 0

@@ -978,3 +978,32 @@ def test_backtrack_levels_out_of_order(ctx, levels, staged):
     for f in (L.F_FOOT, L.F_BTU, L.F_BSTATUS):
         assert_bitwise(mesh.get(f), om.get(f), f"field {f}")
     mesh.close()
+
+
+@pytest.mark.parametrize("u,v", [(0.8, 0.6), (1.0, 0.01), (1.0, 1.0), (0.3, -1.0)])
+def test_backtrack_into_corners(ctx, u, v):
+    """A closed basin of 8 m elements and a uniform flow of many elements a step: every start point
+    slides along a wall, most end in a corner where no substep moves them any more, or after 38."""
+    spec = cases.CaseSpec("corners", 16, 12, 8.0, nvrt=4, depth=10.0, substeps=20)
+    data = cases.make_case(spec)
+    n, sigma = data.xy.shape[0], np.linspace(-1.0, 0.0, 4)
+    mesh = core.Mesh(ctx, data.xy, data.elnode, np.full(n, 10.0), sigma, open_bnd=np.zeros(n, np.int8))
+    om = oracle_mesh_for(mesh, sigma)
+    p = cases.step_params(spec)
+    uvw, su2 = np.zeros((n, 4, 3)), np.zeros((mesh.ns, 4, 2))
+    uvw[..., :2] = su2[...] = (u, v)
+    for m in (mesh, om):
+        m.set(L.F_ETA2, np.zeros(n))
+        m.set(L.F_NODE_UVW, uvw)
+        m.set(L.F_SIDE_U2, su2)
+    mesh.update_levels(p)
+    om.levels(p)
+    for staged in (False, True):
+        mesh.set_backtrack_staging(staged)
+        print(f"[gpu] backtracking into corners, flow {u} {v}, staged {staged}", flush=True)
+        mesh.backtrack(p)
+        om.backtrack(p, nthreads=8)
+        for f in (L.F_FOOT, L.F_BTU, L.F_BSTATUS):
+            assert_bitwise(mesh.get(f), om.get(f), f"field {f}")
+    assert (mesh.get(L.F_BSTATUS) & L.BT_STUCK).any()
+    mesh.close()

@@ -6,7 +6,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from conftest import assert_bitwise
+from conftest import assert_bitwise, oracle_mesh_for
 from gschism_amd import _lib as L
 from gschism_amd import cases, core
 from oracle import pyoracle as O
@@ -195,3 +195,52 @@ def test_backtrack_columns(ctx, grid, state):
     om.backtrack(p, nthreads=8)
     for f in (L.F_FOOT, L.F_BTU, L.F_BSTATUS):
         assert_bitwise(mesh.get(f), om.get(f), f"field {f}")
+
+
+@pytest.mark.parametrize("dx", [400.0, 8.0])
+@pytest.mark.parametrize("grid,nx,ny", [("sigma", 66, 50), ("sigma-kb", 66, 50), ("sz", 132, 112), ("lsc2", 132, 112),
+                                        ("sigma", 60, 40), ("lsc2", 60, 40)])
+def test_backtrack_forms(ctx, grid, nx, ny, dx):
+    """Grids of enough start points that the kept prism's velocities lie in LDS (from 1,537 workgroups of
+    256 on, on per-node sigma and SZ grids from 6,145) and smaller ones, with flows that stay in their
+    elements and, at 8 m, flows that leave one or two in each substep and run along the walls."""
+    nvrt = 41 if grid in ("sigma", "sigma-kb") else 37
+    spec = cases.CaseSpec(f"forms-{grid}", nx, ny, dx, nvrt=nvrt, depth=10.0, substeps=8)
+    data = cases.make_case(spec)
+    depth = 6.0 + 70.0 * (data.xy[:, 0] / data.xy[:, 0].max())
+    sigma, kb, vg = np.linspace(-1.0, 0.0, nvrt), None, None
+    if grid == "sz":
+        vg = core.VGrid(2, nz=3, h_s=40.0, h_c=10.0, theta_b=0.3, theta_f=6.0, ztot=np.array([-160.0, -80.0, -40.0]),
+                        sigma_s=np.linspace(-1.0, 0.0, nvrt - 2))
+    elif grid == "lsc2":
+        vg = core.VGrid(1, sigma_node=-1.0 + np.linspace(0.0, 1.0, nvrt)[None, :] ** (1.0 + 0.7 * np.sin(np.arange(spec.n)))[:, None])
+    if grid in ("sigma-kb", "lsc2"):
+        kb = np.clip((0.4 * nvrt * (1.0 - depth / depth.max())).astype(np.int32), 0, nvrt - 3)
+    if vg is None:
+        mesh = core.Mesh(ctx, data.xy, data.elnode, depth, sigma, open_bnd=data.open_bnd, kb=kb)
+        om = oracle_mesh_for(mesh, sigma)
+        eta, uvw, su2 = cases.initial_state(spec, mesh.topology(L.T_XY), cases.side_centres(mesh), sigma)
+        p = cases.step_params(spec)
+        for m in (mesh, om):
+            m.set(L.F_ETA2, eta)
+            m.set(L.F_NODE_UVW, uvw)
+            m.set(L.F_SIDE_U2, su2)
+        mesh.update_levels(p)
+        om.levels(p)
+    else:
+        mesh, om, p = _setup_vgrid(ctx, spec, depth, vg, kb=kb)
+    uvw = mesh.get(L.F_NODE_UVW)
+    uvw[..., 2] += 0.003 * cases.normal(7, uvw[..., 2].size).reshape(uvw[..., 2].shape)
+    for m in (mesh, om):
+        m.set(L.F_NODE_UVW, uvw)
+    wgs = -(-mesh.ns * nvrt // 256)
+    print(f"[gpu] backtracking forms, {grid}, {wgs} workgroups, dx {dx}", flush=True)
+    assert (wgs > (1536 if "sigma" in grid else 6144)) == (nx > 60)
+    mesh.backtrack(p)
+    om.backtrack(p, nthreads=8)
+    for f in (L.F_FOOT, L.F_BTU, L.F_BSTATUS):
+        assert_bitwise(mesh.get(f), om.get(f), f"field {f}")
+    flags = int(np.bitwise_or.reduce(mesh.get(L.F_BSTATUS).ravel()))
+    print(f"flags met: {flags}", flush=True)
+    assert dx > 8.0 or flags & L.BT_SLIDE
+    mesh.close()
