@@ -245,6 +245,7 @@ struct gsh_solver {
   uint64_t* run_words = nullptr;
   uint32_t run_epoch = 1;
   int32_t max_row = 0, band = 0;
+  int32_t max_chunk = 0;  // the most entries in 64 rows (launch_pcg_phase)
   // their bounded wait; solves still kept on the phases after a launch that gave up, and how many the
   // last one meant; solves that ran whole, and that gave up and took the phases
   int32_t run_polls = kRunPolls, run_skip = 0, run_backoff = 0, run_whole = 0, run_gave_up = 0;
@@ -307,7 +308,9 @@ static void solver_alloc(gsh_solver* s, int32_t n, int64_t nnz, const std::vecto
     bool ok = true;
     for (int32_t r = 0; r < n; r += 64) {
       int32_t lo = r, hi = r;
-      for (int32_t k = indptr[r], end = indptr[std::min(r + 64, n)]; k < end; ++k) {
+      const int32_t start = indptr[r], end = indptr[std::min(r + 64, n)];
+      s->max_chunk = std::max(s->max_chunk, end - start);
+      for (int32_t k = start; k < end; ++k) {
         lo = std::min(lo, col[k]);
         hi = std::max(hi, col[k]);
         out[k] = (int16_t)(col[k] - r);
@@ -658,7 +661,7 @@ template <class VT>
 static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const TileRef* dtiles, int ntiles, int rpt,
                          double rtol, int maxiter, int check_every, double timeout_s, PcgState* dgather,
                          const TileRef* dinit_tiles, int ninit_tiles, PhaseTimes* prof, const double* rtols_dev,
-                         WindowGraph* graph, gsh_solver* solo) {
+                         WindowGraph* graph, gsh_solver* solo, int chunk) {
   hipStream_t st = ctx->stream;
   if (check_every < 1) check_every = 1;
   if (timeout_s <= 0.0) timeout_s = 60.0;
@@ -738,8 +741,8 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
       std::vector<hipEvent_t> evs(4 * w);
       for (auto& e : evs) HIPCHK(hipEventCreate(&e));
       for (int i = 0; i < w; ++i) {
-        launch_pcg_phase<VT>(0, dsys, ptiles, ntiles, rpt, st, evs[4 * i], evs[4 * i + 1]);
-        launch_pcg_phase<VT>(1, dsys, ptiles, ntiles, rpt, st, evs[4 * i + 2], evs[4 * i + 3]);
+        launch_pcg_phase<VT>(0, dsys, ptiles, ntiles, rpt, st, chunk, evs[4 * i], evs[4 * i + 1]);
+        launch_pcg_phase<VT>(1, dsys, ptiles, ntiles, rpt, st, chunk, evs[4 * i + 2], evs[4 * i + 3]);
       }
       HIPCHK(hipEventSynchronize(evs[4 * w - 1]));
       for (int i = 0; i < w; ++i) {
@@ -754,7 +757,7 @@ static void run_pcg_core(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const T
       launch_pcg_check<VT>(dsys, nsys, st);
     } else {
       auto issue = [&]() {
-        for (int i = 0; i < w; ++i) launch_pcg_iter<VT>(dsys, ptiles, ntiles, rpt, st);
+        for (int i = 0; i < w; ++i) launch_pcg_iter<VT>(dsys, ptiles, ntiles, rpt, st, chunk);
         launch_pcg_check<VT>(dsys, nsys, st);
       };
       if (!(graph && launch_window_graph(*graph, st, dsys, w, rpt, issue))) issue();
@@ -785,11 +788,11 @@ static void run_pcg(gsh_ctx* ctx, const PcgSys<VT>* dsys, int nsys, const TileRe
                     double rtol, int maxiter, int check_every, double timeout_s, PcgOutcome& out,
                     const TileRef* dinit_tiles = nullptr, int ninit_tiles = -1, PhaseTimes* prof = nullptr,
                     const double* rtols_dev = nullptr, WindowGraph* graph = nullptr,
-                    gsh_solver* solo = nullptr) {
+                    gsh_solver* solo = nullptr, int chunk = 0) {
   StreamBuffers tmp(ctx->stream);
   PcgState* dgather = tmp.alloc<PcgState>(2 * (size_t)nsys);
   run_pcg_core<VT>(ctx, dsys, nsys, dtiles, ntiles, rpt, rtol, maxiter, check_every, timeout_s, dgather, dinit_tiles,
-                   ninit_tiles, prof, rtols_dev, graph, solo);
+                   ninit_tiles, prof, rtols_dev, graph, solo, chunk);
   const PcgState* slots = ctx->pinned;
   out.st.assign(slots, slots + nsys);
 }
@@ -1184,7 +1187,9 @@ static void run_mixed(gsh_ctx* ctx, gsh_solver* const* S, int count, double rtol
       std::vector<PcgSys<double>> s64(ns);
       std::vector<PcgSys<float>> s32(ns);
       std::vector<TileRef> stl;
+      int chunk = 0;
       for (int j = 0; j < ns; ++j) {
+        chunk = std::max(chunk, S[sub[j]]->max_chunk);
         s64[j] = h64[sub[j]];
         s32[j] = h32[sub[j]];
         for (int t = 0; t < S[sub[j]]->ntiles; ++t) stl.push_back({j, t});
@@ -1194,7 +1199,7 @@ static void run_mixed(gsh_ctx* ctx, gsh_solver* const* S, int count, double rtol
       HIPCHK(hipMemcpyAsync(dtl, stl.data(), sizeof(TileRef) * stl.size(), hipMemcpyHostToDevice, st));
       HIPCHK(hipMemcpyAsync(drt, rts.data(), sizeof(double) * ns, hipMemcpyHostToDevice, st));
       run_pcg<float>(ctx, d32s, ns, dtl, (int)stl.size(), rpt, rtol, maxiter, check_every, timeout_s, o, nullptr, -1,
-                     nullptr, drt, nullptr, ns == 1 ? S[sub[0]] : nullptr);
+                     nullptr, drt, nullptr, ns == 1 ? S[sub[0]] : nullptr, chunk);
       launch_refine_batch(d64s, d32s, dtl, (int)stl.size(), rpt, st);
     }
     for (int j = 0; j < ns; ++j) {
@@ -1292,6 +1297,11 @@ __global__ void k_static_csr(const int32_t* __restrict__ indptr, const int32_t* 
         d = (int32_t)k;
     }
     if (d < 0) f |= 4;
+  }
+  if (i % 64 == 0) {  // not errors: chunks too long for one piece of the wide phases, and for their rule
+    const int64_t chunk = indptr[min(i + 64, n)] - a;
+    if (chunk > kWideChunk) f |= 8;
+    if (chunk > kWideLong) f |= 16;
   }
   diag[i] = d;
   if (f) atomicOr(flag, f);
@@ -2129,10 +2139,10 @@ int gsh_solver_autotune(gsh_solver* s, int iters, int* best_rpt, double* us_per_
           launch_cast_values(s->val, s->val32, s->nnz, st);
           launch_copy_f64(s->r64, s->b, s->n, st);
           run_pcg<float>(s->ctx, s->ds32, 1, s->dtiles, s->ntiles, r, 1e-300, iters, iters, 60.0, o, nullptr, -1, &pt,
-                         nullptr, nullptr, s);
+                         nullptr, nullptr, s, s->max_chunk);
         } else {
           run_pcg<double>(s->ctx, s->ds, 1, s->dtiles, s->ntiles, r, 1e-300, iters, iters, 60.0, o, nullptr, -1, &pt,
-                          nullptr, &s->wg_jacobi, s);
+                          nullptr, &s->wg_jacobi, s, s->max_chunk);
         }
         us = pt.launches ? 1e3 * (pt.ms_a + pt.ms_b) / pt.launches : 1e300;
       }
@@ -2256,7 +2266,7 @@ int gsh_solver_solve(gsh_solver* s, const double* b_host, double* x_host, double
     } else {
       PcgOutcome o;
       run_pcg<double>(s->ctx, s->ds, 1, s->dtiles, s->ntiles, s->rpt, rtol, maxiter, check_every, timeout_s, o,
-                      nullptr, -1, nullptr, nullptr, &s->wg_jacobi, s);
+                      nullptr, -1, nullptr, nullptr, &s->wg_jacobi, s, s->max_chunk);
       const PcgState& r = o.st[0];
       iters = iters_of(r, maxiter);
       status = (r.done >= 0) ? 0 : GSH_W_MAXITER;
@@ -2340,7 +2350,8 @@ int gsh_pcg_solve_static(gsh_ctx* ctx, int32_t n, int64_t nnz, const int32_t* in
     hipLaunchKernelGGL(k_static_desc, dim3(1), dim3(1), 0, st, h, dsys);
     HIPCHK(hipGetLastError());
     run_pcg_core<double>(ctx, dsys, 1, dtiles, ntiles, kStaticRpt, rtol, maxiter, check_every, timeout_s, dgather,
-                         nullptr, -1, nullptr, nullptr, nullptr, nullptr);
+                         nullptr, -1, nullptr, nullptr, nullptr, nullptr,
+                         (f & 16) ? INT32_MAX : ((f & 8) ? kWideChunk + 1 : 0));
     const PcgState r = ctx->pinned[0];
     if (iters_out) *iters_out = iters_of(r, maxiter);
     if (status_out) *status_out = (r.done >= 0) ? 0 : GSH_W_MAXITER;
@@ -2457,7 +2468,10 @@ int gsh_batch_solve(gsh_solver* const* solvers, int count, double rtol, int maxi
     HIPCHK(hipMemcpyAsync(dsys, hs.data(), sizeof(PcgSys<double>) * count, hipMemcpyHostToDevice, st));
     HIPCHK(hipMemcpyAsync(dt, tiles.data(), sizeof(TileRef) * tiles.size(), hipMemcpyHostToDevice, st));
     PcgOutcome o;
-    run_pcg<double>(ctx, dsys, count, dt, (int)tiles.size(), rpt, rtol, maxiter, check_every, timeout_s, o);
+    int chunk = 0;
+    for (int i = 0; i < count; ++i) chunk = std::max(chunk, solvers[i]->max_chunk);
+    run_pcg<double>(ctx, dsys, count, dt, (int)tiles.size(), rpt, rtol, maxiter, check_every, timeout_s, o, nullptr, -1,
+                    nullptr, nullptr, nullptr, nullptr, chunk);
     HIPCHK(hipStreamSynchronize(st));
     for (int i = 0; i < count; ++i) {
       gsh_solver* s = solvers[i];
@@ -3413,7 +3427,7 @@ int gsh_solver_profile(gsh_solver* s, double rtol, int maxiter, int check_every,
     PcgOutcome o;
     PhaseTimes pt;
     run_pcg<double>(s->ctx, s->ds, 1, s->dtiles, s->ntiles, s->rpt, rtol, maxiter, check_every, 60.0, o, nullptr,
-                    -1, &pt);
+                    -1, &pt, nullptr, nullptr, nullptr, s->max_chunk);
     const int it = iters_of(o.st[0], maxiter);
     HIPCHK(hipStreamSynchronize(s->ctx->stream));
     solver_roll(s);

@@ -235,15 +235,18 @@ void launch_pcg_reset(const PcgSys<VT>* sys, int nsys, double rtol, int maxiter,
 template <class VT>
 void launch_pcg_init(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s);
 template <class VT>
-void launch_pcg_iter(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s);
-// tiles = NULL: one system (*sys), whose tiles are 0 .. ntiles - 1
+void launch_pcg_iter(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s, int chunk = 0);
+// tiles = NULL: one system (*sys), whose tiles are 0 .. ntiles - 1. chunk: the most entries in 64 rows
+// from a multiple of 64 on (0: not known, taken for few).
 template <class VT>
 void launch_pcg_phase(int which, const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s,
-                      hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+                      int chunk = 0, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // Up to `iters` iterations of one system in one launch, for systems that pcg_run_fits accepts: max_row,
 // the longest row; band, the largest |column - row|. words: kRunWords exchange words, zero at first;
 // epoch: above iters plus that of every earlier launch on these words, so at least 1. polls: the bound
 // of a workgroup's wait for the others (kRunPolls; 0: every workgroup gives up at its first wait).
+constexpr int kWideChunk = 576;                  // entries of a 64-row chunk that the wide phases take at once
+constexpr int kWideLong = 832;                   // and up to which two pieces cost them their lead (launch_pcg_phase)
 constexpr int kRunTiles = 128;                   // tiles at most
 constexpr int kRunRows = 4 * kTpb * kRunTiles;   // rows at most
 constexpr int kRunWords = 6 * kRunTiles;

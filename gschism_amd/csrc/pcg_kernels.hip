@@ -196,9 +196,10 @@ __global__ void __launch_bounds__(256) k_pcg_init(const PcgSys<VT>* __restrict__
 // rows 19.3 ms against 16.8, of 96 systems of 5,000 to 200,000 rows 12.6 against 11.8).
 template <class VT, bool W>
 struct Chunk {
-  // nonzeros of a 64-row chunk held in registers: 10 per lane; 9 in the wide form, whose 16 waves'
-  // products then take 72 KB of LDS and two workgroups fit a CU
-  static constexpr int kM = W ? 9 : 10, kCap = 64 * kM;
+  // nonzeros of a 64-row chunk held in registers, per lane. The narrow form sums a longer chunk row by
+  // row; the wide one, whose four times as many rows in flight then ran the caches over (500,000 rows of
+  // 15 entries 156 us an iteration against 62), takes it in pieces (50 us).
+  static constexpr int kM = W ? kWideChunk / 64 : 10, kCap = 64 * kM;
   int s0, e0;
   VT v[kM], zc[kM], pc[kM];
 };
@@ -363,6 +364,22 @@ __device__ __forceinline__ void pcg_phase_a_body(const SysView<VT>& S, int tile,
         for (int kk = a; kk < b; ++kk) q += my[kk - c.s0];
       }
       wave_lds_sync();
+    } else if (W) {
+      // a longer chunk in pieces, each loaded as a chunk is and summed by the rows that it holds entries of
+      for (int p0 = c.s0; p0 < c.e0; p0 += kCap) {
+        Chunk<VT, W> d;
+        const int p1 = min(p0 + kCap, c.e0);
+        load_chunk(S, po, r0w, lane, p0, p1, d);
+#pragma unroll
+        for (int m = 0; m < d.kM; ++m) {
+          const int kk = p0 + lane + 64 * m;
+          if (kk < p1) my[kk - p0] = d.v[m] * (d.zc[m] + bv * d.pc[m]);
+        }
+        wave_lds_sync();
+        const int a = max(ra[j], p0), b = min(rb[j], p1);
+        for (int kk = a; kk < b; ++kk) q += my[kk - p0];
+        wave_lds_sync();
+      }
     } else if (i < n) {
       const int a = ra[j], b = rb[j];
       for (int kk = a; kk < b; ++kk) {
@@ -977,11 +994,15 @@ static void launch_stamped(void (*ker)(A...), int grid, int block, hipStream_t s
 // narrow, at R = 4: 16,000 rows 15.1 against 24.3, 66,887 14.8 against 24.2, 501,264 (490 tiles) 30.0
 // against 33.5, 1,048,576 (1,024 tiles) 53.7 against 42.3; at R = 2: 66,887 13.2 against 16.3,
 // 501,264 (980 tiles) 28.7 against 26.0.
-constexpr int kWideTiles = 512;
+// At R = 4 a workgroup's 16 waves fill a CU's registers, so more than 256 tiles come in two rounds; where
+// the chunks also take two pieces each (577 to 832 entries) the narrow form is faster there: 293 tiles
+// of 10 entries a row 36.4 against 39.4, of 13 41.2 against 44.5, of 14 (three pieces' worth of row by row)
+// 46.2 against 46.1; 254 tiles of 10 entries a row 34.0 against 24.3.
+constexpr int kWideTiles = 512, kWideTilesLong = 256;
 
 template <class VT>
 void launch_pcg_phase(int which, const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s,
-                      hipEvent_t e0, hipEvent_t e1) {
+                      int chunk, hipEvent_t e0, hipEvent_t e1) {
   if (ntiles <= 0) return;
   with_rpt(rpt, [&](auto r) {
     constexpr int R = decltype(r)::value;
@@ -991,15 +1012,16 @@ void launch_pcg_phase(int which, const PcgSys<VT>* sys, const TileRef* tiles, in
                      e1, sys, tiles);
     };
     if constexpr (R == 2 || R == 4)
-      if (ntiles <= kWideTiles) return run(std::true_type());
+      if (ntiles <= ((R == 4 && chunk > kWideChunk && chunk <= kWideLong) ? kWideTilesLong : kWideTiles))
+        return run(std::true_type());
     run(std::false_type());
   });
 }
 
 template <class VT>
-void launch_pcg_iter(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s) {
-  launch_pcg_phase<VT>(0, sys, tiles, ntiles, rpt, s);
-  launch_pcg_phase<VT>(1, sys, tiles, ntiles, rpt, s);
+void launch_pcg_iter(const PcgSys<VT>* sys, const TileRef* tiles, int ntiles, int rpt, hipStream_t s, int chunk) {
+  launch_pcg_phase<VT>(0, sys, tiles, ntiles, rpt, s, chunk);
+  launch_pcg_phase<VT>(1, sys, tiles, ntiles, rpt, s, chunk);
 }
 
 bool pcg_run_fits(int ntiles, int rpt, int max_row, int band) {
@@ -1037,11 +1059,11 @@ template void launch_pcg_reset<double>(const PcgSys<double>*, int, double, int, 
 template void launch_pcg_reset<float>(const PcgSys<float>*, int, double, int, int, hipStream_t, const double*);
 template void launch_pcg_init<double>(const PcgSys<double>*, const TileRef*, int, int, hipStream_t);
 template void launch_pcg_init<float>(const PcgSys<float>*, const TileRef*, int, int, hipStream_t);
-template void launch_pcg_iter<double>(const PcgSys<double>*, const TileRef*, int, int, hipStream_t);
-template void launch_pcg_iter<float>(const PcgSys<float>*, const TileRef*, int, int, hipStream_t);
-template void launch_pcg_phase<double>(int, const PcgSys<double>*, const TileRef*, int, int, hipStream_t, hipEvent_t,
+template void launch_pcg_iter<double>(const PcgSys<double>*, const TileRef*, int, int, hipStream_t, int);
+template void launch_pcg_iter<float>(const PcgSys<float>*, const TileRef*, int, int, hipStream_t, int);
+template void launch_pcg_phase<double>(int, const PcgSys<double>*, const TileRef*, int, int, hipStream_t, int, hipEvent_t,
                                        hipEvent_t);
-template void launch_pcg_phase<float>(int, const PcgSys<float>*, const TileRef*, int, int, hipStream_t, hipEvent_t,
+template void launch_pcg_phase<float>(int, const PcgSys<float>*, const TileRef*, int, int, hipStream_t, int, hipEvent_t,
                                        hipEvent_t);
 template void launch_pcg_run<double>(const PcgSys<double>*, int, int, uint64_t*, uint32_t, int, int, int, hipStream_t, hipEvent_t,
                                      hipEvent_t);

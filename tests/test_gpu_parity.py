@@ -746,6 +746,23 @@ def test_small_systems_in_one_launch(ctx, rpt, n, maxiter):
     s.close()
 
 
+@pytest.mark.parametrize("rpt,n,half", [(4, 140 * 1024 + 3, 13), (2, 70 * 512 + 65, 13), (4, 270 * 1024 - 1, 5),
+                                        (4, 270 * 1024 - 1, 6), (4, 270 * 1024 - 1, 7), (2, 500 * 512 + 1, 20)])
+def test_wide_phases_take_long_chunks_in_pieces(ctx, rpt, n, half):
+    """Rows of 11 to 41 entries, whose 64-row chunks hold 704 to 2,624: two to five pieces in the wide
+    phases, the last one short, and rows cut by a piece's end; above 256 tiles of 1,024 rows up to 832 entries
+    go to the narrow phases. Bit for bit."""
+    s, sys = _banded(ctx, n, list(range(-half, half + 1)), rpt)
+    b = cases.normal(48, n)
+    print(f"[gpu] long chunks, n={n}, {rpt} rows per thread, {2 * half + 1} entries a row", flush=True)
+    s.set_one_launch(polls=0)
+    x, it, _ = s.solve(b, rtol=1e-300, maxiter=20, check_every=10)
+    xo, ito, _, _ = O.pcg(*sys, b, rtol=1e-300, maxiter=20, check_every=10, rows_per_thread=rpt, nthreads=8)
+    assert it == ito
+    assert_bitwise(x, xo, f"{n} rows of {2 * half + 1} entries")
+    s.close()
+
+
 @pytest.mark.parametrize("rpt,n,offsets,whole", [
     (4, 9 * 1024 + 3, [-2560, -1, 0, 1, 2560], True),    # the widest window of p: 1024 + 2 * 2560 = 6144
     (4, 9 * 1024 + 3, [-2561, -1, 0, 1, 2561], False),
