@@ -247,6 +247,7 @@ void launch_pcg_phase(int which, const PcgSys<VT>* sys, const TileRef* tiles, in
 // of a workgroup's wait for the others (kRunPolls; 0: every workgroup gives up at its first wait).
 constexpr int kWideChunk = 576;                  // entries of a 64-row chunk that the wide phases take at once
 constexpr int kWideLong = 832;                   // and up to which two pieces cost them their lead (launch_pcg_phase)
+constexpr int kWideLong32 = 1024;                // the same in FP32
 constexpr int kRunTiles = 128;                   // tiles at most
 constexpr int kRunRows = 4 * kTpb * kRunTiles;   // rows at most
 constexpr int kRunWords = 6 * kRunTiles;

@@ -997,7 +997,7 @@ static void launch_stamped(void (*ker)(A...), int grid, int block, hipStream_t s
 // At R = 4 a workgroup's 16 waves fill a CU's registers, so more than 256 tiles come in two rounds; where
 // the chunks also take two pieces each (577 to 832 entries) the narrow form is faster there: 293 tiles
 // of 10 entries a row 36.4 against 39.4, of 13 41.2 against 44.5, of 14 (three pieces' worth of row by row)
-// 46.2 against 46.1; 254 tiles of 10 entries a row 34.0 against 24.3.
+// 46.2 against 46.1; 254 tiles of 10 entries a row 34.0 against 24.3. FP32 up to 16 entries a row.
 constexpr int kWideTiles = 512, kWideTilesLong = 256;
 
 template <class VT>
@@ -1012,7 +1012,7 @@ void launch_pcg_phase(int which, const PcgSys<VT>* sys, const TileRef* tiles, in
                      e1, sys, tiles);
     };
     if constexpr (R == 2 || R == 4)
-      if (ntiles <= ((R == 4 && chunk > kWideChunk && chunk <= kWideLong) ? kWideTilesLong : kWideTiles))
+      if (ntiles <= ((R == 4 && chunk > kWideChunk && chunk <= (sizeof(VT) == 8 ? kWideLong : kWideLong32)) ? kWideTilesLong : kWideTiles))
         return run(std::true_type());
     run(std::false_type());
   });
