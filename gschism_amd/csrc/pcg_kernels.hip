@@ -988,7 +988,7 @@ static void launch_stamped(void (*ker)(A...), int grid, int block, hipStream_t s
     hipLaunchKernelGGL(ker, dim3(grid), dim3(block), 0, s, a...);
 }
 
-// Wide workgroups (R = 2, 4) up to 512 tiles, two for every CU: below that the tiles' serial
+// Wide workgroups (R = 2, 4) up to 512 tiles: below that the tiles' serial
 // sub-rounds leave the chip waiting, above it the narrow form's row pointers, loaded ahead for R
 // sub-rounds, keep more in flight per register. Microseconds per Jacobi iteration, wide against
 // narrow, at R = 4: 16,000 rows 15.1 against 24.3, 66,887 14.8 against 24.2, 501,264 (490 tiles) 30.0
@@ -996,8 +996,8 @@ static void launch_stamped(void (*ker)(A...), int grid, int block, hipStream_t s
 // 501,264 (980 tiles) 28.7 against 26.0.
 // At R = 4 a workgroup's 16 waves fill a CU's registers, so more than 256 tiles come in two rounds; where
 // the chunks also take two pieces each (577 to 832 entries) the narrow form is faster there: 293 tiles
-// of 10 entries a row 36.4 against 39.4, of 13 41.2 against 44.5, of 14 (three pieces' worth of row by row)
-// 46.2 against 46.1; 254 tiles of 10 entries a row 34.0 against 24.3. FP32 up to 16 entries a row.
+// of 10 entries a row 39.4 against 36.4, of 13 44.5 against 41.2, of 14 46.1 against 46.2; 254 tiles of 10
+// entries a row 24.3 against 34.0. FP32 up to 16 entries a row.
 constexpr int kWideTiles = 512, kWideTilesLong = 256;
 
 template <class VT>
