@@ -325,8 +325,8 @@ __device__ __forceinline__ double zlev(const NodeZ& q, double sM, int M, int nv)
 }
 
 // z of level M at the point with shape coordinates s0..s2 (the vertical bracket search's probe).
-// One sigma per level (Lv = 0) reads it once per probe from sig (LDS); otherwise each node's level
-// max(M, kb) comes from its column zn (k_pack_levels), or from z_wet where that is not kept.
+// One sigma per level (VM = 0) reads it once per probe from sig (LDS); otherwise each node's level
+// max(M, kb) comes from its column zn (VM = 1, k_pack_levels) or from z_wet (VM = 2).
 template <bool F>
 struct ZSigma {
   NodeZ q0, q1, q2;
@@ -343,18 +343,28 @@ struct ZSigma {
 };
 struct ZColumns {
   const DMesh& m;
-  double h0;
   int n0, n1, n2;
   __device__ __forceinline__ double level(int node, int M) const {
-    if (m.zn) return m.zn[(uint64_t)ux(node) * ux(m.nvrt) + ux(max(M, 0))];
-    const double2 q = m.nrec[2u * ux(node) + 1u];
-    const int kb = m.kb[ux(node)];
-    if (q.x + q.y <= h0) return 0.0;
-    return (M <= kb) ? -q.y : z_wet(m, node, q.x, q.y, kb, M);
+    return m.zn[(uint64_t)ux(node) * ux(m.nvrt) + ux(max(M, 0))];
   }
   __device__ __forceinline__ double3 nodes(int M) const { return {level(n0, M), level(n1, M), level(n2, M)}; }
   __device__ __forceinline__ double operator()(double s0, double s1, double s2, int M) const {
     return s0 * level(n0, M) + s1 * level(n1, M) + s2 * level(n2, M) + 0.0;
+  }
+};
+
+struct ZLevels {  // the nodes' records, read once per interpolation
+  const DMesh& m;
+  int n0, n1, n2;
+  double2 q0, q1, q2;  // eta, depth
+  int kb0, kb1, kb2;
+  bool d0, d1, d2;     // dry
+  __device__ __forceinline__ double level(int node, const double2& q, int kb, bool dry, int M) const {
+    const double z = (M <= kb) ? -q.y : z_wet(m, node, q.x, q.y, kb, M);
+    return dry ? 0.0 : z;
+  }
+  __device__ __forceinline__ double operator()(double s0, double s1, double s2, int M) const {
+    return s0 * level(n0, q0, kb0, d0, M) + s1 * level(n1, q1, kb1, d1, M) + s2 * level(n2, q2, kb2, d2, M) + 0.0;
   }
 };
 
@@ -524,13 +534,18 @@ __device__ void interp_velocity(const DMesh& m, const double* sig, double h0, in
       z_bracket(z, s0, s1, s2, pz, L0, min(kb0, min(kb1, kb2)), R0, true, hint, L, R, w1, w2);
       c.zL = z.nodes(L);
       c.zR = z.nodes(R);
+    } else if constexpr (VM == 2) {
+      const double2 q0 = m.nrec[2u * ux(n0) + 1u], q1 = m.nrec[2u * ux(n1) + 1u], q2 = m.nrec[2u * ux(n2) + 1u];
+      kb0 = m.kb[ux(n0)], kb1 = m.kb[ux(n1)], kb2 = m.kb[ux(n2)];
+      const ZLevels z{m, n0, n1, n2, q0, q1, q2, kb0, kb1, kb2, q0.x + q0.y <= h0, q1.x + q1.y <= h0, q2.x + q2.y <= h0};
+      mono = false;
+      z_bracket(z, s0, s1, s2, pz, L0, 0, R0, false, hint, L, R, w1, w2);
     } else {
-      // kb with a flag where the node's column is not non-decreasing (k_pack_levels), or is not kept
-      const int f0 = m.zn ? m.nkz[ux(n0)] : m.kb[ux(n0)], f1 = m.zn ? m.nkz[ux(n1)] : m.kb[ux(n1)],
-                f2 = m.zn ? m.nkz[ux(n2)] : m.kb[ux(n2)];
+      // kb with a flag where the node's column is not non-decreasing (k_pack_levels)
+      const int f0 = m.nkz[ux(n0)], f1 = m.nkz[ux(n1)], f2 = m.nkz[ux(n2)];
       kb0 = f0 & kKbMask, kb1 = f1 & kKbMask, kb2 = f2 & kKbMask;
-      const ZColumns z{m, h0, n0, n1, n2};
-      mono = m.zn && !((f0 | f1 | f2) & ~kKbMask);
+      const ZColumns z{m, n0, n1, n2};
+      mono = !((f0 | f1 | f2) & ~kKbMask);
       z_bracket(z, s0, s1, s2, pz, L0, min(kb0, min(kb1, kb2)), R0, mono, hint, L, R, w1, w2);
       c.zL = z.nodes(L);
       c.zR = z.nodes(R);
@@ -754,12 +769,13 @@ __device__ void btrack(const DMesh& m, const double* sig, double* lv, const int*
 // backtrackAllNodes (meshdata.cu:3547-3660), one thread per (side, level): consecutive
 // lanes are consecutive levels of one side, so the nodal [node][level] gathers of a wave
 // fall on a few contiguous cache lines.
-// LV: BtCell's velocities in LDS. VM: 0, one sigma per level (kept in LDS) and levels that do not decrease in any wet column; 1, each
-// node's own levels (DMesh::vmode 1 and 2, and 0 where levels may decrease).
+// LV: BtCell's velocities in LDS. VM: 0, one sigma per level (kept in LDS) and levels that do not
+// decrease in any wet column; 1, each node's column (DMesh::vmode 1 and 2); 2, each node's levels evaluated
+// at each probe, always searched in full (short lists of vmode 1 and 2, and vmode 0 where levels may decrease).
 // ST: the workgroup first stages its element patch in LDS (all sides and levels, no list).
 // F: a mesh with kb = 0 at every node whose last sigma is 0 (VM = 0).
 template <int VM, bool ST, bool F, bool LV>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LV ? 4 : 3, 8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LV || VM == 2 ? 4 : 3, 8)))
 k_backtrack(DMesh m, StepArgs a, const int32_t* list_side, const int32_t* list_lev, int32_t count) {
   extern __shared__ double bt_lds[];  // LV: kCellVel x 256; VM = 0: the sigma levels
   double* sig = bt_lds + (LV ? kCellVel * 256 : 0);
@@ -864,9 +880,12 @@ constexpr unsigned kBtFill = 1536, kBtFillColumns = 6144;
 void launch_backtrack(const DMesh& mesh, const StepArgs& a, const int32_t* ls, const int32_t* ll, int32_t count,
                       hipStream_t st) {
   DMesh m = mesh;
-  // A list shorter than the nodes evaluates the levels it probes: the columns cost one evaluation per
-  // node and level, a start point several per substep, so that they pay from a list of about n on.
-  if (ls && count < m.n) m.zn = nullptr;
+  // Columns cost one evaluation per node and level, a start point without them several per substep and a
+  // longer search. Lists, levels evaluated / columns: 52,073 nodes x 24 levels 300 start points 98 / 77 us, x 60
+  // 64 of them 67 / 66; 350,000 x 31 4,000 of them 118 / 119, 256,000 612 / 402 (SZ 451 / 421); 1,400,000 x 20
+  // 64,000 of them 233 / 312, 256,000 686 / 540 (SZ 521 / 564).
+  const int64_t items = (int64_t)m.n * m.nvrt;
+  if (ls && items > (4 << 20) && count < items / 96) m.zn = nullptr;
   if (m.n > 0) hipLaunchKernelGGL(k_pack_nodes, dim3((m.n + kTpb - 1) / kTpb), dim3(kTpb), 0, st, m, a.h0);
   const int64_t total = ls ? (int64_t)count : (int64_t)m.ns * m.nvrt;
   if (total <= 0) return;
@@ -877,10 +896,11 @@ void launch_backtrack(const DMesh& mesh, const StepArgs& a, const int32_t* ls, c
   const dim3 grid((unsigned)((total + 255) / 256));
   const bool stage = m.bt_stage != 0 && !ls;
   // One sigma per level: a wet node's levels do not decrease where 0 <= h0 < H and every sigma between
-  // bed and surface lies in [-1, 0], which VM = 0 relies on. Outside that, VM = 1 searches in full.
+  // bed and surface lies in [-1, 0], which VM = 0 relies on. Outside that, VM = 2 searches in full.
   const bool sigma = m.vmode == 0 && m.sig_mono && a.h0 >= 0.0;
   const size_t lds_sig = sigma ? 8 * (size_t)m.nvrt : 0;
   auto go = [&](auto ker, size_t lds) { hipLaunchKernelGGL(ker, grid, dim3(256), lds, st, m, a, ls, ll, count); };
+  if (!sigma && !m.zn) return go(k_backtrack<2, false, false, false>, 0);
   if (stage) {
     if (sigma)
       go(k_backtrack<0, true, false, false>, lds_sig);

@@ -244,3 +244,33 @@ def test_backtrack_forms(ctx, grid, nx, ny, dx):
     print(f"flags met: {flags}", flush=True)
     assert dx > 8.0 or flags & L.BT_SLIDE
     mesh.close()
+
+
+@pytest.mark.parametrize("grid", ["sz", "lsc2"])
+@pytest.mark.parametrize("count", [1, 700, 50000])
+def test_backtrack_lists_without_columns(ctx, grid, count):
+    """Lists of start points too short for the columns of 4.5 million node levels, whose levels are
+    evaluated at each probe, and one long enough for them."""
+    nvrt, nx, ny = 37, 404, 300
+    spec = cases.CaseSpec(f"lists-{grid}", nx, ny, 300.0, nvrt=nvrt, depth=10.0, substeps=5)
+    data = cases.make_case(spec)
+    depth = np.where(np.hypot(data.xy[:, 0] - 4e4, data.xy[:, 1] - 3e4) < 9e3, -2.0,
+                     6.0 + 70.0 * (data.xy[:, 0] / data.xy[:, 0].max()))
+    kb = None
+    if grid == "sz":
+        vg = core.VGrid(2, nz=3, h_s=40.0, h_c=10.0, theta_b=0.3, theta_f=6.0, ztot=np.array([-160.0, -80.0, -40.0]),
+                        sigma_s=np.linspace(-1.0, 0.0, nvrt - 2))
+    else:
+        vg = core.VGrid(1, sigma_node=-1.0 + np.linspace(0.0, 1.0, nvrt)[None, :] ** (1.0 + 0.7 * np.sin(np.arange(spec.n)))[:, None])
+        kb = np.clip((0.4 * nvrt * (1.0 - depth / depth.max())).astype(np.int32), 0, nvrt - 3)
+    mesh, om, p = _setup_vgrid(ctx, spec, depth, vg, kb=kb)
+    assert mesh.n * nvrt > 4 << 20
+    rng = np.random.default_rng(count)
+    sides = rng.integers(0, mesh.ns, count).astype(np.int32)
+    levs = rng.integers(0, nvrt, count).astype(np.int32)
+    print(f"[gpu] backtracking list of {count}, {grid}", flush=True)
+    mesh.backtrack_list(p, sides, levs)
+    om.backtrack(p, sides, levs, nthreads=8)
+    for f in (L.F_FOOT, L.F_BTU, L.F_BSTATUS):
+        assert_bitwise(mesh.get(f)[sides, levs], om.get(f)[sides, levs], f"field {f}")
+    mesh.close()
