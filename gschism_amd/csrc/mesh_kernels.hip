@@ -1009,7 +1009,9 @@ __global__ void __launch_bounds__(256) k_nodal_velocity(DMesh m, double rx, doub
         }
     }
   };
-  if (j1 - jb <= nst)
+  // levels below the node's bed are 0 and read nothing
+  if (!above) {
+  } else if (j1 - jb <= nst)
     pass([&](int j) { return Lrec[j - jb]; }, [&](int j) { return Larea[j - jb]; });
   else
     pass([&](int j) { return m.ball_rec[j]; }, [&](int j) { return area_of(m.ball_rec[j].x); });
