@@ -1355,7 +1355,7 @@ __device__ __forceinline__ void momentum_side(int nv, const StepArgs& a, const M
     // dz/6, dz/3 and dt dfv0 / dz of layer (k, k+1); the next row reuses them for its layer
     // (k-1, k), whose dz is the same difference of the same two levels. dz/6 = (dz/3) 0.5
     // exactly: halving commutes with rounding for normal values.
-    double zm = zc[kb], z0 = zc[kb + 1], zp = zc[kb + 2];                               // zc[k-1], zc[k], zc[k+1]
+    double z0 = zc[kb + 1], zp = zc[kb + 2];                                        // zc[k], zc[k+1]
     double bm = u[2 * kb + c], b0 = u[2 * (kb + 1) + c], bp = u[2 * (kb + 2) + c];  // btu of this component
     // row kb + 1 (never the top one)
     double dzp = zp - z0;
@@ -1364,7 +1364,7 @@ __device__ __forceinline__ void momentum_side(int nv, const StepArgs& a, const M
     double cprev = d6p - tp;
     double up = (-(0.5 * dzp) * dt * G + d6p * (2.0 * b0 + bp)) / bet;
     u[2 * kb + c] = up;
-    zm = z0, z0 = zp, bm = b0, b0 = bp;
+    z0 = zp, bm = b0, b0 = bp;
     // rows kb + 2 .. nv - 2
     for (int k0 = kb + 2; k0 < nv - 1; k0 += kMomAhead) {
       double zb[kMomAhead], bb[kMomAhead];
@@ -1832,7 +1832,10 @@ void launch_vertical_velocity(const DMesh& m, double h0, hipStream_t st) {
   // just above the line, 20.0 and 24.4)
   const size_t per_elem = 8 * (3 * (size_t)nvp + 1) + sizeof(VvElem);
   auto elems = [&](int items) { return max(1, min(items * 256 / nvp, (int)((32 * 1024) / per_elem))); };
-  const int E = m.ne >= 512 * elems(4) ? elems(4) : elems(1);
+  // two elements on more than 512 levels: phase 2 is one thread per element, and of workgroups of one
+  // element registers let only five onto a CU (18,802 elements x 700 levels 622 us with one, 442 with two)
+  const int two = 2 * per_elem <= 64 * 1024 ? 2 : 1;
+  const int E = m.ne >= 512 * elems(4) ? max(two, elems(4)) : elems(1);
   const size_t lds = per_elem * E;
   auto go = [&](auto ker) { hipLaunchKernelGGL(ker, dim3((unsigned)((m.ne + E - 1) / E)), dim3(256), lds, st, m, h0, E); };
   if (m.vmode == 0)

@@ -924,7 +924,7 @@ def test_concurrent_one_launch_solves(ctx):
                 assert_bitwise(x, xo, "concurrent solve")
 
 
-@pytest.mark.parametrize("nvrt", [2, 3, 4, 5, 6, 7, 8, 9, 10, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("nvrt", [2, 3, 4, 5, 6, 7, 8, 9, 10, 16, 17, 33, 64, 65, 514, 1024])
 def test_velocity_kernels_level_edges(ctx, nvrt):
     """Momentum, Shapiro filter, vertical and nodal velocity around their unrolled levels, items per
     thread and staged ball entries (at two levels a workgroup's nodes have more than are staged), with
