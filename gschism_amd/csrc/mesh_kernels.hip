@@ -446,12 +446,12 @@ __device__ __forceinline__ void z_bracket(const Z& z, double s0, double s1, doub
 // the element's area: every operand is here, in the operations of the full search.
 // LV: the velocities (36 registers' worth) lie in LDS and the area is read again, which leaves four waves
 // a SIMD; otherwise all of it is in registers, for three. With three waves the full search, which every
-// substep pays that enters a new element, was slower than without anything kept: 700x500 nodes x 31
-// levels, 15 s substeps of flows up to 1 m/s, ms without / kept in registers / kept with LV:
-//   one sigma, dx 1000 m 4.32 / 3.45 / 3.20, 50 m 5.82 / 6.80 / 5.98, 10 m 8.86 / 10.87 / 9.36
-//   per-node sigma       5.33 / 4.09 / 3.90        7.16 / 8.55 / 8.01       12.5 / 15.4 / 14.1
+// substep pays that enters a new element, was slower on one sigma than without anything kept: 700x500 nodes
+// x 31 levels, 15 s substeps of flows up to 1 m/s, ms without / kept in registers / kept with LV:
+//   one sigma, dx 1000 m 4.32 / 3.45 / 3.16, 50 m 5.82 / 6.80 / 5.97, 10 m 8.86 / 10.9 / 9.35
+//   per-node sigma       5.33 / 3.60 / 3.65        7.16 / 7.71 / 7.75       12.5 / 14.2 / 13.9
 // (before brackets were kept either: one sigma 5.17, 6.57, 9.60, per-node 9.52, 11.1, 14.7). 1,048,576
-// nodes x 31 levels 8.58 ms with nothing kept, 7.48 in registers (16.8 at four waves, which spill), 6.94 LV.
+// nodes x 31 levels 8.58 ms with nothing kept, 7.48 in registers (16.8 at four waves, which spill), 6.90 LV.
 constexpr int kCellVel = 18;  // (u, v, w) of nodes 0-2 at the lower level, then at the upper one
 template <bool LV>
 struct BtCell {
@@ -871,11 +871,11 @@ __global__ void k_pack_levels(DMesh m, double h0) {
 }
 
 // Workgroups from which the fourth wave a SIMD of the LV form pays for its LDS trips: three waves hold 768
-// on the chip. Register form / LV, flows that stay in their elements and that leave one each substep:
-// one sigma, 60x40x11 (303 workgroups) 45 / 49 and 119 / 126 us, 110x80x12 (1,220) 71 / 71 and 193 /
-// 190, 120x90x14 (1,750) 87 / 87 and 240 / 224; per-node sigma, whose search spills at four waves,
-// 120x80x21 (2,350) 116 / 119 and 368 / 385, 301x173x31 (18,900) 679 / 670 and 1,956 / 1,791.
-constexpr unsigned kBtFill = 1536, kBtFillColumns = 6144;
+// on the chip. One sigma, register form / LV, flows that stay in their elements and that leave one each
+// substep: 60x40x11 (303 workgroups) 45 / 49 and 119 / 126 us, 110x80x12 (1,220) 71 / 71 and 193 / 190,
+// 120x90x14 (1,750) 87 / 87 and 240 / 224. Columns, whose probes are loads and whose search spills at four
+// waves, stay in registers (BtCell has the figures).
+constexpr unsigned kBtFill = 1536;
 
 void launch_backtrack(const DMesh& mesh, const StepArgs& a, const int32_t* ls, const int32_t* ll, int32_t count,
                       hipStream_t st) {
@@ -908,19 +908,18 @@ void launch_backtrack(const DMesh& mesh, const StepArgs& a, const int32_t* ls, c
       go(k_backtrack<1, true, false, false>, 0);
     return;
   }
-  const bool lv = grid.x > (sigma ? kBtFill : kBtFillColumns);
+  if (!sigma) return go(k_backtrack<1, false, false, false>, 0);
+  const bool lv = grid.x > kBtFill;
   auto pick = [&](auto ldsv, auto regv) {
     if (lv)
       go(ldsv, lds_sig + 8 * kCellVel * 256);
     else
       go(regv, lds_sig);
   };
-  if (sigma && m.flat)
+  if (m.flat)
     pick(k_backtrack<0, false, true, true>, k_backtrack<0, false, true, false>);
-  else if (sigma)
-    pick(k_backtrack<0, false, false, true>, k_backtrack<0, false, false, false>);
   else
-    pick(k_backtrack<1, false, false, true>, k_backtrack<1, false, false, false>);
+    pick(k_backtrack<0, false, false, true>, k_backtrack<0, false, false, false>);
 }
 
 // ---------------------------------------------------------------- nodal velocities
