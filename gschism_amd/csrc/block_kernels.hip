@@ -35,7 +35,7 @@ namespace gsh {
 
 constexpr int kBlkRows = 4;  // rows of a thread in flight
 template <int W>
-constexpr int kBlkThreads = W == 16 ? 512 : 1024;
+constexpr int kBlkThreads = W == 16 ? 512 : (W == 8 ? 1024 : 256);
 
 // A thread's place: member m, tile, and the rows rl, rl + L, ... of the tile.
 struct BlkPlace {
@@ -56,44 +56,38 @@ __device__ __forceinline__ BlkPlace blk_place(int M) {
   return q;
 }
 
+// 0.0 + f(0) + f(1) + ... + f(n - 1), n below 16 or a multiple of it, f a value in LDS: 16 are read
+// ahead of their additions, without selects, which took longer than the additions (k_blk_reduce on
+// 958 tiles of one member 23.7 us against 13.1).
+template <class F>
+__device__ __forceinline__ double blk_chain(int n, F&& f) {
+  constexpr int B = 16;
+  double x = 0.0;
+  if (n < B) {
+    for (int i = 0; i < n; ++i) x += f(i);
+    return x;
+  }
+  for (int i0 = 0; i0 < n; i0 += B) {
+    double v[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) v[u] = f(i0 + u);
+#pragma unroll
+    for (int u = 0; u < B; ++u) x += v[u];
+  }
+  return x;
+}
+
 // The tile partial of each member of the workgroup from the rows' products in pr ([row][W]), which
 // every thread passes after its own are written. A row beyond n or of a stopped member has the
 // product +0.0, and a sum that started at 0.0 is never -0.0, so adding it changes no bit.
 __device__ __forceinline__ void blk_tile_sum(const BlkPlace& q, const double* pr, double* slot,
                                              double* __restrict__ part) {
-  constexpr int B = 16;
   const int SS = kTpb >> q.lm, J = kBlkTile / kTpb << q.lm;
   __syncthreads();
-  if (q.rl < SS) {
-    double x = 0.0;
-    const int jn = min(B, J);
-    for (int j0 = 0; j0 < J; j0 += B) {
-      double v[B];
-#pragma unroll
-      for (int u = 0; u < B; ++u) {
-        const double y = pr[((q.rl + SS * (j0 + (u & (jn - 1)))) << q.lw) + q.w];
-        v[u] = u < jn ? y : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < B; ++u) x += v[u];
-    }
-    slot[threadIdx.x] = x;
-  }
+  if (q.rl < SS) slot[threadIdx.x] = blk_chain(J, [&](int j) { return pr[((q.rl + SS * j) << q.lw) + q.w]; });
   __syncthreads();
-  if (q.rl == 0) {
-    double x = 0.0;
-    for (int r0 = 0; r0 < SS; r0 += B) {
-      double v[B];
-#pragma unroll
-      for (int u = 0; u < B; ++u) {
-        const double y = slot[(min(r0 + u, SS - 1) << q.lw) + q.w];
-        v[u] = r0 + u < SS ? y : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < B; ++u) x += v[u];
-    }
-    part[(int64_t)q.tile * q.M + q.m] = x;
-  }
+  if (q.rl == 0)
+    part[(int64_t)q.tile * q.M + q.m] = blk_chain(SS, [&](int r) { return slot[(r << q.lw) + q.w]; });
 }
 
 // ---------------------------------------------------------------- init
@@ -254,19 +248,9 @@ __device__ __forceinline__ double blk_total(const double* __restrict__ P, int nt
   }
   lds[threadIdx.x] = u;
   __syncthreads();
-  // slots beyond the tiles hold +0.0, which changes no sum; the others are read 16 ahead of their
-  // additions (1,024 slots one at a time took most of an iteration of a one-member block)
-  double t = 0.0;
-  if (r == 0) {
-    const int nr = min(RS, ntiles);
-    for (int q0 = 0; q0 < nr; q0 += 16) {
-      double v[16];
-#pragma unroll
-      for (int q = 0; q < 16; ++q) v[q] = q0 + q < nr ? lds[(q0 + q) * M + m] : 0.0;
-#pragma unroll
-      for (int q = 0; q < 16; ++q) t += v[q];
-    }
-  }
+  // slots beyond the tiles hold +0.0, which changes no sum: the chain ends with the 16 that hold the last tile
+  const int nr = RS < 16 ? RS : min(RS, (ntiles + 15) & ~15);
+  const double t = r == 0 ? blk_chain(nr, [&](int q) { return lds[q * M + m]; }) : 0.0;
   __syncthreads();
   return t;
 }
@@ -332,14 +316,17 @@ __global__ void k_blk_get(double* __restrict__ x, const VT* __restrict__ xblk, i
 // is a whole 128-byte line and the columns are read once for twice the members (305,500 rows x 64
 // members: 830 us per iteration against 980; 30,000 x 256: 420 against 490); with 8 a small block
 // fills twice the CUs (16,000 x 64: 54 us against 75). 512 threads measured best with 16 members,
-// 1024 with 8.
+// 1024 with 8. A block of one or two members takes a tile with 256 threads: most of 1024 would have
+// no row of it (1,048,576 rows, with the chains of blk_chain, 100 us per iteration against 227).
 template <class VT, class F>
 static void blk_wide(const BlkSys<VT>& S, F&& launch) {
   constexpr int kFill = 512;  // workgroups
   if (S.M >= 16 && S.ntiles * (S.M / 16) >= kFill)
     launch(std::integral_constant<int, 16>(), dim3(S.ntiles * (S.M / 16)));
-  else
+  else if (S.M > 2)
     launch(std::integral_constant<int, 8>(), dim3(S.ntiles * (S.M / std::min(S.M, 8))));
+  else
+    launch(std::integral_constant<int, 2>(), dim3(S.ntiles));
 }
 template <class VT>
 void launch_blk_init(const BlkSys<VT>& S, hipStream_t st) {

@@ -84,10 +84,12 @@ def test_block_set_member_zero_rhs_and_maxiter(ctx):
     solo.close()
 
 
-@pytest.mark.parametrize("members,nx,ny", [(1, 31, 19), (3, 40, 27), (100, 48, 23), (256, 164, 100)])
+@pytest.mark.parametrize("members,nx,ny", [(1, 31, 19), (1, 260, 200), (2, 37, 21), (3, 40, 27), (100, 48, 23),
+                                           (256, 164, 100)])
 def test_block_member_and_row_splits(ctx, members, nx, ny):
-    """One to 256 members: 8 or fewer and 16 members per workgroup (the last size), chains of 2 to
-    512 rows per slot, last tiles of a few rows; 25 iterations, bit for bit."""
+    """One to 256 members: 2, 8 and 16 members per workgroup (the last size), chains of 2 to
+    512 rows per slot and of 1 to 256 slots, tile counts that are no multiple of 16, last tiles of a
+    few rows; 25 iterations, bit for bit."""
     mesh, p, blk, solo, vals, bs = _ensemble(ctx, members, nx, ny)
     ip, ix = mesh.topology(L.T_CSR_INDPTR), mesh.topology(L.T_CSR_INDICES)
     print(f"[gpu] block of {members} members, n={mesh.n}", flush=True)
