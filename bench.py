@@ -738,8 +738,8 @@ def main() -> int:
         ip_h, ix_h = mesh.topology(L.T_CSR_INDPTR), mesh.topology(L.T_CSR_INDICES)
         val = solver.get_values()
         bvec = solver.get_rhs()
-        # the host cores this process may use: the CPU share the GPU box gives one GPU
-        # (OMP_NUM_THREADS there), else every core of the affinity mask
+        # the host cores this process may use: OMP_NUM_THREADS where it is set (a host's CPU
+        # share of one GPU), else every core of the affinity mask
         affinity = len(os.sched_getaffinity(0))
         share = int(os.environ.get("OMP_NUM_THREADS", "0") or 0)
         threads = args.cpu_threads or (min(share, affinity) if share > 0 else affinity)
